@@ -2348,13 +2348,8 @@ __global__ void __launch_bounds__(TPB) k_fill(T *x, long n, T v)
     if (q < n) x[q] = v;
 }
 
-// -------------------------------------------- single-workgroup coarse cycle
-// The cycle (V, W or F) over levels lc..nlev-1 and the FP64 CG bottom
-// solve, all inside one 512-thread workgroup (these levels are latency
-// bound; one launch replaces dozens).  When they fit, the levels are
-// staged in LDS for the whole cycle; otherwise they stay in global memory
-// (L2 resident).  512 threads leave 256 VGPRs per lane, so the inlined
-// cycle does not spill.
+// ------------------------------------------------ bottom solve of large bottoms
+// 512 threads leave 256 VGPRs per lane, so the inlined solvers do not spill
 static constexpr int CTPB = 512;
 
 __device__ __forceinline__ double blk_sum(double v, double *sh)
@@ -2612,386 +2607,20 @@ __device__ void blk_bottom_bicgstab(const Lev<T> &L, double *cg, double eps, int
     __syncthreads();
 }
 
-// sums over the 64 lanes of a wave in a fixed order (butterfly), so every
-// lane holds the same, deterministic result
-__device__ __forceinline__ double wave_sum(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
-// The bottom solve of a level of at most 64 cells inside one wave: nub
-// red-black sweeps, the FP64 CG of blk_bottom_cg or BiCGStab of
-// blk_bottom_bicgstab (mean projected out on singular problems; neither for
-// smoothing only), nub sweeps.  Lane q owns cell q; neighbour values come
-// by lane shuffles (zero outside a non-periodic side), so the wave needs no
-// barrier.  Same updates and stopping rule as the block form; only the order
-// of the CG's sums differs.
+// The bottom solve of a level too large for the single-workgroup cycle's LDS
+// image (COARSE_BOTTOM cells, mac_legs.hip): nub sweeps, the block CG or
+// BiCGStab (none for smoothing only), nub sweeps, in one 512-thread workgroup
+// on global memory.
 template <int DIM, typename T>
-__device__ void wave_bottom(const Lev<T> &L, const CoarseOpts &o)
+__global__ void __launch_bounds__(CTPB) k_bottom(Lev<T> L, CoarseOpts o, double *cg)
 {
-    const int q = threadIdx.x & 63;
-    const int nx = L.nx, ny = L.ny, nz = L.nz, n = nx * ny * nz, plane = nx * ny;
-    const bool live = q < n;
-    const int qc = live ? q : 0;
-    const int i = qc % nx, j = (qc / nx) % ny, k = qc / plane;
-    // neighbour lanes (-1: outside a non-periodic side) and face weights
-    int nb[6];
-    nb[0] = i > 0 ? qc - 1 : (L.perx ? qc + nx - 1 : -1);
-    nb[1] = i < nx - 1 ? qc + 1 : (L.perx ? qc - (nx - 1) : -1);
-    nb[2] = j > 0 ? qc - nx : (L.pery ? qc + (ny - 1) * nx : -1);
-    nb[3] = j < ny - 1 ? qc + nx : (L.pery ? qc - (ny - 1) * nx : -1);
-    if (DIM == 3) {
-        nb[4] = k > 0 ? qc - plane : (L.perz ? qc + (nz - 1) * plane : -1);
-        nb[5] = k < nz - 1 ? qc + plane : (L.perz ? qc - (nz - 1) * plane : -1);
-    } else {
-        nb[4] = nb[5] = -1;
-    }
-    T w[6];
-    w[0] = L.bx[qc];
-    w[1] = (i < nx - 1) ? L.bx[qc + 1] : L.bxh[j + ny * k];
-    w[2] = L.by[qc];
-    w[3] = (j < ny - 1) ? L.by[qc + nx] : L.byh[i + nx * k];
-    if (DIM == 3) {
-        w[4] = L.bz[qc];
-        w[5] = (k < nz - 1) ? L.bz[qc + plane] : L.bzh[i + nx * j];
-    } else {
-        w[4] = w[5] = T(0);
-    }
-    const int colour = (i + j + k) & 1;
-    T phi = live ? L.phi[qc] : T(0);
-    const T rhs = live ? L.rhs[qc] : T(0);
-    const T acell = alpha_at(L, qc);
-    auto gather = [&](auto v, auto *p) {   // neighbour values of v (all lanes shuffle)
-#pragma unroll
-        for (int s = 0; s < 6; ++s) {
-            const auto t = __shfl(v, nb[s] < 0 ? q : nb[s], 64);
-            p[s] = nb[s] < 0 ? decltype(v)(0) : t;
-        }
-    };
-    auto sweeps = [&](int count) {
-        for (int it = 0; it < count; ++it)
-            for (int c = 0; c < 2; ++c) {
-                T p[6];
-                gather(phi, p);
-                const T v = gs_value<DIM, T>(L, w, p, rhs, acell);
-                if (live && colour == c) phi = v;
-            }
-    };
-    sweeps(o.nub);
-    // ---- CG in FP64 on A x = rhs (- mean)
-    Lev<double> D;
-    D.nx = nx; D.ny = ny; D.nz = nz;
-    D.perx = L.perx; D.pery = L.pery; D.perz = L.perz;
-    D.ih2x = L.ih2x; D.ih2y = L.ih2y; D.ih2z = L.ih2z;
-    double wd[6];
-#pragma unroll
-    for (int s = 0; s < 6; ++s) wd[s] = (double)w[s];
-    auto apply = [&](double x) -> double {
-        double p[6];
-        gather(x, p);
-        if (!live) return 0.0;
-        const double ap = apply_value<DIM, double>(D, wd, p, x);
-        return L.alpha ? fma((double)acell, x, ap) : ap;
-    };
-    const double nd = (double)n;
-    const double m = o.singular ? wave_sum(live ? (double)rhs : 0.0) / nd : 0.0;
-    double x = live ? (double)phi : 0.0;
-    double r = live ? ((double)rhs - m) - apply(x) : 0.0;
-    if (o.singular) {
-        const double rm = wave_sum(r) / nd;
-        if (live) r -= rm;
-    }
-    const double r0 = wave_max(fabs(r));
-    if (r0 > 0.0 && o.bottom == MAC_BOTTOM_BICGSTAB) {
-        // the BiCGStab of blk_bottom_bicgstab, one cell per lane
-        const double rh = r;
-        double p = 0.0, v = 0.0, rho_old = 1.0, al = 1.0, om = 1.0;
-        auto project = [&]() {
-            if (o.singular) {
-                const double rm = wave_sum(r) / nd;
-                if (live) r -= rm;
-            }
-        };
-        for (int it = 0; it < o.bottom_maxit; ++it) {
-            const double rho = wave_sum(rh * r);
-            if (rho == 0.0) break;
-            if (it == 0) p = r;
-            else p = r + ((rho / rho_old) * (al / om)) * (p - om * v);
-            v = apply(p);
-            const double rv = wave_sum(rh * v);
-            if (rv == 0.0) break;
-            al = rho / rv;
-            r -= al * v;
-            project();
-            if (wave_max(fabs(r)) <= o.bottom_eps * r0) {
-                x += al * p;
-                break;
-            }
-            const double t = apply(r);
-            const double tt = wave_sum(t * t);
-            if (!(tt > 0.0)) {
-                x += al * p;
-                break;
-            }
-            om = wave_sum(t * r) / tt;
-            x += al * p + om * r;
-            r -= om * t;
-            project();
-            rho_old = rho;
-            if (wave_max(fabs(r)) <= o.bottom_eps * r0 || om == 0.0) break;
-        }
-    } else if (r0 > 0.0 && o.bottom == MAC_BOTTOM_CG) {
-        double p = r;
-        double rr = wave_sum(r * r);
-        for (int it = 0; it < o.bottom_maxit; ++it) {
-            const double Ap = apply(p);
-            const double pap = wave_sum(p * Ap);
-            if (!(pap > 0.0)) break;
-            const double alpha = rr / pap;
-            x += alpha * p;
-            r -= alpha * Ap;
-            if (o.singular) {
-                const double rm = wave_sum(r) / nd;
-                if (live) r -= rm;
-            }
-            const double am = wave_max(fabs(r));
-            const double rr1 = wave_sum(r * r);
-            if (am <= o.bottom_eps * r0) break;
-            const double beta = rr1 / rr;
-            rr = rr1;
-            p = r + beta * p;
-        }
-    }
-    phi = live ? (T)x : T(0);
-    sweeps(o.nub);
-    if (live) L.phi[qc] = phi;
-}
-
-template <int DIM, typename T>
-__device__ void blk_resid_restrict(const Lev<T> &F, const Lev<T> &C)
-{
-    const int nc = C.nx * C.ny * C.nz;
-    for (int q = threadIdx.x; q < nc; q += blockDim.x) {
-        const int rq = q / C.nx, I = q - rq * C.nx;
-        const int K = rq / C.ny, J = rq - K * C.ny;
-        T rv[2][2][2];
-        for (int c = 0; c < (DIM == 3 ? 2 : 1); ++c)
-            for (int b = 0; b < 2; ++b)
-                for (int a = 0; a < 2; ++a) {
-                    int i = 2 * I + a, j = 2 * J + b, k = (DIM == 3) ? 2 * K + c : 0;
-                    const int f = i + F.nx * (j + F.ny * k);
-                    T w[6], p[6];
-                    stencil<DIM, T>(F, F.phi, i, j, k, f, w, p);
-                    rv[c][b][a] = F.rhs[f] - with_alpha(F, f, apply_value<DIM, T>(F, w, p, F.phi[f]), F.phi[f]);
-                }
-        T v;
-        if (DIM == 3) {
-            v = ((rv[0][0][0] + rv[0][0][1]) + (rv[0][1][0] + rv[0][1][1])) +
-                ((rv[1][0][0] + rv[1][0][1]) + (rv[1][1][0] + rv[1][1][1]));
-            C.rhs[q] = T(0.125) * v;
-        } else {
-            v = (rv[0][0][0] + rv[0][0][1]) + (rv[0][1][0] + rv[0][1][1]);
-            C.rhs[q] = T(0.25) * v;
-        }
-        C.phi[q] = T(0);
-    }
-    __syncthreads();
-}
-
-template <int DIM, typename T>
-__device__ void blk_prolong(const Lev<T> &F, const Lev<T> &C, const EllBC &bc)
-{
-    const int n = F.nx * F.ny * F.nz;
-    for (int q = threadIdx.x; q < n; q += blockDim.x) {
-        const int r = q / F.nx, i = q - r * F.nx;
-        const int k = r / F.ny, j = r - k * F.ny;
-        F.phi[q] = F.phi[q] + prolong_value<DIM, T>(C.phi, C.nx, C.ny, C.nz, bc, i, j, k);
-    }
-    __syncthreads();
-}
-
-// LDS image of the coarse levels: per level phi, rhs, bx, by, (bz), then the
-// high-face slabs, each rounded to 16 bytes; after the last level the four
-// FP64 CG vectors.  The host sizes the allocation with the same function.
-__host__ __device__ inline int lds_round(int bytes) { return (bytes + 15) & ~15; }
-
-template <int DIM, typename T>
-__host__ __device__ inline int lds_level_bytes(int nx, int ny, int nz)
-{
-    const int n = nx * ny * nz, s = (int)sizeof(T);
-    int b = 4 * lds_round(n * s) + lds_round(ny * nz * s) + lds_round(nx * nz * s);
-    if (DIM == 3) b += lds_round(n * s) + lds_round(nx * ny * s);
-    return b;
-}
-
-template <int DIM, typename T>
-__device__ Lev<T> lds_view(const Lev<T> &G, char *p)
-{
-    Lev<T> S = G;
-    const int n = G.nx * G.ny * G.nz;
-    auto carve = [&](int cnt) {
-        T *r = (T *)p;
-        p += lds_round(cnt * (int)sizeof(T));
-        return r;
-    };
-    S.phi = carve(n);
-    S.rhs = carve(n);
-    S.bx = carve(n);
-    S.by = carve(n);
-    S.bxh = carve(G.ny * G.nz);
-    S.byh = carve(G.nx * G.nz);
-    if (DIM == 3) {
-        S.bz = carve(n);
-        S.bzh = carve(G.nx * G.ny);
-    }
-    S.res = S.phi2 = nullptr;
-    return S;
-}
-
-// Level l of the coarse cycle: the global level itself, or its LDS image.
-template <int DIM, typename T, bool LDS>
-__device__ Lev<T> coarse_level(const Lev<T> *levs, int lc, int l, char *smem)
-{
-    if (!LDS) return levs[l];
-    char *p = smem;
-    for (int m = lc; m < l; ++m) p += lds_level_bytes<DIM, T>(levs[m].nx, levs[m].ny, levs[m].nz);
-    return lds_view<DIM, T>(levs[l], p);
-}
-
-// the bottom level: one wave for at most 64 cells (one cell per lane in
-// registers, no block barriers), else nub sweeps, the block CG or BiCGStab
-// (none for smoothing only), nub sweeps
-template <int DIM, typename T>
-__device__ __forceinline__ void coarse_bottom(const Lev<T> &L, const CoarseOpts &o, double *cg, double *sh)
-{
-    if (L.nx * L.ny * L.nz <= 64) {
-        if (threadIdx.x < 64) wave_bottom<DIM, T>(L, o);
-        __syncthreads();
-    } else {
-        for (int s = 0; s < o.nub; ++s) blk_gsrb<DIM, T>(L);
-        if (o.bottom == MAC_BOTTOM_CG)
-            blk_bottom_cg<DIM, T>(L, cg, o.bottom_eps, o.bottom_maxit, o.singular, sh);
-        else if (o.bottom == MAC_BOTTOM_BICGSTAB)
-            blk_bottom_bicgstab<DIM, T>(L, cg, o.bottom_eps, o.bottom_maxit, o.singular, sh);
-        for (int s = 0; s < o.nub; ++s) blk_gsrb<DIM, T>(L);
-    }
-}
-
-// VC: a V-cycle (straight down and up); else a W or F cycle
-template <int DIM, typename T, bool LDS, bool VC>
-__global__ void __launch_bounds__(CTPB) k_coarse_cycle(const Lev<T> *__restrict__ levs, int lc,
-                                                       int nlev, CoarseOpts o, double *cg)
-{
-    extern __shared__ __align__(16) char smem[];
     __shared__ double sh[CTPB / 64];
-    const int bot = nlev - 1;
-    if (LDS) {
-        // stage the weights of every coarse level, and phi/rhs of the first
-        // (deeper phi/rhs are written by the restriction before use).  One
-        // pass per level: a thread issues every load of its cell and slab
-        // entries before it stores any, so each level costs one round of
-        // global latency rather than one per array
-        for (int l = lc; l <= bot; ++l) {
-            const Lev<T> G = levs[l];
-            const Lev<T> S = coarse_level<DIM, T, true>(levs, lc, l, smem);
-            const int n = G.nx * G.ny * G.nz, nsx = G.ny * G.nz, nsy = G.nx * G.nz;
-            const int nsz = (DIM == 3) ? G.nx * G.ny : 0;
-            const int m = max(max(n, nsx), max(nsy, nsz));
-            for (int q = threadIdx.x; q < m; q += blockDim.x) {
-                const bool c = q < n, hx = q < nsx, hy = q < nsy, hz = q < nsz;
-                T vx = T(0), vy = T(0), vz = T(0), vp = T(0), vr = T(0), wx = T(0), wy = T(0), wz = T(0);
-                if (c) {
-                    vx = G.bx[q];
-                    vy = G.by[q];
-                    if (DIM == 3) vz = G.bz[q];
-                    if (l == lc) {
-                        vp = G.phi[q];
-                        vr = G.rhs[q];
-                    }
-                }
-                if (hx) wx = G.bxh[q];
-                if (hy) wy = G.byh[q];
-                if (hz) wz = G.bzh[q];
-                if (c) {
-                    S.bx[q] = vx;
-                    S.by[q] = vy;
-                    if (DIM == 3) S.bz[q] = vz;
-                    if (l == lc) {
-                        S.phi[q] = vp;
-                        S.rhs[q] = vr;
-                    }
-                }
-                if (hx) S.bxh[q] = wx;
-                if (hy) S.byh[q] = wy;
-                if (hz) S.bzh[q] = wz;
-            }
-        }
-        char *p = smem;
-        for (int m = lc; m <= bot; ++m) p += lds_level_bytes<DIM, T>(levs[m].nx, levs[m].ny, levs[m].nz);
-        cg = (double *)p;
-        __syncthreads();
-    }
-    if constexpr (VC) {
-        for (int l = lc; l < bot; ++l) {
-            const Lev<T> L = coarse_level<DIM, T, LDS>(levs, lc, l, smem);
-            for (int s = 0; s < o.nu1; ++s) blk_gsrb<DIM, T>(L);
-            blk_resid_restrict<DIM, T>(L, coarse_level<DIM, T, LDS>(levs, lc, l + 1, smem));
-        }
-        coarse_bottom<DIM, T>(coarse_level<DIM, T, LDS>(levs, lc, bot, smem), o, cg, sh);
-        for (int l = bot - 1; l >= lc; --l) {
-            const Lev<T> L = coarse_level<DIM, T, LDS>(levs, lc, l, smem);
-            blk_prolong<DIM, T>(L, coarse_level<DIM, T, LDS>(levs, lc, l + 1, smem), o.bc);
-            for (int s = 0; s < o.nu2; ++s) blk_gsrb<DIM, T>(L);
-        }
-    } else {
-        // W and F cycles, without recursion.  Going down, each level owes a
-        // second visit of the next coarser level (bit l of `again`; bit l of
-        // `again_w`: that visit is a W, else a V); going up, a level that
-        // owes one turns back down before its prolongation.  The first visit
-        // has the shape of the visiting level.  The masks are the same in
-        // every thread, so the block stays in step.
-        unsigned again = 0u, again_w = 0u;
-        bool w = o.cycle == MAC_CYCLE_W;   // shape of the current visit (W, or F/V below)
-        bool v = false;                     // the current visit is a V
-        int l = lc;
-        for (;;) {
-            for (; l < bot; ++l) {
-                const Lev<T> L = coarse_level<DIM, T, LDS>(levs, lc, l, smem);
-                for (int s = 0; s < o.nu1; ++s) blk_gsrb<DIM, T>(L);
-                blk_resid_restrict<DIM, T>(L, coarse_level<DIM, T, LDS>(levs, lc, l + 1, smem));
-                if (!v) {
-                    again |= 1u << l;
-                    if (w) again_w |= 1u << l;
-                    else again_w &= ~(1u << l);
-                }
-            }
-            coarse_bottom<DIM, T>(coarse_level<DIM, T, LDS>(levs, lc, bot, smem), o, cg, sh);
-            bool down = false;
-            while (l > lc) {
-                --l;
-                if (again & (1u << l)) {   // second visit of level l + 1
-                    again &= ~(1u << l);
-                    w = (again_w >> l) & 1u;
-                    v = !w;
-                    ++l;
-                    down = true;
-                    break;
-                }
-                const Lev<T> L = coarse_level<DIM, T, LDS>(levs, lc, l, smem);
-                blk_prolong<DIM, T>(L, coarse_level<DIM, T, LDS>(levs, lc, l + 1, smem), o.bc);
-                for (int s = 0; s < o.nu2; ++s) blk_gsrb<DIM, T>(L);
-            }
-            if (!down) break;
-        }
-    }
-    if (LDS) {
-        const Lev<T> G = levs[lc];
-        const Lev<T> S = coarse_level<DIM, T, true>(levs, lc, lc, smem);
-        const int n = G.nx * G.ny * G.nz;
-        for (int q = threadIdx.x; q < n; q += blockDim.x) G.phi[q] = S.phi[q];
-    }
+    for (int s = 0; s < o.nub; ++s) blk_gsrb<DIM, T>(L);
+    if (o.bottom == MAC_BOTTOM_CG)
+        blk_bottom_cg<DIM, T>(L, cg, o.bottom_eps, o.bottom_maxit, o.singular, sh);
+    else if (o.bottom == MAC_BOTTOM_BICGSTAB)
+        blk_bottom_bicgstab<DIM, T>(L, cg, o.bottom_eps, o.bottom_maxit, o.singular, sh);
+    for (int s = 0; s < o.nub; ++s) blk_gsrb<DIM, T>(L);
 }
 
 // ------------------------------------------------------ face correction
@@ -4046,41 +3675,9 @@ void launch_fill(T *x, long n, T v, hipStream_t s)
 // LDS bytes the coarse cycle needs to keep levels lc..nlev-1 and the bottom
 // CG vectors on chip
 template <typename T>
-static long coarse_lds_bytes(int dim, const Lev<T> *levs_host, int lc, int nlev)
+void launch_bottom(int dim, const Lev<T> &L, const CoarseOpts &o, double *cg, hipStream_t s)
 {
-    long b = 0;
-    for (int l = lc; l < nlev; ++l) {
-        const Lev<T> &L = levs_host[l];
-        b += dim == 3 ? lds_level_bytes<3, T>(L.nx, L.ny, L.nz) : lds_level_bytes<2, T>(L.nx, L.ny, 1);
-    }
-    const Lev<T> &B = levs_host[nlev - 1];
-    return b + (long)BOTTOM_VECS * B.nx * B.ny * B.nz * (long)sizeof(double);
-}
-
-static constexpr long COARSE_LDS_MAX = 64 * 1024;
-
-template <typename T>
-void launch_coarse_cycle(int dim, const Lev<T> *levs_dev, const Lev<T> *levs_host, int lc, int nlev,
-                         const CoarseOpts &o, double *cg, hipStream_t s)
-{
-    const long lds = coarse_lds_bytes<T>(dim, levs_host, lc, nlev);
-    const bool in_lds = lds <= COARSE_LDS_MAX;
-    const unsigned sh = in_lds ? (unsigned)lds : 0u;
-    if (o.cycle == MAC_CYCLE_V) {
-        if (in_lds)
-            DISPATCH_DIM(dim, hipLaunchKernelGGL((k_coarse_cycle<D_, T, true, true>), dim3(1), dim3(CTPB), sh, s,
-                                                 levs_dev, lc, nlev, o, cg));
-        else
-            DISPATCH_DIM(dim, hipLaunchKernelGGL((k_coarse_cycle<D_, T, false, true>), dim3(1), dim3(CTPB), sh,
-                                                 s, levs_dev, lc, nlev, o, cg));
-    } else {
-        if (in_lds)
-            DISPATCH_DIM(dim, hipLaunchKernelGGL((k_coarse_cycle<D_, T, true, false>), dim3(1), dim3(CTPB), sh,
-                                                 s, levs_dev, lc, nlev, o, cg));
-        else
-            DISPATCH_DIM(dim, hipLaunchKernelGGL((k_coarse_cycle<D_, T, false, false>), dim3(1), dim3(CTPB), sh,
-                                                 s, levs_dev, lc, nlev, o, cg));
-    }
+    DISPATCH_DIM(dim, hipLaunchKernelGGL((k_bottom<D_, T>), dim3(1), dim3(CTPB), 0, s, L, o, cg));
 }
 
 void launch_correct(const CorrectArgs &A, int maxcols, int maxez, int maxghost, hipStream_t s)
@@ -4152,7 +3749,7 @@ template void launch_prolong<double>(int, const Lev<double> &, const Lev<double>
 template void launch_prolong<float>(int, const Lev<float> &, const Lev<float> &, const EllBC &, hipStream_t);
 template void launch_fill<double>(double *, long, double, hipStream_t);
 template void launch_fill<float>(float *, long, float, hipStream_t);
-template void launch_coarse_cycle<double>(int, const Lev<double> *, const Lev<double> *, int, int, const CoarseOpts &, double *, hipStream_t);
-template void launch_coarse_cycle<float>(int, const Lev<float> *, const Lev<float> *, int, int, const CoarseOpts &, double *, hipStream_t);
+template void launch_bottom<double>(int, const Lev<double> &, const CoarseOpts &, double *, hipStream_t);
+template void launch_bottom<float>(int, const Lev<float> &, const CoarseOpts &, double *, hipStream_t);
 
 }  // namespace mac

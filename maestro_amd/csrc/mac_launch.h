@@ -67,6 +67,31 @@ struct CoarseOpts {
     EllBC bc;
 };
 
+// ---- the small levels (mac_legs.hip)
+// levels whose way down or up runs as one launch: measured limits
+static constexpr long LEG_MAX_3D = 1L << 18, LEG_MAX_2D = 1L << 22;
+static constexpr long LEG_SMALL_3D = 1L << 16;
+// the single-workgroup coarse cycle: cells of its first level, cells of the
+// bottom, levels, threads, LDS bytes
+static constexpr int COARSE_CELLS = 4096, COARSE_BOTTOM = 1024, COARSE_LEVELS = 8, COARSE_THREADS = 1024;
+static constexpr long COARSE_LDS = 150 * 1024;
+// whether a level takes the fused legs (even extents, phi2, size)
+template <typename T> bool leg_ok(int dim, const Lev<T> &L);
+// two sweeps of pin (zero: known zero, not read) -> pout, the restricted
+// residual into C.rhs, C.phi = 0
+template <typename T>
+void launch_leg_down(int dim, const Lev<T> &L, const T *pin, T *pout, bool zero, const Lev<T> &C, hipStream_t s);
+// pin + P C.phi and two sweeps -> pout
+template <typename T>
+void launch_leg_up(int dim, const Lev<T> &L, const T *pin, T *pout, const Lev<T> &C, const EllBC &bc, hipStream_t s);
+// the first level from which the single-workgroup cycle can take over (its
+// levels fit LDS), -1: none (a bottom of more than COARSE_BOTTOM cells)
+template <typename T> int coarse_first(int dim, const Lev<T> *levs, int nlev);
+// the cycle over levs[lc ..] (host table) on levs[lc].phi; zero: that iterate
+// is zero and not read.  False (nothing launched) where it does not fit
+template <typename T>
+bool launch_coarse(int dim, const Lev<T> *levs, int lc, int nlev, const CoarseOpts &o, bool zero, hipStream_t s);
+
 // whole-domain (natural layout) forward arguments
 struct LevelIO {
     double *ux, *uy, *uz;
@@ -306,9 +331,10 @@ void launch_restrict(int dim, const T *r, int fnx, int fny, const Lev<T> &C, hip
 template <typename T>
 void launch_prolong(int dim, const Lev<T> &F, const Lev<T> &C, const EllBC &bc, hipStream_t s);
 template <typename T> void launch_fill(T *x, long n, T v, hipStream_t s);
+// the bottom solve of a level that the single-workgroup cycle does not take,
+// on L.phi (cg: scratch of BOTTOM_VECS vectors)
 template <typename T>
-void launch_coarse_cycle(int dim, const Lev<T> *levs_dev, const Lev<T> *levs_host, int lc, int nlev,
-                         const CoarseOpts &o, double *cg, hipStream_t s);
+void launch_bottom(int dim, const Lev<T> &L, const CoarseOpts &o, double *cg, hipStream_t s);
 void launch_correct(const CorrectArgs &A, int maxcols, int maxez, int maxghost, hipStream_t s);
 // the ghost faces of the caller's boxes: box and periodic images (fill),
 // then the physical edge-velocity rules of every non-periodic side whose

@@ -41,11 +41,10 @@ template <typename T>
 struct Hier {
     int nlev = 0, lc = 0;
     std::vector<Lev<T>> lev;
-    Lev<T> *lev_dev = nullptr;
     std::vector<void *> allocs;
     bool built = false;
     std::vector<T *> alpha;   // per-level alpha storage (mac_solve), in the level's allocation
-    bool alpha_on = false;    // whether lev[].alpha (and lev_dev) point at it
+    bool alpha_on = false;    // whether lev[].alpha point at it
     // FP32 3D level 0 only: the rho form of the finest level (parts of its
     // allocation, so the row kernels reach them through the weights' buffer)
     RhoLev rho0 = {};
@@ -258,11 +257,9 @@ extern "C" const char *mac_version(void) { return "maestro_mac 0.1 (gfx950)"; }
 
 // ------------------------------------------------------------ hierarchy
 
-// Levels of at most this many cells run inside the single-workgroup coarse
-// cycle (8^3 in 3D, 32^2 in 2D).  A 16^3 level fits its LDS in FP32 but is
-// slower there than as separate multi-block launches: one workgroup runs on
-// one CU.
-static int coarse_threshold(int dim) { return dim == 3 ? 512 : 1024; }
+// Levels of at most this many cells (8^3 in 3D, 32^2 in 2D) keep Gauss-Seidel
+// sweeps where the others are over-relaxed
+static long relaxed_above(int dim) { return dim == 3 ? 512 : 1024; }
 
 template <typename T>
 static int build_hier(mac_plan *P, Hier<T> &H)
@@ -306,11 +303,11 @@ static int build_hier(mac_plan *P, Hier<T> &H)
         T *rho_p = nullptr, *cxy_p = nullptr, *cz_p = nullptr, *bzl_p = nullptr;
         T **arr[15] = {&L.phi, &L.phi2, &L.rhs, &L.res, &L.bx, &L.by, &L.bz, &L.bxh, &L.byh, &L.bzh, &alpha_part,
                        &rho_p, &cxy_p, &cz_p, &bzl_p};
-        // second iterate: ping-pong of the fused 3D sweep, and on level 0
-        // the output of the fused refinement update
-        const bool has2 = P->dim == 3 || l == 0, d3 = P->dim == 3;
+        // phi2, the second iterate: ping-pong of the fused 3D sweep and of the
+        // legs, and on level 0 the output of the fused refinement update
+        const bool d3 = P->dim == 3;
         const bool rh = sizeof(T) == 4 && l == 0 && d3;
-        const long len[15] = {nc, has2 ? nc : 0, nc, nc, nc, nc, d3 ? nc : 0, (long)n[1] * n[2],
+        const long len[15] = {nc, nc, nc, nc, nc, nc, d3 ? nc : 0, (long)n[1] * n[2],
                               (long)n[0] * n[2], d3 ? (long)n[0] * n[1] : 0, nc,
                               rh ? nc : 0, rh ? (long)n[2] : 0, rh ? (long)n[2] + 1 : 0, rh ? (long)n[0] * n[1] : 0};
         auto part = [](long cnt) { return ((cnt * (long)sizeof(T) + 255) / 256) * 256; };
@@ -329,15 +326,10 @@ static int build_hier(mac_plan *P, Hier<T> &H)
         H.alpha.push_back(alpha_part);
         for (int d = 0; d < P->dim; ++d) { n[d] /= 2; h[d] *= 2.0; }
     }
-    int thr = coarse_threshold(P->dim);
-    H.lc = nl - 1;
-    for (int l = 0; l < nl; ++l)
-        if ((long)H.lev[l].nx * H.lev[l].ny * H.lev[l].nz <= thr) { H.lc = l; break; }
-    void *q = nullptr;
-    HIPCHK(hipMalloc(&q, sizeof(Lev<T>) * nl));
-    H.allocs.push_back(q);
-    H.lev_dev = (Lev<T> *)q;
-    HIPCHK(hipMemcpy(H.lev_dev, H.lev.data(), sizeof(Lev<T>) * nl, hipMemcpyHostToDevice));
+    // the single-workgroup cycle takes over at level lc; a bottom too large for
+    // it is solved alone
+    H.lc = coarse_first<T>(P->dim, H.lev.data(), nl);
+    if (H.lc < 0) H.lc = nl - 1;
     // bottom solver scratch (doubles)
     const Lev<T> &B = H.lev[nl - 1];
     long nb = (long)B.nx * B.ny * B.nz;
@@ -368,7 +360,6 @@ static int set_alpha(mac_plan *P, Hier<T> &H, bool on)
 {
     if (!H.built || on == H.alpha_on) return MAC_OK;
     for (int l = 0; l < H.nlev; ++l) H.lev[l].alpha = on ? H.alpha[l] : nullptr;
-    HIPCHK(hipMemcpyAsync(H.lev_dev, H.lev.data(), sizeof(Lev<T>) * H.nlev, hipMemcpyHostToDevice, P->stream));
     H.alpha_on = on;
     return MAC_OK;
 }
@@ -487,29 +478,50 @@ static void cycle_from(mac_plan *P, Hier<T> &H, int l, int type, bool zero, cons
     Lev<T> &L = H.lev[l];
     const long n = (long)L.nx * L.ny * L.nz;
     if (l == H.lc) {
-        // below level 0 the fused restriction has zeroed the iterate already
-        if (zero && (l == 0 || !use_fused(P))) launch_fill<T>(L.phi, n, T(0), s);
+        const CoarseOpts co = coarse_opts(P, type);
         int q = prof_begin(P, MAC_PROF_COARSE);
-        launch_coarse_cycle<T>(dim, H.lev_dev, H.lev.data(), H.lc, H.nlev, coarse_opts(P, type), P->cg, s);
+        if (!launch_coarse<T>(dim, H.lev.data(), H.lc, H.nlev, co, zero, s)) {
+            if (zero) launch_fill<T>(L.phi, n, T(0), s);
+            launch_bottom<T>(dim, L, co, P->cg, s);
+        }
         prof_end(P, q);
         return;
     }
     const int again = second_visit(type);
-    if (use_fused(P)) {
+    // legs: the level's way down or up in one launch each, where its size and
+    // the number of sweeps allow
+    const bool leg = leg_ok<T>(dim, L) && !(l == 0 && (K || Rh));
+    if (use_fused(P) || (leg && o.nu1 == 2 && o.nu2 == 2)) {
         int cur = 0;   // 1: the iterate is in phi2
         const Compact16 *Kl = l == 0 ? K : nullptr;
         const RhoLev *Rl = l == 0 ? Rh : nullptr;
-        if (o.nu1 > 0) fused_sweeps<T>(P, H, l, o.nu1, zero ? SWEEP_ZERO : SWEEP_PLAIN, cur, Kl, Rl);
-        else if (zero) launch_fill<T>(L.phi, n, T(0), s);
-        int q = (l == 0) ? prof_begin(P, sizeof(T) == 8 ? MAC_PROF_RESTRICT64 : MAC_PROF_RESTRICT32) : -1;
-        // also zeroes level l + 1's iterate
-        if (!launch_resid_restrict<T>(dim, L, cur ? L.phi2 : L.phi, H.lev[l + 1], s, Kl, Rl))
-            P->launch_failed = true;
-        prof_end(P, q);
+        if (leg && o.nu1 == 2) {
+            const int cls = zero ? (sizeof(T) == 8 ? MAC_PROF_GSRB64_ZERO : MAC_PROF_GSRB32_ZERO)
+                                 : (sizeof(T) == 8 ? MAC_PROF_GSRB64 : MAC_PROF_GSRB32);
+            int q = (l == 0) ? prof_begin(P, cls) : -1;
+            launch_leg_down<T>(dim, L, L.phi, L.phi2, zero, H.lev[l + 1], s);
+            prof_end(P, q);
+            cur = 1;
+        } else {
+            if (o.nu1 > 0) fused_sweeps<T>(P, H, l, o.nu1, zero ? SWEEP_ZERO : SWEEP_PLAIN, cur, Kl, Rl);
+            else if (zero) launch_fill<T>(L.phi, n, T(0), s);
+            int q = (l == 0) ? prof_begin(P, sizeof(T) == 8 ? MAC_PROF_RESTRICT64 : MAC_PROF_RESTRICT32) : -1;
+            // also zeroes level l + 1's iterate
+            if (!launch_resid_restrict<T>(dim, L, cur ? L.phi2 : L.phi, H.lev[l + 1], s, Kl, Rl))
+                P->launch_failed = true;
+            prof_end(P, q);
+        }
         cycle_from<T>(P, H, l + 1, type, true, K);
         if (again) cycle_from<T>(P, H, l + 1, again, false, K);
-        prolong_cur<T>(P, H, l, cur);
-        if (o.nu2 > 0) fused_sweeps<T>(P, H, l, o.nu2, SWEEP_PLAIN, cur, Kl, Rl);
+        if (leg && o.nu2 == 2) {
+            int q = (l == 0) ? prof_begin(P, sizeof(T) == 8 ? MAC_PROF_GSRB64 : MAC_PROF_GSRB32) : -1;
+            launch_leg_up<T>(dim, L, cur ? L.phi2 : L.phi, cur ? L.phi : L.phi2, H.lev[l + 1], P->bc, s);
+            prof_end(P, q);
+            cur ^= 1;
+        } else {
+            prolong_cur<T>(P, H, l, cur);
+            if (o.nu2 > 0) fused_sweeps<T>(P, H, l, o.nu2, SWEEP_PLAIN, cur, Kl, Rl);
+        }
         if (cur)   // bring the iterate back to phi
             HIPCHK_V(hipMemcpyAsync(L.phi, L.phi2, sizeof(T) * (size_t)n, hipMemcpyDeviceToDevice, s));
         return;
@@ -708,9 +720,13 @@ static double sweep_omega(const mac_plan *P)
 }
 
 template <typename T>
-static void set_omega(Hier<T> &H, double w)
+static void set_omega(int dim, Hier<T> &H, double w)
 {
-    for (int l = 0; l < H.nlev; ++l) H.lev[l].omega = (l < H.lc) ? (T)w : T(1);
+    for (int l = 0; l < H.nlev; ++l) {
+        const Lev<T> &L = H.lev[l];
+        const bool small = (long)L.nx * L.ny * L.nz <= relaxed_above(dim) || l == H.nlev - 1;
+        H.lev[l].omega = small ? T(1) : (T)w;
+    }
 }
 
 static int solve(mac_plan *P, mac_stats *st)
@@ -726,7 +742,7 @@ static int solve(mac_plan *P, mac_stats *st)
     HIPCHK(hipMemsetAsync(res_slot(P), 0, sizeof(unsigned long long), P->stream));
     if (o.precision == MAC_PREC_MIXED || o.precision == MAC_PREC_MIXED_BF16) {
         if ((rc = build_hier<float>(P, P->H32))) return rc;
-        set_omega(P->H32, sweep_omega(P));
+        set_omega(P->dim, P->H32, sweep_omega(P));
         // alpha in FP32 (from the FP64 level 0 and by coarsening) where the FP64 level has it
         if ((rc = set_alpha<float>(P, P->H32, P->helm && P->H64.alpha_on))) return rc;
         const Compact16 *K = nullptr;
@@ -758,7 +774,6 @@ static int solve(mac_plan *P, mac_stats *st)
         const Lev<float> &E = P->H32.lev[0];
         const int per_step = inner_per_step(o, K != nullptr);
         Lev<double> &L0 = P->H64.lev[0];
-        bool swapped = false;
         while (rc == MAC_OK && !converged(o, r, r0) && it < o.max_iter) {
             for (int c = 0; c < per_step; ++c) {
                 vcycle<float>(P, P->H32, c == 0, K, Rh);
@@ -771,19 +786,14 @@ static int solve(mac_plan *P, mac_stats *st)
                                       K ? K->rhs : nullptr);
             prof_end(P, q);
             std::swap(L0.phi, L0.phi2);
-            swapped = !swapped;
             if ((rc = read_norm(P, &r))) break;
             if (P->launch_failed) { rc = MAC_ERR_INVALID; break; }
             ++it;
             if (o.verbose) fprintf(stderr, "maestro_mac: IR step %d  res/res0 = %.3e\n", it, r / r0);
         }
-        // the device copy of the level table follows the buffer swaps, on
-        // every exit of the loop (a later coarse cycle may read level 0)
-        if (swapped)
-            HIPCHK(hipMemcpyAsync(P->H64.lev_dev, &L0, sizeof(Lev<double>), hipMemcpyHostToDevice, P->stream));
         if (rc) return rc;
     } else {
-        set_omega(P->H64, sweep_omega(P));
+        set_omega(P->dim, P->H64, sweep_omega(P));
         // the FP64 hierarchy's coarse weights (the mixed paths coarsen the FP32 one)
         coarsen_all<double>(P, P->H64);
         int bad = 0;
@@ -1759,14 +1769,14 @@ extern "C" int mac_debug_op(mac_plan *P, int level, int op, int count)
     if (!P || level < 0 || level >= P->H64.nlev || count < 0) return MAC_ERR_INVALID;
     if (!(P->opts.omega >= 0 && P->opts.omega < 2)) return MAC_ERR_INVALID;
     Hier<double> &H = P->H64;
-    set_omega(H, sweep_omega(P));
+    set_omega(P->dim, H, sweep_omega(P));
     const Lev<double> &L = H.lev[level];
     hipStream_t s = P->stream;
     bool has_next = level + 1 < H.nlev;
     if (op == MAC_OP_GSRB32) {
         int rc;
         if ((rc = build_hier<float>(P, P->H32))) return rc;
-        set_omega(P->H32, sweep_omega(P));
+        set_omega(P->dim, P->H32, sweep_omega(P));
         const Lev<float> &F = P->H32.lev[level];
         const long n = (long)L.nx * L.ny * L.nz;
         launch_weights_to_f32(P->dim, L, F, s);
@@ -1794,7 +1804,7 @@ extern "C" int mac_debug_op(mac_plan *P, int level, int op, int count)
     if (op == MAC_OP_GSRB32_RHO) {
         if (level != 0 || !P->H32.built || !P->H32.rho0.rho || !rho_level_ok(P->dim, P->H32.lev[0]))
             return MAC_ERR_INVALID;
-        set_omega(P->H32, sweep_omega(P));
+        set_omega(P->dim, P->H32, sweep_omega(P));
         const Lev<float> &F = P->H32.lev[0];
         const long n = (long)L.nx * L.ny * L.nz;
         launch_convert<double, float>(L.phi, F.phi, n, s);
@@ -2552,7 +2562,7 @@ static int ml_inner_f32(mac_plan *P)
 {
     int rc;
     if ((rc = build_hier<float>(P, P->H32))) return rc;
-    set_omega(P->H32, sweep_omega(P));
+    set_omega(P->dim, P->H32, sweep_omega(P));
     if ((rc = set_alpha<float>(P, P->H32, P->helm && P->H64.alpha_on))) return rc;
     launch_weights_to_f32(P->dim, P->H64.lev[0], P->H32.lev[0], P->stream);
     coarsen_all<float>(P, P->H32);
@@ -2695,7 +2705,7 @@ static int ml_project_dev(mac_ml_plan *M, double *const *const *umac, double *co
         ml_inner_opts(M, P);
         // the weights stay for the whole call: the hierarchy once
         if (M->opts.precision == MAC_PREC_FP64) {
-            set_omega(P->H64, sweep_omega(P));
+            set_omega(P->dim, P->H64, sweep_omega(P));
             coarsen_all<double>(P, P->H64);
         } else if ((rc = ml_inner_f32(P))) {
             return rc;
