@@ -185,18 +185,15 @@ template <typename T>
 __device__ __forceinline__ void lin_w(int fi, int nc, int kind_lo, int kind_hi, int &P, int &Q,
                                       T &wp, T &wq)
 {
-    int p = fi >> 1;
-    int q = (fi & 1) ? p + 1 : p - 1;
+    const int p = fi >> 1, q = (fi & 1) ? p + 1 : p - 1;
+    const bool out = q < 0 || q >= nc;
+    const int kind = (q < 0) ? kind_lo : kind_hi;
     P = p;
     wp = T(0.75);
-    wq = T(0.25);
-    if (q < 0 || q >= nc) {
-        int kind = (q < 0) ? kind_lo : kind_hi;
-        if (kind == ELL_PER) q = (q + nc) % nc;
-        else if (kind == ELL_DIR) { q = p; wq = T(-0.25); }
-        else q = p;
-    }
-    Q = q;
+    // selects, no branch: the parent (Neumann, Dirichlet with -1/4) or the
+    // periodic image stands in for a point outside
+    wq = (out && kind == ELL_DIR) ? T(-0.25) : T(0.25);
+    Q = !out ? q : (kind == ELL_PER ? (q < 0 ? nc - 1 : 0) : p);
 }
 
 struct EllBC {

@@ -98,43 +98,64 @@ struct Pair {
     T den[2], inv[2], rhs[2];
 };
 
-// the pair with left cell (i, j, k), i even, of a level with even nx
+// what a pair is made of, as loaded
 template <int DIM, typename T>
-__device__ __forceinline__ Pair<DIM, T> load_pair(const Lev<T> &L, int i, int j, int k)
+struct PairRaw {
+    Two<T> x, yl, yh, zl, zh, r, al;
+    T xh;
+};
+
+// of the pair with left cell (i, j, k), i even, of a level with even nx
+template <int DIM, typename T>
+__device__ __forceinline__ PairRaw<DIM, T> load_raw(const Lev<T> &L, int i, int j, int k)
 {
     const int nx = L.nx, ny = L.ny, nz = L.nz, plane = nx * ny;
     const int c = i + nx * (j + ny * k);
-    const Two<T> xa = load2(L.bx + c);
-    const T xh = (i + 2 < nx) ? L.bx[c + 2] : L.bxh[j + ny * k];
-    const Two<T> yl = load2(L.by + c), yh = load2(j < ny - 1 ? L.by + c + nx : L.byh + i + nx * k);
-    Two<T> zl{T(0), T(0)}, zh{T(0), T(0)}, al{T(-0.0), T(-0.0)};
+    PairRaw<DIM, T> R;
+    R.x = load2(L.bx + c);
+    R.xh = *((i + 2 < nx) ? L.bx + c + 2 : L.bxh + j + ny * k);
+    R.yl = load2(L.by + c);
+    R.yh = load2(j < ny - 1 ? L.by + c + nx : L.byh + i + nx * k);
     if constexpr (DIM == 3) {
-        zl = load2(L.bz + c);
-        zh = load2(k < nz - 1 ? L.bz + c + plane : L.bzh + i + nx * j);
+        R.zl = load2(L.bz + c);
+        R.zh = load2(k < nz - 1 ? L.bz + c + plane : L.bzh + i + nx * j);
     }
-    const Two<T> r = load2(L.rhs + c);
-    if (L.alpha) al = load2(L.alpha + c);
+    R.r = load2(L.rhs + c);
+    R.al = Two<T>{T(-0.0), T(-0.0)};
+    if (L.alpha) R.al = load2(L.alpha + c);
+    return R;
+}
+
+// s: j + k is odd
+template <int DIM, typename T>
+__device__ __forceinline__ Pair<DIM, T> make_pair(const Lev<T> &L, const PairRaw<DIM, T> &R, bool s)
+{
     T l[2 * DIM], h[2 * DIM];   // left and right cell
-    l[0] = xa.a; l[1] = xa.b; l[2] = yl.a; l[3] = yh.a;
-    h[0] = xa.b; h[1] = xh;   h[2] = yl.b; h[3] = yh.b;
+    l[0] = R.x.a; l[1] = R.x.b; l[2] = R.yl.a; l[3] = R.yh.a;
+    h[0] = R.x.b; h[1] = R.xh;  h[2] = R.yl.b; h[3] = R.yh.b;
     if constexpr (DIM == 3) {
-        l[4] = zl.a; l[5] = zh.a;
-        h[4] = zl.b; h[5] = zh.b;
+        l[4] = R.zl.a; l[5] = R.zh.a;
+        h[4] = R.zl.b; h[5] = R.zh.b;
     }
-    const bool s = (j + k) & 1;
     Pair<DIM, T> P;
 #pragma unroll
     for (int q = 0; q < 2 * DIM; ++q) {
         P.w[0][q] = s ? h[q] : l[q];
         P.w[1][q] = s ? l[q] : h[q];
     }
-    P.rhs[0] = s ? r.b : r.a;
-    P.rhs[1] = s ? r.a : r.b;
-    P.den[0] = gs_den<DIM, T>(L, P.w[0], s ? al.b : al.a);
-    P.den[1] = gs_den<DIM, T>(L, P.w[1], s ? al.a : al.b);
+    P.rhs[0] = s ? R.r.b : R.r.a;
+    P.rhs[1] = s ? R.r.a : R.r.b;
+    P.den[0] = gs_den<DIM, T>(L, P.w[0], s ? R.al.b : R.al.a);
+    P.den[1] = gs_den<DIM, T>(L, P.w[1], s ? R.al.a : R.al.b);
 #pragma unroll
-    for (int c2 = 0; c2 < 2; ++c2) P.inv[c2] = T(1) / P.den[c2];
+    for (int c = 0; c < 2; ++c) P.inv[c] = T(1) / P.den[c];
     return P;
+}
+
+template <int DIM, typename T>
+__device__ __forceinline__ Pair<DIM, T> load_pair(const Lev<T> &L, int i, int j, int k)
+{
+    return make_pair<DIM, T>(L, load_raw<DIM, T>(L, i, j, k), (j + k) & 1);
 }
 
 // a pair outside the domain: its cells stay zero through every update
@@ -222,17 +243,37 @@ struct LegTile {
     static constexpr int PX = HX + 2, PY = RY + 2, PZ = DIM == 3 ? RZ + 2 : 1;
     static constexpr int NPAIR = HX * RY * RZ, NPOS = PX * PY * PZ;
     static constexpr int SY = PX, SZ = PX * PY;
+    // coarse rows and planes that a way up reads: the parents of the ring's
+    // cells and one more on each side
+    static constexpr int RYC = PY / 2 + 2, RZC = DIM == 3 ? PZ / 2 + 2 : 1;
 };
 
-// the domain's image of g; false outside a non-periodic side
+// lin_w for a row or plane index that is not wrapped: the periodic image of
+// Q stands at Q itself
+template <typename T>
+__device__ __forceinline__ void row_w(int g, int nc, int kind_lo, int kind_hi, int &P, int &Q, T &wp, T &wq)
+{
+    const int p = g >> 1, q = (g & 1) ? p + 1 : p - 1;
+    const int kind = q < 0 ? kind_lo : (q >= nc ? kind_hi : ELL_PER);
+    P = p;
+    Q = kind == ELL_PER ? q : p;
+    wp = T(0.75);
+    wq = kind == ELL_DIR ? T(-0.25) : T(0.25);
+}
+
+// the domain's image of g; false outside a non-periodic side.  per: 0 not
+// periodic, 1 one period reaches (selects), 2 the region spans several
 __device__ __forceinline__ bool wrap_into(int &g, int n, int per)
 {
     if (per) {
-        while (g < 0) g += n;
-        while (g >= n) g -= n;
-        return true;
+        g = g < 0 ? g + n : g;
+        g = g >= n ? g - n : g;
+        if (per == 2) {
+            while (g < 0) g += n;
+            while (g >= n) g -= n;
+        }
     }
-    return g >= 0 && g < n;
+    return (unsigned)g < (unsigned)n;
 }
 
 // UP false: two sweeps of pin -> pout (MODE SWEEP_ZERO: pin is zero and not
@@ -251,6 +292,10 @@ __global__ void __launch_bounds__(NTH) k_leg(Lev<T> L, const T *__restrict__ pin
     const int tz = idx / (ntx * nty), tr = idx - tz * (ntx * nty), ty = tr / ntx, tx = tr - ty * ntx;
     const int x0 = tx * TX - 4, y0 = ty * TY - H, z0 = DIM == 3 ? tz * TZ - H : 0;   // the region's low corner
     const int nx = L.nx, ny = L.ny, nz = L.nz;
+    // a tile starts inside the domain, so an extent of at least a tile and its
+    // halo (coarse rows: half of both) is wrapped once
+    const int px = L.perx ? (nx < TX + 8 ? 2 : 1) : 0, py = L.pery ? (ny < TY + 8 ? 2 : 1) : 0;
+    const int pz = L.perz ? (nz < TZ + 8 ? 2 : 1) : 0;
     __shared__ T S[2][G::NPOS];
     // ---- pair weights of the region, all loads in flight together
     Pair<DIM, T> P[NP];
@@ -264,12 +309,38 @@ __global__ void __launch_bounds__(NTH) k_leg(Lev<T> L, const T *__restrict__ pin
         int gi = x0 + 2 * m, gj = y0 + jj, gk = z0 + kk;
         s[a] = (gj + gk) & 1;
         bool live = q < G::NPAIR;
-        live = wrap_into(gi, nx, L.perx) && live;
-        live = wrap_into(gj, ny, L.pery) && live;
-        if constexpr (DIM == 3) live = wrap_into(gk, nz, L.perz) && live;
+        live = wrap_into(gi, nx, px) && live;
+        live = wrap_into(gj, ny, py) && live;
+        if constexpr (DIM == 3) live = wrap_into(gk, nz, pz) && live;
         if (live) P[a] = load_pair<DIM, T>(L, gi, gj, gk);
         else P[a] = dead_pair<DIM, T>();
         if (q >= G::NPAIR) pos[a] = 0;   // a ring corner that no cell reads
+    }
+    // ---- going up: the coarse rows that the region touches, interpolated in x
+    // to its pairs (both cells), so a cell reads 4 values instead of 12
+    const int JB = (y0 - 1) / 2 - 1, KB = DIM == 3 ? (z0 - 1) / 2 - 1 : 0;   // y0 - 1, z0 - 1 are even
+    __shared__ Two<T> xr[UP ? G::PX * G::RYC * G::RZC : 1];
+    if constexpr (UP) {
+        for (int q = threadIdx.x; q < G::PX * G::RYC * G::RZC; q += NTH) {
+            const int m = q % G::PX, r = q / G::PX;
+            int gi = x0 - 2 + 2 * m, J = JB + r % G::RYC, K = KB + r / G::RYC;
+            bool live = wrap_into(gi, nx, px);
+            live = wrap_into(J, C.ny, py) && live;
+            if constexpr (DIM == 3) live = wrap_into(K, C.nz, pz) && live;
+            Two<T> v{T(0), T(0)};
+            if (live) {
+                int pc, ql, qr;
+                T wp, wl, wr;
+                lin_w<T>(gi, C.nx, bc.k[0][0], bc.k[0][1], pc, ql, wp, wl);
+                lin_w<T>(gi + 1, C.nx, bc.k[0][0], bc.k[0][1], pc, qr, wp, wr);
+                const T *e = C.phi + C.nx * (J + C.ny * K);
+                const T ep = wp * e[pc];
+                v.a = dfma(wl, e[ql], ep);
+                v.b = dfma(wr, e[qr], ep);
+            }
+            xr[q] = v;
+        }
+        __syncthreads();
     }
     // ---- the iterate of the region and its ring
     for (int q = threadIdx.x; q < G::NPOS; q += NTH) {
@@ -278,18 +349,34 @@ __global__ void __launch_bounds__(NTH) k_leg(Lev<T> L, const T *__restrict__ pin
         const bool sq = (gj + gk) & 1;
         Two<T> v{T(0), T(0)};
         if (UP || !zero) {
-            bool live = wrap_into(gi, nx, L.perx);
-            live = wrap_into(gj, ny, L.pery) && live;
-            if constexpr (DIM == 3) live = wrap_into(gk, nz, L.perz) && live;
+            const int uj = gj, uk = gk;   // not wrapped
+            bool live = wrap_into(gi, nx, px);
+            live = wrap_into(gj, ny, py) && live;
+            if constexpr (DIM == 3) live = wrap_into(gk, nz, pz) && live;
             if (live) {
                 v = load2(pin + gi + nx * (gj + ny * gk));
                 if constexpr (UP) {
-                    const T *e = C.phi;
-                    const Two<T> d = prolong_pair<DIM, T>(C.nx, C.ny, C.nz, bc, gi, gj, gk, [&](int I, int J, int K) {
-                        return e[I + C.nx * (J + C.ny * K)];
-                    });
-                    v.a = v.a + d.a;
-                    v.b = v.b + d.b;
+                    // y and z of prolong_value from the rows' x parts
+                    int y0r, y1r, z0r = 0, z1r = 0;
+                    T wy0, wy1, wz0 = T(1), wz1 = T(0);
+                    row_w(uj, C.ny, bc.k[1][0], bc.k[1][1], y0r, y1r, wy0, wy1);
+                    if constexpr (DIM == 3) row_w(uk, C.nz, bc.k[2][0], bc.k[2][1], z0r, z1r, wz0, wz1);
+                    const Two<T> *e = xr + m - G::PX * (JB + (DIM == 3 ? G::RYC * KB : 0));
+                    T vl[2], vr[2];
+#pragma unroll
+                    for (int cz = 0; cz < (DIM == 3 ? 2 : 1); ++cz) {
+                        const int kr = DIM == 3 ? G::RYC * (cz ? z1r : z0r) : 0;
+                        const Two<T> a = e[G::PX * (y0r + kr)], d = e[G::PX * (y1r + kr)];
+                        vl[cz] = dfma(wy1, d.a, wy0 * a.a);
+                        vr[cz] = dfma(wy1, d.b, wy0 * a.b);
+                    }
+                    if constexpr (DIM == 3) {
+                        v.a = v.a + dfma(wz1, vl[1], wz0 * vl[0]);
+                        v.b = v.b + dfma(wz1, vr[1], wz0 * vr[0]);
+                    } else {
+                        v.a = v.a + vl[0];
+                        v.b = v.b + vr[0];
+                    }
                 }
             }
         }
@@ -386,20 +473,27 @@ bool leg_ok(int dim, const Lev<T> &L)
     return n <= (dim == 3 ? LEG_MAX_3D : LEG_MAX_2D);
 }
 
+// The tile: the smallest that gives at most one block per CU (256), else the
+// largest.  A larger tile repeats less of its halo, a smaller one spreads a
+// small level over more CUs.  Down / up, microseconds: 32^3 FP32 8 x 4 x 4
+// (256 blocks) 6.0 / 6.2, 4 x 4 x 4 (512) 8.9 / 9.3, 8 x 8 x 8 (64) 7.2 / 8.1;
+// 64^3 FP32 16 x 8 x 8 (256) 10.8 / 11.5, 8 x 8 x 8 (512) 11.9 / 16.7, FP64
+// 8 x 8 x 8 18.9 / 19.9, 16 x 8 x 4 (512) 21.5 / 22.6.
 template <typename T, bool UP>
 static void launch_leg(int dim, const Lev<T> &L, const T *pin, T *pout, const Lev<T> &C, const EllBC &bc, bool zero,
                        hipStream_t s)
 {
-    const long n = (long)L.nx * L.ny * L.nz;
-    if (dim == 2) {
+    auto tiles = [&](int tx, int ty, int tz) {
+        return (long)((L.nx + tx - 1) / tx) * ((L.ny + ty - 1) / ty) * ((L.nz + tz - 1) / tz);
+    };
+    if (dim == 2)
         launch_leg_t<2, T, 32, 32, 1, 832, UP>(L, pin, pout, C, bc, zero, s);
-    } else if (n <= LEG_SMALL_3D) {
-        launch_leg_t<3, T, 4, 4, 4, 896, UP>(L, pin, pout, C, bc, zero, s);
-    } else if constexpr (sizeof(T) == 4) {
-        launch_leg_t<3, T, 16, 8, 8, 1024, UP>(L, pin, pout, C, bc, zero, s);
-    } else {
+    else if (tiles(8, 4, 4) <= 256)
+        launch_leg_t<3, T, 8, 4, 4, sizeof(T) == 4 ? 1024 : 640, UP>(L, pin, pout, C, bc, zero, s);
+    else if (sizeof(T) == 8 || tiles(8, 8, 8) <= 256)
         launch_leg_t<3, T, 8, 8, 8, 1024, UP>(L, pin, pout, C, bc, zero, s);
-    }
+    else if constexpr (sizeof(T) == 4)
+        launch_leg_t<3, T, 16, 8, 8, 1024, UP>(L, pin, pout, C, bc, zero, s);
 }
 
 template <typename T>
@@ -442,26 +536,43 @@ __device__ __forceinline__ double lane_xor(double v)
     return __hiloint2double(lane_xor<MASK>(__double2hiint(v)), lane_xor<MASK>(__double2loint(v)));
 }
 
-// sum over the 64 lanes in a fixed order (butterfly): every lane holds the
-// same, deterministic result
+// v of lane i plus (or max with) v of lane i ^ 32, i ^ 16: the swap
+// instructions exchange the upper and lower halves (odd and even rows of 16)
+// of two registers, here of two copies of v
+template <int MASK, typename F>
+__device__ __forceinline__ double swap_op(double v, F &&f)
+{
+    static_assert(MASK == 32 || MASK == 16, "halves or rows");
+    const unsigned hi = (unsigned)__double2hiint(v), lo = (unsigned)__double2loint(v);
+    if constexpr (MASK == 32) {
+        const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        return f(__hiloint2double((int)h[0], (int)l[0]), __hiloint2double((int)h[1], (int)l[1]));
+    } else {
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        return f(__hiloint2double((int)h[0], (int)l[0]), __hiloint2double((int)h[1], (int)l[1]));
+    }
+}
+// over the 64 lanes in a fixed order (butterfly): every lane holds the same,
+// deterministic result
+template <typename F>
+__device__ __forceinline__ double wave_all(double v, F &&f)
+{
+    v = swap_op<32>(v, f);
+    v = swap_op<16>(v, f);
+    v = f(v, lane_xor<8>(v));
+    v = f(v, lane_xor<4>(v));
+    v = f(v, lane_xor<2>(v));
+    return f(v, lane_xor<1>(v));
+}
 __device__ __forceinline__ double wsum(double v)
 {
-    v += __shfl_xor(v, 32, 64);
-    v += __shfl_xor(v, 16, 64);
-    v += lane_xor<8>(v);
-    v += lane_xor<4>(v);
-    v += lane_xor<2>(v);
-    v += lane_xor<1>(v);
-    return v;
+    return wave_all(v, [](double a, double b) { return a + b; });
 }
 __device__ __forceinline__ double wmax(double v)
 {
-    v = fmax(v, __shfl_xor(v, 32, 64));
-    v = fmax(v, __shfl_xor(v, 16, 64));
-    v = fmax(v, lane_xor<8>(v));
-    v = fmax(v, lane_xor<4>(v));
-    v = fmax(v, lane_xor<2>(v));
-    return fmax(v, lane_xor<1>(v));
+    return wave_all(v, [](double a, double b) { return fmax(a, b); });
 }
 
 // ------------------------------------------------------- the bottom solve
@@ -469,7 +580,9 @@ __device__ __forceinline__ double wmax(double v)
 // (- mean on singular problems) to eps, nub sweeps.  The three forms differ
 // in how neighbours and sums reach a thread; X provides
 //   nbrs(v, p)      the 2 DIM neighbours' values of v (0 outside)
-//   sum(v), max(v)  over all cells, the same in every thread, fixed order
+//   nbrs_any(v, p)  the same, where has(s) is false any finite value
+//   sum(v), max(v), sum_max(s, m)  over all cells, the same in every thread,
+//                   fixed order
 // and says which threads hold a cell (live).
 template <int DIM, typename T, typename X>
 __device__ __forceinline__ T bottom_solve(const Lev<T> &L, X &x_, const T *w, T acell, int colour, T phi, T rhs,
@@ -477,20 +590,11 @@ __device__ __forceinline__ T bottom_solve(const Lev<T> &L, X &x_, const T *w, T 
 {
     const bool live = x_.live;
     const T den = gs_den<DIM, T>(L, w, acell), inv = T(1) / den;
-    auto sweeps = [&](int count) {
-        for (int it = 0; it < count; ++it)
-            for (int c = 0; c < 2; ++c) {
-                T p[2 * DIM];
-                x_.nbrs(phi, p);
-                const T v = quot(gs_num<DIM, T>(L, w, p, rhs), den, inv);
-                if (live && colour == c) phi = v;
-            }
-    };
-    sweeps(o.nub);
-    if (o.bottom == MAC_BOTTOM_SMOOTH) {
-        sweeps(o.nub);
-        return phi;
-    }
+    T wn[2 * DIM];   // for the sweeps' sums of neighbours
+#pragma unroll
+    for (int s = 0; s < 2 * DIM; ++s) wn[s] = x_.has(s) ? w[s] : T(0);
+    // the mean of a sum over the cells
+    auto mean = [&](double v) -> double { return X::POW2 ? v * (1.0 / n) : v / (double)n; };
     Lev<double> D;
     D.ih2x = L.ih2x; D.ih2y = L.ih2y; D.ih2z = L.ih2z;
     double wd[2 * DIM];
@@ -503,109 +607,150 @@ __device__ __forceinline__ T bottom_solve(const Lev<T> &L, X &x_, const T *w, T 
         const double ap = apply_w<DIM, double>(D, wd, p, v);
         return L.alpha ? fma((double)acell, v, ap) : ap;
     };
-    const double nd = (double)n;
-    const double m = o.singular ? x_.sum(live ? (double)rhs : 0.0) / nd : 0.0;
-    double x = live ? (double)phi : 0.0;
-    const double ax = apply(x);
-    double r = live ? ((double)rhs - m) - ax : 0.0;
-    auto project = [&]() {   // the mean off r on singular problems
-        if (o.singular) {
-            const double rm = x_.sum(r) / nd;
-            if (live) r -= rm;
+#pragma unroll 1
+    for (int part = 0; part < 2; ++part) {
+#pragma unroll 1
+        for (int h = 0; h < 2 * o.nub; ++h) {
+            T p[2 * DIM];
+            x_.nbrs_any(phi, p);
+            const T v = quot(gs_num<DIM, T>(L, wn, p, rhs), den, inv);
+            if (live && colour == (h & 1)) phi = v;
         }
-    };
-    project();
-    const double r0 = x_.max(fabs(r));
-    if (r0 > 0.0 && o.bottom == MAC_BOTTOM_BICGSTAB) {
-        // van der Vorst, SIAM J. Sci. Stat. Comput. 13 (1992) 631-644
-        // (FBoxLib's default, mg_bottom_solver = 1, mg.tex:242-243)
-        const double rh = r;
-        double p = 0.0, v = 0.0, rho_old = 1.0, al = 1.0, om = 1.0;
-        for (int it = 0; it < o.bottom_maxit; ++it) {
-            const double rho = x_.sum(rh * r);
-            if (rho == 0.0) break;
-            if (it == 0) p = r;
-            else p = r + ((rho / rho_old) * (al / om)) * (p - om * v);
-            v = apply(p);
-            const double rv = x_.sum(rh * v);
-            if (rv == 0.0) break;
-            al = rho / rv;
-            r -= al * v;
-            project();
-            if (x_.max(fabs(r)) <= o.bottom_eps * r0) {
-                x += al * p;
-                break;
+        if (part == 1 || o.bottom == MAC_BOTTOM_SMOOTH) continue;
+        const double m = o.singular ? mean(x_.sum(live ? (double)rhs : 0.0)) : 0.0;
+        double x = live ? (double)phi : 0.0;
+        const double ax = apply(x);
+        double r = live ? ((double)rhs - m) - ax : 0.0;
+        auto project = [&]() {   // the mean off r on singular problems
+            if (o.singular) {
+                const double rm = mean(x_.sum(r));
+                if (live) r -= rm;
             }
-            const double t = apply(r);
-            const double tt = x_.sum(t * t);
-            if (!(tt > 0.0)) {
-                x += al * p;
-                break;
+        };
+        project();
+        const double r0 = x_.max(fabs(r));
+        if (r0 > 0.0 && o.bottom == MAC_BOTTOM_BICGSTAB) {
+            // van der Vorst, SIAM J. Sci. Stat. Comput. 13 (1992) 631-644
+            // (FBoxLib's default, mg_bottom_solver = 1, mg.tex:242-243)
+            const double rh = r;
+            double p = 0.0, v = 0.0, rho_old = 1.0, al = 1.0, om = 1.0;
+#pragma unroll 1
+            for (int it = 0; it < o.bottom_maxit; ++it) {
+                const double rho = x_.sum(rh * r);
+                if (rho == 0.0) break;
+                if (it == 0) p = r;
+                else p = r + ((rho / rho_old) * (al / om)) * (p - om * v);
+                v = apply(p);
+                const double rv = x_.sum(rh * v);
+                if (rv == 0.0) break;
+                al = rho / rv;
+                r -= al * v;
+                project();
+                if (x_.max(fabs(r)) <= o.bottom_eps * r0) {
+                    x += al * p;
+                    break;
+                }
+                const double t = apply(r);
+                const double tt = x_.sum(t * t);
+                if (!(tt > 0.0)) {
+                    x += al * p;
+                    break;
+                }
+                om = x_.sum(t * r) / tt;
+                x += al * p + om * r;
+                r -= om * t;
+                project();
+                rho_old = rho;
+                if (x_.max(fabs(r)) <= o.bottom_eps * r0 || om == 0.0) break;
             }
-            om = x_.sum(t * r) / tt;
-            x += al * p + om * r;
-            r -= om * t;
-            project();
-            rho_old = rho;
-            if (x_.max(fabs(r)) <= o.bottom_eps * r0 || om == 0.0) break;
+        } else if (r0 > 0.0) {
+            double p = r;
+            double rr = x_.sum(r * r);
+#pragma unroll 1
+            for (int it = 0; it < o.bottom_maxit; ++it) {
+                const double irr = 1.0 / rr;   // off the chain of the step
+                const double Ap = apply(p);
+                const double pap = x_.sum(p * Ap);
+                if (!(pap > 0.0)) break;
+                const double alpha = rr / pap;
+                x += alpha * p;
+                r -= alpha * Ap;
+                project();
+                double rr1 = r * r, am = fabs(r);
+                x_.sum_max(rr1, am);
+                if (am <= o.bottom_eps * r0) break;
+                const double beta = quot(rr1, rr, irr);
+                rr = rr1;
+                p = r + beta * p;
+            }
         }
-    } else if (r0 > 0.0) {
-        double p = r;
-        double rr = x_.sum(r * r);
-        for (int it = 0; it < o.bottom_maxit; ++it) {
-            const double Ap = apply(p);
-            const double pap = x_.sum(p * Ap);
-            if (!(pap > 0.0)) break;
-            const double alpha = rr / pap;
-            x += alpha * p;
-            r -= alpha * Ap;
-            project();
-            const double am = x_.max(fabs(r));
-            const double rr1 = x_.sum(r * r);
-            if (am <= o.bottom_eps * r0) break;
-            const double beta = rr1 / rr;
-            rr = rr1;
-            p = r + beta * p;
-        }
+        phi = live ? (T)x : T(0);
     }
-    phi = live ? (T)x : T(0);
-    sweeps(o.nub);
     return phi;
 }
 
 // 2 cells per direction (2 x 2 x 2, or 2 x 2 in 2D): every group of 8 (4)
 // lanes of the wave solves the same problem, neighbours and sums by
-// data-parallel primitives.  The sums pair the lanes in the butterfly's order
+// data-parallel primitives.  In a sweep a side without a neighbour is left out
+// by a zero weight, so no value is selected.  The sums pair the lanes in the
+// butterfly's order
+// lane i ^ 4 where lanes 8 apart hold the same: a rotation by 4 in the row
+__device__ __forceinline__ float group_xor4(float v) { return __int_as_float(dpp<0x124>(__float_as_int(v))); }
+__device__ __forceinline__ double group_xor4(double v)
+{
+    return __hiloint2double(dpp<0x124>(__double2hiint(v)), dpp<0x124>(__double2loint(v)));
+}
 template <int DIM>
 struct BottomTwos {
-    bool live = true, in[2 * DIM];   // whether there is a neighbour on each side
+    static constexpr bool POW2 = true;   // 4 or 8 cells: 1 / n is exact
+    bool live = true, in[2 * DIM];       // whether there is a neighbour on each side
+    __device__ __forceinline__ bool has(int s) const { return in[s]; }
     template <typename V>
-    __device__ __forceinline__ void nbrs(V v, V *p) const
+    __device__ __forceinline__ void nbrs_any(V v, V *p) const
     {
         V o[3];
         o[0] = lane_xor<1>(v);
         o[1] = lane_xor<2>(v);
-        if constexpr (DIM == 3) o[2] = lane_xor<4>(v);
+        if constexpr (DIM == 3) o[2] = group_xor4(v);
 #pragma unroll
-        for (int s = 0; s < 2 * DIM; ++s) p[s] = in[s] ? o[s >> 1] : V(0);
+        for (int s = 0; s < 2 * DIM; ++s) p[s] = o[s >> 1];
+    }
+    template <typename V>
+    __device__ __forceinline__ void nbrs(V v, V *p) const
+    {
+        nbrs_any(v, p);
+#pragma unroll
+        for (int s = 0; s < 2 * DIM; ++s) p[s] = in[s] ? p[s] : V(0);
     }
     __device__ __forceinline__ double sum(double v) const
     {
-        if constexpr (DIM == 3) v += lane_xor<4>(v);
+        if constexpr (DIM == 3) v += group_xor4(v);
         v += lane_xor<2>(v);
         return v + lane_xor<1>(v);
     }
     __device__ __forceinline__ double max(double v) const
     {
-        if constexpr (DIM == 3) v = fmax(v, lane_xor<4>(v));
+        if constexpr (DIM == 3) v = fmax(v, group_xor4(v));
         v = fmax(v, lane_xor<2>(v));
         return fmax(v, lane_xor<1>(v));
+    }
+    __device__ __forceinline__ void sum_max(double &s, double &m) const
+    {
+        s = sum(s);
+        m = max(m);
     }
 };
 
 // at most 64 cells: one wave, neighbours by lane shuffles
 template <int DIM>
 struct BottomWave {
+    static constexpr bool POW2 = false;
+    __device__ __forceinline__ bool has(int) const { return true; }
+    template <typename V>
+    __device__ __forceinline__ void nbrs_any(V v, V *p)
+    {
+        nbrs(v, p);
+    }
     bool live;
     int nb[2 * DIM];   // neighbour lanes, -1 outside
     template <typename V>
@@ -619,6 +764,11 @@ struct BottomWave {
     }
     __device__ __forceinline__ double sum(double v) const { return wsum(v); }
     __device__ __forceinline__ double max(double v) const { return wmax(v); }
+    __device__ __forceinline__ void sum_max(double &s, double &m) const
+    {
+        s = wsum(s);
+        m = wmax(m);
+    }
 };
 
 // up to a block of cells: neighbours and sums through LDS, one barrier each
@@ -626,9 +776,16 @@ struct BottomWave {
 // all its readers have passed)
 template <int DIM>
 struct BottomBlock {
+    static constexpr bool POW2 = false;
+    __device__ __forceinline__ bool has(int) const { return true; }
+    template <typename V>
+    __device__ __forceinline__ void nbrs_any(V v, V *p)
+    {
+        nbrs(v, p);
+    }
     bool live;
     int nb[2 * DIM];      // neighbour cells; outside: the zero cell n
-    double *xs, *sh;      // two exchange arrays of n + 1 values; 2 x 32 partial sums
+    double *xs, *sh;      // two exchange arrays of n + 1 values; 2 x 32 partial results
     int n, flip, fs;
     template <typename V>
     __device__ __forceinline__ void nbrs(V v, V *p)
@@ -658,6 +815,7 @@ struct BottomBlock {
     {
         const double *a = post(wsum(v));
         double s = 0.0;
+#pragma unroll 1
         for (int w = 0; w < (n + 63) >> 6; ++w) s += a[w];
         return s;
     }
@@ -665,8 +823,23 @@ struct BottomBlock {
     {
         const double *a = post(wmax(v));
         double s = 0.0;
+#pragma unroll 1
         for (int w = 0; w < (n + 63) >> 6; ++w) s = fmax(s, a[w]);
         return s;
+    }
+    __device__ __forceinline__ void sum_max(double &s, double &m)   // one barrier for both
+    {
+        s = wsum(s);
+        m = wmax(m);
+        double *a = sh + 32 * fs;
+        if ((threadIdx.x & 63) == 0) a[16 + (threadIdx.x >> 6)] = m;
+        post(s);
+        s = m = 0.0;
+#pragma unroll 1
+        for (int w = 0; w < (n + 63) >> 6; ++w) {
+            s += a[w];
+            m = fmax(m, a[16 + w]);
+        }
     }
 };
 
@@ -687,47 +860,83 @@ __device__ __forceinline__ void cell_nbrs(const Lev<T> &L, int q, int none, int 
 }
 
 // ---------------------------------------------------------- the coarse cycle
-// LDS image, offsets in units of T: level 0 of the cycle (`lc` of the
-// hierarchy) takes its pair weights from global memory, into registers, on
-// its way down and again up; each level between it and the bottom has its
-// pairs' fields (weights, diagonals, reciprocals, rhs) as arrays over the
-// pairs; all have the iterate by colour (with a zero at the
-// end of each colour for neighbours outside) and, below level 0, as a plain
-// array for the prolongation.  The bottom: weights, alpha and rhs by cell.
+// LDS image, offsets in bytes.  Level 0 of the cycle (`lc` of the hierarchy)
+// has its iterate by colour at 0, its pairs' weights come from global memory
+// on the way down and again up.  A pair of a level between it and the bottom
+// belongs to one thread throughout, which keeps the weights in registers; LDS
+// holds the iterate by colour and, for the prolongation, as a plain array.  A
+// colour array ends in a zero cell for neighbours outside; colour 1 lies a
+// constant stride behind colour 0, so an access is one address and an
+// immediate offset.  The bottom: weights, alpha, rhs and iterate by cell.
 struct CoarseMap {
     int nl;                    // levels in the cycle
-    int S[COARSE_LEVELS], F[COARSE_LEVELS], E[COARSE_LEVELS];
+    int S[COARSE_LEVELS], E[COARSE_LEVELS];
     int rs, bw, br, xs, sh;    // pair residuals; bottom weights, rhs, exchange, sums
+    int park, mid;             // waiting pairs of the levels between, their number
+    // factors of fast_div by a row's pairs (the bottom: cells) and by the rows
+    unsigned mx[COARSE_LEVELS], my[COARSE_LEVELS];
     int bytes;
 };
+
+// pairs of all levels between the first and the bottom: one thread each
+static constexpr int COARSE_MID = COARSE_CELLS / 8 + 1;   // of one level, and the zero cell
+template <typename T> static constexpr int colour0() { return (COARSE_CELLS / 2 + 2) * (int)sizeof(T); }
+template <typename T> static constexpr int colour_mid() { return (COARSE_MID + 1) * (int)sizeof(T); }
+
+// q / d for q d < 2^32: the high word of q times m = floor(2^32 / d) + 1 (0: d = 1)
+__device__ __forceinline__ int fast_div(int q, unsigned m)
+{
+    return m ? (int)__umulhi((unsigned)q, m) : q;
+}
+static unsigned fast_div_factor(int d)
+{
+    return d == 1 ? 0u : (unsigned)(4294967296.0 / d) + 1u;
+}
+// position q of a row-major array of rows of nx in planes of ny rows
+struct Ijk {
+    int i, j, k;
+};
+__device__ __forceinline__ Ijk ijk_of(int q, int nx, int ny, unsigned mx, unsigned my)
+{
+    const int r = fast_div(q, mx), k = fast_div(r, my);
+    return Ijk{q - r * nx, r - k * ny, k};
+}
 
 template <typename T>
 struct CoarseLevs {
     Lev<T> l[COARSE_LEVELS];
 };
 
-template <int DIM>
-static constexpr int pair_fields() { return 2 * (2 * DIM + 3); }
-
-// positions of a pair's neighbours within a colour array of hx x ny x nz pairs
+// a pair: its place among its level's pairs and the LDS offsets (colour 0) of
+// itself, of the x neighbours across its ends (x[c]: colour c's) and of its
+// row and plane neighbours
 struct PairPos {
-    int q, xl, xr, ym, yp, zm, zp;
+    int q, m, j, k;
+    int at, x[2], ym, yp, zm, zp;
+    bool s, on;
 };
 template <int DIM, typename T>
-__device__ __forceinline__ PairPos pair_pos(const Lev<T> &L, int q)
+__device__ __forceinline__ PairPos pair_pos(const Lev<T> &L, int q, int S, unsigned mx, unsigned my)
 {
     const int hx = L.nx >> 1, ny = L.ny, nz = L.nz, sz = hx * ny, none = sz * nz;
-    const int m = q % hx, r = q / hx, j = r % ny, k = r / ny;
     PairPos o;
-    o.q = q;
-    o.xl = m > 0 ? q - 1 : (L.perx ? q + hx - 1 : none);
-    o.xr = m < hx - 1 ? q + 1 : (L.perx ? q - (hx - 1) : none);
-    o.ym = j > 0 ? q - hx : (L.pery ? q + (ny - 1) * hx : none);
-    o.yp = j < ny - 1 ? q + hx : (L.pery ? q - (ny - 1) * hx : none);
-    o.zm = o.zp = none;
+    o.on = q < none;
+    if (!o.on) q = 0;
+    const Ijk c = ijk_of(q, hx, ny, mx, my);
+    o.q = q; o.m = c.i; o.j = c.j; o.k = c.k;
+    o.s = (c.j + c.k) & 1;
+    auto off = [&](int p) { return S + p * (int)sizeof(T); };
+    o.at = off(q);
+    const int xl = off(c.i > 0 ? q - 1 : (L.perx ? q + hx - 1 : none));
+    const int xr = off(c.i < hx - 1 ? q + 1 : (L.perx ? q - (hx - 1) : none));
+    o.x[0] = o.s ? xr : xl;   // the red cell is the right one where s
+    o.x[1] = o.s ? xl : xr;
+    o.ym = off(c.j > 0 ? q - hx : (L.pery ? q + (ny - 1) * hx : none));
+    o.yp = off(c.j < ny - 1 ? q + hx : (L.pery ? q - (ny - 1) * hx : none));
+    o.zm = o.zp = 0;
     if constexpr (DIM == 3) {
-        o.zm = k > 0 ? q - sz : (L.perz ? q + (nz - 1) * sz : none);
-        o.zp = k < nz - 1 ? q + sz : (L.perz ? q - (nz - 1) * sz : none);
+        o.zm = off(c.k > 0 ? q - sz : (L.perz ? q + (nz - 1) * sz : none));
+        o.zp = off(c.k < nz - 1 ? q + sz : (L.perz ? q - (nz - 1) * sz : none));
     }
     return o;
 }
@@ -739,120 +948,112 @@ template <int DIM, typename T, bool VC>
 __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, CoarseMap M, CoarseOpts o, int zero)
 {
     extern __shared__ __align__(16) char smem_[];
-    T *sm = reinterpret_cast<T *>(smem_);
-    constexpr int NT = COARSE_THREADS, NP = COARSE_CELLS / 2 / NT, NF = pair_fields<DIM>();
+    constexpr int NT = COARSE_THREADS, NP = COARSE_CELLS / 2 / NT;
+    constexpr int C0 = colour0<T>(), CM = colour_mid<T>();
     const int t = threadIdx.x, bot = M.nl - 1;
-    // ---- stage: the iterate of level 0, the deeper levels' pairs and the
-    // bottom's weights into LDS
+    auto arr = [&](int off) -> T * { return reinterpret_cast<T *>(smem_ + off); };
+    auto ref = [&](int off) -> T & { return *reinterpret_cast<T *>(smem_ + off); };
     const Lev<T> &L0 = LV.l[0];
-    {
-        if (bot > 0) {
-            const int hx = L0.nx >> 1, h = hx * L0.ny * L0.nz;
+    // in 3D and FP64 (or the W and F shapes) the pairs of the levels between
+    // wait in LDS and come into registers for a leg: they would spill
+    constexpr bool PARK = DIM == 3 && (sizeof(T) == 8 || !VC);
+    Pair<DIM, T> Pm;      // the pair of a level between that this thread owns
+    PairPos om;
+    int lm = 0, qm = 0;   // that level (0: none), the pair's place in it
+    // the deeper levels' pairs, the bottom's weights and level 0's iterate
+    // (pairs at o0): every load issued before the first is waited for
+    auto stage = [&](const PairPos(&o0)[NP]) {
+        Two<T> v0[NP];
 #pragma unroll
-            for (int a = 0; a < NP; ++a) {
-                const int q = t + a * NT;
-                if (q < h) {
-                    const int r = q / hx;
-                    const bool s = (r % L0.ny + r / L0.ny) & 1;
-                    Two<T> v{T(0), T(0)};
-                    if (!zero) v = load2(L0.phi + 2 * q);
-                    sm[M.S[0] + q] = s ? v.b : v.a;
-                    sm[M.S[0] + h + 1 + q] = s ? v.a : v.b;
-                }
-            }
-            if (t < 2) sm[M.S[0] + (t + 1) * (h + 1) - 1] = T(0);
+        for (int a = 0; a < NP; ++a) {
+            v0[a] = Two<T>{T(0), T(0)};
+            if (bot > 0 && !zero) v0[a] = load2(L0.phi + 2 * o0[a].q);
         }
-        int first = 0;   // the flattened pairs of the levels between
+        PairRaw<DIM, T> Rm;
+        int first = 0;
         for (int l = 1; l < bot; ++l) {
             const Lev<T> &L = LV.l[l];
-            const int hx = L.nx >> 1, h = hx * L.ny * L.nz;
-            const int q = t - first;
-            first = (first + h) % NT;
-            // h <= NT / 2 pairs, laid over the threads one level after the other
-            const int qq = q < 0 ? q + NT : q;
-            if (qq < h) {
-                const int m = qq % hx, r = qq / hx, j = r % L.ny, k = r / L.ny;
-                const Pair<DIM, T> P = load_pair<DIM, T>(L, 2 * m, j, k);
-                T *f = sm + M.F[l] + qq;
+            const int h = (L.nx >> 1) * L.ny * L.nz;
+            if (t >= first && t < first + h) {
+                lm = l;
+                qm = t - first;
+                om = pair_pos<DIM, T>(L, qm, M.S[l], M.mx[l], M.my[l]);
+                Rm = load_raw<DIM, T>(L, 2 * om.m, om.j, om.k);
+            }
+            first += h;
+            if (t < 2) ref(M.S[l] + h * (int)sizeof(T) + t * CM) = T(0);   // the zero cells
+        }
+        const Lev<T> &L = LV.l[bot];
+        const int n = L.nx * L.ny * L.nz, nx = L.nx, ny = L.ny, nz = L.nz;
+        for (int q = NT - 1 - t; q < n; q += NT) {   // from the last thread: the first own other levels' pairs
+            const Ijk c = ijk_of(q, nx, ny, M.mx[bot], M.my[bot]);
+            const int i = c.i, j = c.j, k = c.k;
+            T *f = arr(M.bw) + q;
+            T g[2 * DIM + 1], r = T(0), p = T(0);
+            g[0] = L.bx[q];
+            g[1] = *((i < nx - 1) ? L.bx + q + 1 : L.bxh + j + ny * k);
+            g[2] = L.by[q];
+            g[3] = *((j < ny - 1) ? L.by + q + nx : L.byh + i + nx * k);
+            if constexpr (DIM == 3) {
+                g[4] = L.bz[q];
+                g[5] = *((k < nz - 1) ? L.bz + q + nx * ny : L.bzh + i + nx * j);
+            }
+            g[2 * DIM] = alpha_at(L, q);
+            if (bot == 0) {
+                r = L.rhs[q];
+                if (!zero) p = L.phi[q];
+            }
+#pragma unroll
+            for (int d = 0; d < 2 * DIM + 1; ++d) f[d * n] = g[d];
+            if (bot == 0) {
+                arr(M.br)[q] = r;
+                arr(M.E[0])[q] = p;
+            }
+        }
+        if (lm) {
+            Pm = make_pair<DIM, T>(LV.l[lm], Rm, om.s);
+            if constexpr (PARK) {
+                T *f = arr(M.park) + t;
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
 #pragma unroll
-                    for (int d = 0; d < 2 * DIM; ++d) f[(c * (2 * DIM + 3) + d) * h] = P.w[c][d];
-                    f[(c * (2 * DIM + 3) + 2 * DIM) * h] = P.den[c];
-                    f[(c * (2 * DIM + 3) + 2 * DIM + 1) * h] = P.inv[c];
-                }
-            }
-            if (t < 2) sm[M.S[l] + (t + 1) * (h + 1) - 1] = T(0);   // the zero cells
-        }
-        {
-            const Lev<T> &L = LV.l[bot];
-            const int n = L.nx * L.ny * L.nz, nx = L.nx, ny = L.ny, nz = L.nz;
-            for (int q = NT - 1 - t; q < n; q += NT) {   // from the last thread: the first hold other levels' pairs
-                const int i = q % nx, r = q / nx, j = r % ny, k = r / ny;
-                T *f = sm + M.bw + q;
-                f[0] = L.bx[q];
-                f[n] = (i < nx - 1) ? L.bx[q + 1] : L.bxh[j + ny * k];
-                f[2 * n] = L.by[q];
-                f[3 * n] = (j < ny - 1) ? L.by[q + nx] : L.byh[i + nx * k];
-                if constexpr (DIM == 3) {
-                    f[4 * n] = L.bz[q];
-                    f[5 * n] = (k < nz - 1) ? L.bz[q + nx * ny] : L.bzh[i + nx * j];
-                }
-                f[2 * DIM * n] = alpha_at(L, q);
-                if (bot == 0) {
-                    sm[M.br + q] = L.rhs[q];
-                    sm[M.E[0] + q] = zero ? T(0) : L.phi[q];
+                    for (int d = 0; d < 2 * DIM; ++d) f[(c * 2 * DIM + d) * M.mid] = Pm.w[c][d];
+                    f[(4 * DIM + c) * M.mid] = Pm.den[c];
+                    f[(4 * DIM + 2 + c) * M.mid] = Pm.inv[c];
                 }
             }
         }
-    }
-    __syncthreads();
-
-    // `count` sweeps of one pair set; v: the pairs' values, also in LDS
-    auto sweeps = [&](const Lev<T> &L, const auto &P, const auto &pos, const auto &s, const auto &on, auto &v, T *S, int h,
-                      int count, bool sor) {
-        constexpr int N = sizeof(P) / sizeof(P[0]);
-        for (int it = 0; it < count; ++it)
+        if (bot > 0) {
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                T *own = S + c * (h + 1), *oth = S + (1 - c) * (h + 1);
-#pragma unroll
-                for (int a = 0; a < N; ++a)
-                    if (on[a]) {
-                        T p[2 * DIM];
-                        pair_nbrs<DIM, T>(oth, s[a], c, v[a][1 - c], pos[a].xl, pos[a].xr, pos[a].ym, pos[a].yp,
-                                          pos[a].zm, pos[a].zp, p);
-                        v[a][c] = pair_update<DIM, T>(L, P[a], c, p, v[a][c], sor, L.omega);
-                        own[pos[a].q] = v[a][c];
-                    }
-                __syncthreads();
-            }
-    };
-    // the pairs' residuals into rs, then (after a barrier) the next level's
-    // right side and zero iterate
-    auto resid = [&](const Lev<T> &L, const auto &P, const auto &pos, const auto &s, const auto &on, const auto &v,
-                     const T *S, int h) {
-        constexpr int N = sizeof(P) / sizeof(P[0]);
-#pragma unroll
-        for (int a = 0; a < N; ++a)
-            if (on[a]) {
-                T res[2];
-#pragma unroll
-                for (int c = 0; c < 2; ++c) {
-                    T p[2 * DIM];
-                    pair_nbrs<DIM, T>(S + (1 - c) * (h + 1), s[a], c, v[a][1 - c], pos[a].xl, pos[a].xr, pos[a].ym,
-                                      pos[a].yp, pos[a].zm, pos[a].zp, p);
-                    T ap = apply_w<DIM, T>(L, P[a].w[c], p, v[a][c]);
-                    if (L.alpha) ap = dfma(L.alpha[2 * pos[a].q + (s[a] != (c == 1) ? 1 : 0)], v[a][c], ap);
-                    res[c] = P[a].rhs[c] - ap;
+            for (int a = 0; a < NP; ++a)
+                if (o0[a].on) {
+                    ref(o0[a].at) = o0[a].s ? v0[a].b : v0[a].a;
+                    ref(o0[a].at + C0) = o0[a].s ? v0[a].a : v0[a].b;
                 }
-                sm[M.rs + pos[a].q] = res[0] + res[1];
-            }
+            const int none = ((L0.nx >> 1) * L0.ny * L0.nz) * (int)sizeof(T);
+            if (t < 2) ref(none + t * C0) = T(0);
+        }
         __syncthreads();
     };
-    auto restricted = [&](const Lev<T> &F, int I, int J, int K) -> T {   // coarse cell from rs
+
+    // the neighbours of the pair's cell of colour c, in an iterate whose colours lie CS apart
+    auto nbrs = [&](const PairPos &o_, int c, int CS, T oth, T *p) {
+        const int d = (1 - c) * CS;
+        const bool right = o_.s != (c == 1);
+        const T xo = ref(o_.x[c] + d);
+        p[0] = right ? oth : xo;
+        p[1] = right ? xo : oth;
+        p[2] = ref(o_.ym + d);
+        p[3] = ref(o_.yp + d);
+        if constexpr (DIM == 3) {
+            p[4] = ref(o_.zm + d);
+            p[5] = ref(o_.zp + d);
+        }
+    };
+    // coarse cell (I, J, K) from the residuals of level F's pairs
+    auto restricted = [&](const Lev<T> &F, int I, int J, int K) -> T {
         const int hx = F.nx >> 1;
-        const T *a = sm + M.rs + I + hx * (2 * J + (DIM == 3 ? F.ny * 2 * K : 0));
+        const T *a = arr(M.rs) + I + hx * (2 * J + (DIM == 3 ? F.ny * 2 * K : 0));
         if constexpr (DIM == 3) {
             const int sz = hx * F.ny;
             return T(0.125) * ((a[0] + a[hx]) + (a[sz] + a[sz + hx]));
@@ -860,133 +1061,131 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
             return T(0.25) * (a[0] + a[hx]);
         }
     };
-    auto to_level = [&](int l) {   // right side and zero iterate of level l > 0
+    // right side and zero iterate of level l > 0 (and a barrier)
+    auto to_level = [&](int l) {
         const Lev<T> &F = LV.l[l - 1], &C = LV.l[l];
         if (l == bot) {
             const int n = C.nx * C.ny * C.nz;
             for (int q = t; q < n; q += NT) {
-                const int r = q / C.nx;
-                sm[M.br + q] = restricted(F, q % C.nx, r % C.ny, r / C.ny);
-                sm[M.E[l] + q] = T(0);
+                const Ijk c = ijk_of(q, C.nx, C.ny, M.mx[l], M.my[l]);
+                arr(M.br)[q] = restricted(F, c.i, c.j, c.k);
+                arr(M.E[l])[q] = T(0);
             }
-            __syncthreads();   // the bottom reads other threads' cells
-        } else {
-            const int hx = C.nx >> 1, h = hx * C.ny * C.nz;
-            if (t < h) {   // read again by this thread only, and S after the sweep's barrier
-                const int m = t % hx, r = t / hx, j = r % C.ny, k = r / C.ny;
-                const bool s = (j + k) & 1;
-                const T a = restricted(F, 2 * m, j, k), b = restricted(F, 2 * m + 1, j, k);
-                T *f = sm + M.F[l] + t;
-                f[(2 * DIM + 2) * h] = s ? b : a;
-                f[(2 * DIM + 3 + 2 * DIM + 2) * h] = s ? a : b;
-                sm[M.S[l] + t] = T(0);
-                sm[M.S[l] + h + 1 + t] = T(0);
+        } else if (lm == l) {
+            PairPos pos;
+            if constexpr (PARK) pos = pair_pos<DIM, T>(C, qm, M.S[l], M.mx[l], M.my[l]);
+            else pos = om;
+            const T a = restricted(F, 2 * pos.m, pos.j, pos.k), b = restricted(F, 2 * pos.m + 1, pos.j, pos.k);
+            const T r0 = pos.s ? b : a, r1 = pos.s ? a : b;
+            if constexpr (PARK) {
+                arr(M.park)[(4 * DIM + 4) * M.mid + t] = r0;
+                arr(M.park)[(4 * DIM + 5) * M.mid + t] = r1;
+            } else {
+                Pm.rhs[0] = r0;
+                Pm.rhs[1] = r1;
             }
-            __syncthreads();
+            ref(pos.at) = T(0);
+            ref(pos.at + CM) = T(0);
         }
+        __syncthreads();
     };
-    // the pair of level l that this thread holds, from LDS
-    auto pair_of = [&](int l, int h) -> Pair<DIM, T> {
-        Pair<DIM, T> P;
-        const T *f = sm + M.F[l] + t;
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-#pragma unroll
-            for (int d = 0; d < 2 * DIM; ++d) P.w[c][d] = f[(c * (2 * DIM + 3) + d) * h];
-            P.den[c] = f[(c * (2 * DIM + 3) + 2 * DIM) * h];
-            P.inv[c] = f[(c * (2 * DIM + 3) + 2 * DIM + 1) * h];
-            P.rhs[c] = f[(c * (2 * DIM + 3) + 2 * DIM + 2) * h];
-        }
-        return P;
-    };
-    // level l < bot: down (sweeps, residual, restriction) or up (prolongation, sweeps)
-    auto leg = [&](int l, bool up) {
+    // The pairs P of level l (N a thread, colours CS apart) down: `nu1` sweeps,
+    // the residual, the next level's right side; or up: the prolongation of
+    // level l + 1, nu2 sweeps, the values for the level above
+    auto leg = [&](int l, bool up, auto CSt, auto &P, const auto &pos, auto &&on) {
+        constexpr int N = sizeof(P) / sizeof(P[0]), CS = decltype(CSt)::value;
         const Lev<T> &L = LV.l[l];
-        const int h = (L.nx >> 1) * L.ny * L.nz;
-        T *S = sm + M.S[l];
-        auto go = [&](const auto &P, const auto &pos, const auto &s, const auto &on) {
-            constexpr int N = sizeof(P) / sizeof(P[0]);
-            T v[N][2];
+        T v[N][2];
 #pragma unroll
-            for (int a = 0; a < N; ++a) {
-                v[a][0] = v[a][1] = T(0);
-                if (!on[a]) continue;
-                v[a][0] = S[pos[a].q];
-                v[a][1] = S[h + 1 + pos[a].q];
-                if (up) {
-                    const int hx = L.nx >> 1, m = pos[a].q % hx, r = pos[a].q / hx;
-                    const Lev<T> &C = LV.l[l + 1];
-                    const T *e = sm + M.E[l + 1];
-                    const Two<T> d = prolong_pair<DIM, T>(C.nx, C.ny, C.nz, o.bc, 2 * m, r % L.ny, r / L.ny,
-                                                          [&](int I, int J, int K) { return e[I + C.nx * (J + C.ny * K)]; });
-                    v[a][0] = v[a][0] + (s[a] ? d.b : d.a);
-                    v[a][1] = v[a][1] + (s[a] ? d.a : d.b);
-                    S[pos[a].q] = v[a][0];   // read and written by this thread only until the barrier
-                    S[h + 1 + pos[a].q] = v[a][1];
-                }
+        for (int a = 0; a < N; ++a) {
+            v[a][0] = v[a][1] = T(0);
+            if (!on(a)) continue;
+            v[a][0] = ref(pos[a].at);
+            v[a][1] = ref(pos[a].at + CS);
+            if (up) {
+                const Lev<T> &C = LV.l[l + 1];
+                const T *e = arr(M.E[l + 1]);
+                const Two<T> d = prolong_pair<DIM, T>(C.nx, C.ny, C.nz, o.bc, 2 * pos[a].m, pos[a].j, pos[a].k,
+                                                      [&](int I, int J, int K) { return e[I + C.nx * (J + C.ny * K)]; });
+                v[a][0] = v[a][0] + (pos[a].s ? d.b : d.a);
+                v[a][1] = v[a][1] + (pos[a].s ? d.a : d.b);
+                ref(pos[a].at) = v[a][0];   // read and written by this thread only until the barrier
+                ref(pos[a].at + CS) = v[a][1];
             }
-            if (up) __syncthreads();
-            const bool sor = l == 0 && L.omega != T(1);
-            sweeps(L, P, pos, s, on, v, S, h, up ? o.nu2 : o.nu1, sor);
-            if (!up) {
-                resid(L, P, pos, s, on, v, S, h);
-                return;
-            }
-#pragma unroll
-            for (int a = 0; a < N; ++a)
-                if (on[a]) {
-                    const T lo = s[a] ? v[a][1] : v[a][0], hi = s[a] ? v[a][0] : v[a][1];
-                    if (l == 0) store2(L.phi + 2 * pos[a].q, lo, hi);
-                    else store2(sm + M.E[l] + 2 * pos[a].q, lo, hi);
-                }
-            if (l > 0) __syncthreads();
-        };
-        if (l == 0) {
-            // from global memory on each visit (L2): held in registers through
-            // the deeper levels they would spill
-            Pair<DIM, T> P[NP];
-            PairPos pos[NP];
-            bool s[NP], on[NP];
-#pragma unroll
-            for (int a = 0; a < NP; ++a) {
-                const int q = t + a * NT;
-                P[a] = dead_pair<DIM, T>();
-                pos[a] = PairPos{0, 0, 0, 0, 0, 0, 0};
-                s[a] = false;
-                on[a] = q < h;
-                if (on[a]) {
-                    const int hx = L.nx >> 1, m = q % hx, r = q / hx, j = r % L.ny, k = r / L.ny;
-                    P[a] = load_pair<DIM, T>(L, 2 * m, j, k);
-                    pos[a] = pair_pos<DIM, T>(L, q);
-                    s[a] = (j + k) & 1;
-                }
-            }
-            go(P, pos, s, on);
-        } else {
-            Pair<DIM, T> P[1] = {dead_pair<DIM, T>()};
-            PairPos pos[1] = {PairPos{0, 0, 0, 0, 0, 0, 0}};
-            bool s[1] = {false}, on[1] = {t < h};
-            if (on[0]) {
-                P[0] = pair_of(l, h);
-                pos[0] = pair_pos<DIM, T>(L, t);
-                const int r = t / (L.nx >> 1);
-                s[0] = (r % L.ny + r / L.ny) & 1;
-            }
-            go(P, pos, s, on);
         }
+        if (up) __syncthreads();
+        const bool sor = l == 0 && L.omega != T(1);
+        const int count = up ? o.nu2 : o.nu1;
+        for (int it = 0; it < count; ++it)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+#pragma unroll
+                for (int a = 0; a < N; ++a)
+                    if (on(a)) {
+                        T p[2 * DIM];
+                        nbrs(pos[a], c, CS, v[a][1 - c], p);
+                        v[a][c] = pair_update<DIM, T>(L, P[a], c, p, v[a][c], sor, L.omega);
+                        ref(pos[a].at + c * CS) = v[a][c];
+                    }
+                __syncthreads();
+            }
+#pragma unroll
+        for (int a = 0; a < N; ++a) {
+            if (!on(a)) continue;
+            if (up) {
+                const T lo = pos[a].s ? v[a][1] : v[a][0], hi = pos[a].s ? v[a][0] : v[a][1];
+                if (l == 0) store2(L.phi + 2 * pos[a].q, lo, hi);
+                else store2(arr(M.E[l]) + 2 * pos[a].q, lo, hi);
+                continue;
+            }
+            T res[2];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                T p[2 * DIM];
+                nbrs(pos[a], c, CS, v[a][1 - c], p);
+                T ap = apply_w<DIM, T>(L, P[a].w[c], p, v[a][c]);
+                if (L.alpha) ap = dfma(L.alpha[2 * pos[a].q + (pos[a].s != (c == 1) ? 1 : 0)], v[a][c], ap);
+                res[c] = P[a].rhs[c] - ap;
+            }
+            arr(M.rs)[pos[a].q] = res[0] + res[1];
+        }
+        if (!up || l > 0) __syncthreads();
         if (!up) to_level(l + 1);
+    };
+    auto leg_mid = [&](int l, bool up) {
+        if constexpr (PARK) {
+            Pair<DIM, T> P[1] = {dead_pair<DIM, T>()};
+            const PairPos pos[1] = {pair_pos<DIM, T>(LV.l[l], lm == l ? qm : 0, M.S[l], M.mx[l], M.my[l])};
+            if (lm == l) {
+                const T *f = arr(M.park) + t;
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+#pragma unroll
+                    for (int d = 0; d < 2 * DIM; ++d) P[0].w[c][d] = f[(c * 2 * DIM + d) * M.mid];
+                    P[0].den[c] = f[(4 * DIM + c) * M.mid];
+                    P[0].inv[c] = f[(4 * DIM + 2 + c) * M.mid];
+                    P[0].rhs[c] = f[(4 * DIM + 4 + c) * M.mid];
+                }
+            }
+            leg(l, up, std::integral_constant<int, CM>{}, P, pos, [&](int) { return lm == l; });
+        } else {
+            Pair<DIM, T>(&P)[1] = *reinterpret_cast<Pair<DIM, T>(*)[1]>(&Pm);
+            const PairPos(&pos)[1] = *reinterpret_cast<const PairPos(*)[1]>(&om);
+            leg(l, up, std::integral_constant<int, CM>{}, P, pos, [&](int) { return lm == l; });
+        }
     };
     auto bottom = [&]() {
         const Lev<T> &L = LV.l[bot];
         const int n = L.nx * L.ny * L.nz;
-        T *E = sm + M.E[bot];
+        T *E = arr(M.E[bot]);
+        const T *R = arr(M.br);
         auto cell = [&](int q, T *w, T &a, int &colour) {
-            const T *f = sm + M.bw + q;
+            const T *f = arr(M.bw) + q;
 #pragma unroll
             for (int d = 0; d < 2 * DIM; ++d) w[d] = f[d * n];
             a = f[2 * DIM * n];
-            const int r = q / L.nx;
-            colour = (q % L.nx + r % L.ny + r / L.ny) & 1;
+            const Ijk c = ijk_of(q, L.nx, L.ny, M.mx[bot], M.my[bot]);
+            colour = (c.i + c.j + c.k) & 1;
         };
         T w[2 * DIM], a;
         int colour;
@@ -1001,7 +1200,7 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
                     X.in[2 * d] = hi || per;
                     X.in[2 * d + 1] = !hi || per;
                 }
-                const T v = bottom_solve<DIM, T>(L, X, w, a, colour, E[q], sm[M.br + q], o, n);
+                const T v = bottom_solve<DIM, T>(L, X, w, a, colour, E[q], R[q], o, n);
                 if (t < n) E[t] = v;
             }
         } else if (n <= 64) {
@@ -1012,7 +1211,7 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
                 BottomWave<DIM> X;
                 X.live = live;
                 cell_nbrs<DIM, T>(L, q, -1, X.nb);
-                const T v = bottom_solve<DIM, T>(L, X, w, a, colour, live ? E[q] : T(0), live ? sm[M.br + q] : T(0), o, n);
+                const T v = bottom_solve<DIM, T>(L, X, w, a, colour, live ? E[q] : T(0), live ? R[q] : T(0), o, n);
                 if (live) E[t] = v;
             }
         } else {
@@ -1026,15 +1225,37 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
             X.xs = reinterpret_cast<double *>(smem_ + M.xs);
             X.sh = reinterpret_cast<double *>(smem_ + M.sh);
             cell_nbrs<DIM, T>(L, q, n, X.nb);
-            const T v = bottom_solve<DIM, T>(L, X, w, a, colour, live ? E[q] : T(0), live ? sm[M.br + q] : T(0), o, n);
+            const T v = bottom_solve<DIM, T>(L, X, w, a, colour, live ? E[q] : T(0), live ? R[q] : T(0), o, n);
             if (live) E[t] = v;
         }
         __syncthreads();
     };
+    // Level 0's pairs, from global memory (L2) on the way down and up: held in
+    // registers through the levels below they would spill.  In FP32 they load
+    // together with the rest of the stage; FP64 has no registers for that.
+    {
+        PairRaw<DIM, T> R0[NP];
+        Pair<DIM, T> P0[NP];
+        PairPos o0[NP];
+#pragma unroll
+        for (int a = 0; a < NP; ++a) o0[a] = pair_pos<DIM, T>(L0, t + a * NT, 0, M.mx[0], M.my[0]);
+        auto load0 = [&]() {
+#pragma unroll
+            for (int a = 0; a < NP; ++a) R0[a] = load_raw<DIM, T>(L0, 2 * o0[a].m, o0[a].j, o0[a].k);
+        };
+        if (sizeof(T) == 4 && bot > 0) load0();
+        stage(o0);
+        if (bot > 0) {
+            if (sizeof(T) == 8) load0();
+#pragma unroll
+            for (int a = 0; a < NP; ++a) P0[a] = make_pair<DIM, T>(L0, R0[a], o0[a].s);
+            leg(0, false, std::integral_constant<int, C0>{}, P0, o0, [&](int a) { return o0[a].on; });
+        }
+    }
     if constexpr (VC) {
-        for (int l = 0; l < bot; ++l) leg(l, false);
+        for (int l = 1; l < bot; ++l) leg_mid(l, false);
         bottom();
-        for (int l = bot - 1; l >= 0; --l) leg(l, true);
+        for (int l = bot - 1; l > 0; --l) leg_mid(l, true);
     } else {
         // W and F cycles, without recursion.  Going down, each level owes a
         // second visit of the next coarser level (bit l of `again`; bit l of
@@ -1042,13 +1263,13 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
         // owes one turns back down before its prolongation.  The first visit
         // has the shape of the visiting level.  The masks are the same in
         // every thread, so the block stays in step.
-        unsigned again = 0u, again_w = 0u;
         bool w = o.cycle == MAC_CYCLE_W;   // shape of the current visit (W, or F/V below)
         bool v = false;                     // the current visit is a V
-        int l = 0;
+        unsigned again = 1u, again_w = w ? 1u : 0u;
+        int l = min(1, bot);
         for (;;) {
             for (; l < bot; ++l) {
-                leg(l, false);
+                leg_mid(l, false);
                 if (!v) {
                     again |= 1u << l;
                     if (w) again_w |= 1u << l;
@@ -1057,8 +1278,7 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
             }
             bottom();
             bool down = false;
-            while (l > 0) {
-                --l;
+            for (--l; l >= 0; --l) {
                 if (again & (1u << l)) {   // second visit of level l + 1
                     again &= ~(1u << l);
                     w = (again_w >> l) & 1u;
@@ -1067,14 +1287,25 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
                     down = true;
                     break;
                 }
-                leg(l, true);
+                if (l > 0) leg_mid(l, true);
             }
             if (!down) break;
         }
     }
-    if (bot == 0) {
+    if (bot > 0) {
+        int tp = t;
+        asm volatile("" : "+v"(tp));   // positions and addresses made again, not kept
+        Pair<DIM, T> P0[NP];
+        PairPos o0[NP];
+#pragma unroll
+        for (int a = 0; a < NP; ++a) {
+            o0[a] = pair_pos<DIM, T>(L0, tp + a * NT, 0, M.mx[0], M.my[0]);
+            P0[a] = load_pair<DIM, T>(L0, 2 * o0[a].m, o0[a].j, o0[a].k);
+        }
+        leg(0, true, std::integral_constant<int, C0>{}, P0, o0, [&](int a) { return o0[a].on; });
+    } else {
         const int n = L0.nx * L0.ny * L0.nz;
-        for (int q = t; q < n; q += NT) L0.phi[q] = sm[M.E[0] + q];
+        for (int q = t; q < n; q += NT) L0.phi[q] = arr(M.E[0])[q];
     }
 }
 
@@ -1085,43 +1316,45 @@ static bool coarse_map(int dim, const Lev<T> *levs, int lc, int nlev, CoarseMap 
     M = CoarseMap{};
     M.nl = nlev - lc;
     if (M.nl < 1 || M.nl > COARSE_LEVELS) return false;
-    const int NF = dim == 3 ? pair_fields<3>() : pair_fields<2>();
-    long off = 0;
-    auto take = [&](long cnt) {
+    long off = 0, mid = 0;
+    auto take = [&](long bytes) {
         const long r = off;
-        off += (cnt + 3) / 4 * 4;   // 16-byte steps at least
+        off += (bytes + 15) / 16 * 16;
         return (int)r;
     };
+    const long sz = sizeof(T);
     for (int a = 0; a < M.nl; ++a) {
         const Lev<T> &L = levs[lc + a];
         const long n = (long)L.nx * L.ny * L.nz;
         const bool bottom = a == M.nl - 1;
         if (n > (bottom ? COARSE_BOTTOM : COARSE_CELLS)) return false;
+        M.mx[a] = fast_div_factor(bottom ? L.nx : std::max(1, L.nx / 2));
+        M.my[a] = fast_div_factor(L.ny);
         if (bottom) {
-            M.bw = take((2 * dim + 1) * n);
-            M.br = take(n);
-            M.E[a] = take(n);
+            M.bw = take((2 * dim + 1) * n * sz);
+            M.br = take(n * sz);
+            M.E[a] = take(n * sz);
             continue;
         }
         if ((L.nx & 1) || (L.ny & 1) || (dim == 3 && (L.nz & 1))) return false;
-        if (a > 0 && n / 2 > COARSE_THREADS) return false;
-        M.S[a] = take(2 * (n / 2 + 1));
-        if (a > 0) {
-            M.F[a] = take(NF * (n / 2));
-            M.E[a] = take(n);
-        } else {
-            M.rs = take(n / 2);
+        if (a == 0) {
+            M.S[0] = take(2 * colour0<T>());
+            M.rs = take(n / 2 * sz);
+            continue;
         }
+        mid += n / 2;
+        if (n / 2 >= COARSE_MID || mid > COARSE_THREADS) return false;   // a thread per pair
+        M.S[a] = take(2 * colour_mid<T>());
+        M.E[a] = take(n * sz);
     }
     const Lev<T> &B = levs[nlev - 1];
     const long nb = (long)B.nx * B.ny * B.nz;
-    long bytes = (off * (long)sizeof(T) + 15) / 16 * 16;
-    M.xs = (int)bytes;
-    if (nb > 64) bytes += 2 * (nb + 1) * 8;
-    M.sh = (int)bytes;
-    if (nb > 64) bytes += 64 * 8;
-    M.bytes = (int)bytes;
-    return bytes <= COARSE_LDS;
+    M.xs = take(nb > 64 ? 2 * (nb + 1) * 8 : 0);
+    M.sh = take(nb > 64 ? 64 * 8 : 0);
+    M.mid = (int)mid;
+    M.park = take(dim == 3 ? mid * (long)sizeof(Pair<3, T>) : 0);
+    M.bytes = (int)off;
+    return off <= COARSE_LDS;
 }
 
 template <typename T>
