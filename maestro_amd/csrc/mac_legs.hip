@@ -57,6 +57,25 @@ __device__ __forceinline__ T quot(T n, T d, T r)
     return dfma(dfma(-d, q, n), r, q);
 }
 
+// A copy of x that stays in a register.  A kernel argument used in a loop with
+// barriers is otherwise loaded again in each round, at 100 to 200 cycles in a
+// chain of some 300.
+template <typename T>
+__device__ __forceinline__ T held(T x)
+{
+    asm volatile("" : "+v"(x));
+    return x;
+}
+template <typename T>
+__device__ __forceinline__ Lev<T> held_ih2(const Lev<T> &L)
+{
+    Lev<T> H = L;
+    H.ih2x = held(L.ih2x);
+    H.ih2y = held(L.ih2y);
+    H.ih2z = held(L.ih2z);
+    return H;
+}
+
 // numerator and denominator of gs_value
 template <int DIM, typename T>
 __device__ __forceinline__ T gs_num(const Lev<T> &L, const T *w, const T *p, T rhs)
@@ -585,10 +604,14 @@ __device__ __forceinline__ double wmax(double v)
 //                   fixed order
 // and says which threads hold a cell (live).
 template <int DIM, typename T, typename X>
-__device__ __forceinline__ T bottom_solve(const Lev<T> &L, X &x_, const T *w, T acell, int colour, T phi, T rhs,
+__device__ __forceinline__ T bottom_solve(const Lev<T> &L_, X &x_, const T *w, T acell, int colour, T phi, T rhs,
                                           const CoarseOpts &o, int n)
 {
     const bool live = x_.live;
+    const Lev<T> L = held_ih2(L_);
+    const bool has_alpha = held((int)(L_.alpha != nullptr));
+    const int n_sweeps = held(o.nub), singular = held(o.singular);
+    const double eps = held(o.bottom_eps);
     const T den = gs_den<DIM, T>(L, w, acell), inv = T(1) / den;
     T wn[2 * DIM];   // for the sweeps' sums of neighbours
 #pragma unroll
@@ -605,24 +628,24 @@ __device__ __forceinline__ T bottom_solve(const Lev<T> &L, X &x_, const T *w, T 
         x_.nbrs(v, p);
         if (!live) return 0.0;
         const double ap = apply_w<DIM, double>(D, wd, p, v);
-        return L.alpha ? fma((double)acell, v, ap) : ap;
+        return has_alpha ? fma((double)acell, v, ap) : ap;
     };
 #pragma unroll 1
     for (int part = 0; part < 2; ++part) {
 #pragma unroll 1
-        for (int h = 0; h < 2 * o.nub; ++h) {
+        for (int h = 0; h < 2 * n_sweeps; ++h) {
             T p[2 * DIM];
             x_.nbrs_any(phi, p);
             const T v = quot(gs_num<DIM, T>(L, wn, p, rhs), den, inv);
             if (live && colour == (h & 1)) phi = v;
         }
         if (part == 1 || o.bottom == MAC_BOTTOM_SMOOTH) continue;
-        const double m = o.singular ? mean(x_.sum(live ? (double)rhs : 0.0)) : 0.0;
+        const double m = singular ? mean(x_.sum(live ? (double)rhs : 0.0)) : 0.0;
         double x = live ? (double)phi : 0.0;
         const double ax = apply(x);
         double r = live ? ((double)rhs - m) - ax : 0.0;
         auto project = [&]() {   // the mean off r on singular problems
-            if (o.singular) {
+            if (singular) {
                 const double rm = mean(x_.sum(r));
                 if (live) r -= rm;
             }
@@ -646,7 +669,7 @@ __device__ __forceinline__ T bottom_solve(const Lev<T> &L, X &x_, const T *w, T 
                 al = rho / rv;
                 r -= al * v;
                 project();
-                if (x_.max(fabs(r)) <= o.bottom_eps * r0) {
+                if (x_.max(fabs(r)) <= eps * r0) {
                     x += al * p;
                     break;
                 }
@@ -661,7 +684,7 @@ __device__ __forceinline__ T bottom_solve(const Lev<T> &L, X &x_, const T *w, T 
                 r -= om * t;
                 project();
                 rho_old = rho;
-                if (x_.max(fabs(r)) <= o.bottom_eps * r0 || om == 0.0) break;
+                if (x_.max(fabs(r)) <= eps * r0 || om == 0.0) break;
             }
         } else if (r0 > 0.0) {
             double p = r;
@@ -678,7 +701,7 @@ __device__ __forceinline__ T bottom_solve(const Lev<T> &L, X &x_, const T *w, T 
                 project();
                 double rr1 = r * r, am = fabs(r);
                 x_.sum_max(rr1, am);
-                if (am <= o.bottom_eps * r0) break;
+                if (am <= eps * r0) break;
                 const double beta = quot(rr1, rr, irr);
                 rr = rr1;
                 p = r + beta * p;
@@ -773,28 +796,49 @@ struct BottomWave {
 
 // up to a block of cells: neighbours and sums through LDS, one barrier each
 // (two slots in turn, so a slot is written again only after a barrier that
-// all its readers have passed)
+// all its readers have passed).  Only the waves that hold cells run the solve;
+// the others wait at its barriers (idle), since their instructions would take
+// the busy waves' turns: 6 x 5 x 7 cells FP64, 3100 -> 2150 cycles a CG step.
 template <int DIM>
 struct BottomBlock {
     static constexpr bool POW2 = false;
+    bool live;
+    int nb[2 * DIM];      // neighbour cells; outside: -1, the zeros before an array
+    double *xs, *sh;      // two exchange arrays of 1 + n values; 2 x 32 partial results
+    volatile int *last;   // number of the last barrier, set before it
+    int n, flip, fs, bar; // bar: barriers passed
     __device__ __forceinline__ bool has(int) const { return true; }
+    __device__ __forceinline__ void sync()
+    {
+        ++bar;
+        __syncthreads();
+    }
+    // the barriers of a solve, for a wave without cells; each compares its own
+    // count, so a late look at `last` cannot end it early
+    __device__ __forceinline__ void idle() const
+    {
+        for (int k = 1;; ++k) {
+            __syncthreads();
+            if (*last == k) break;
+        }
+    }
+    __device__ __forceinline__ void finish()
+    {
+        if (threadIdx.x == 0) *last = bar + 1;
+        sync();
+    }
     template <typename V>
     __device__ __forceinline__ void nbrs_any(V v, V *p)
     {
         nbrs(v, p);
     }
-    bool live;
-    int nb[2 * DIM];      // neighbour cells; outside: the zero cell n
-    double *xs, *sh;      // two exchange arrays of n + 1 values; 2 x 32 partial results
-    int n, flip, fs;
     template <typename V>
     __device__ __forceinline__ void nbrs(V v, V *p)
     {
-        V *a = reinterpret_cast<V *>(xs + flip * (n + 1));
+        V *a = reinterpret_cast<V *>(xs + (flip ? n + 2 : 1));
         flip ^= 1;
         if (live) a[threadIdx.x] = v;
-        if ((int)threadIdx.x == n || (n == (int)blockDim.x && threadIdx.x == 0)) a[n] = V(0);
-        __syncthreads();
+        sync();
         if (live) {
 #pragma unroll
             for (int s = 0; s < 2 * DIM; ++s) p[s] = a[nb[s]];
@@ -803,45 +847,74 @@ struct BottomBlock {
             for (int s = 0; s < 2 * DIM; ++s) p[s] = V(0);
         }
     }
-    __device__ __forceinline__ double *post(double v)
+    // over the waves' partial results in order, four reads at a time (those
+    // of idle waves are zero)
+    template <typename F>
+    __device__ __forceinline__ double over(const double *a, F &&f) const
+    {
+        double s = 0.0;
+#pragma unroll 1
+        for (int w = 0; w < n; w += 256, a += 4) {
+            const double a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];
+            s = f(f(f(f(s, a0), a1), a2), a3);
+        }
+        return s;
+    }
+    __device__ __forceinline__ double *slot()
     {
         double *a = sh + 32 * fs;
         fs ^= 1;
-        if ((threadIdx.x & 63) == 0) a[threadIdx.x >> 6] = v;
-        __syncthreads();
         return a;
     }
     __device__ __forceinline__ double sum(double v)
     {
-        const double *a = post(wsum(v));
-        double s = 0.0;
-#pragma unroll 1
-        for (int w = 0; w < (n + 63) >> 6; ++w) s += a[w];
-        return s;
+        double *a = slot();
+        v = wsum(v);
+        if ((threadIdx.x & 63) == 0) a[threadIdx.x >> 6] = v;
+        sync();
+        return over(a, [](double x, double y) { return x + y; });
     }
     __device__ __forceinline__ double max(double v)
     {
-        const double *a = post(wmax(v));
-        double s = 0.0;
-#pragma unroll 1
-        for (int w = 0; w < (n + 63) >> 6; ++w) s = fmax(s, a[w]);
-        return s;
+        double *a = slot();
+        v = wmax(v);
+        if ((threadIdx.x & 63) == 0) a[threadIdx.x >> 6] = v;
+        sync();
+        return over(a, [](double x, double y) { return fmax(x, y); });
     }
     __device__ __forceinline__ void sum_max(double &s, double &m)   // one barrier for both
     {
+        double *a = slot();
         s = wsum(s);
         m = wmax(m);
-        double *a = sh + 32 * fs;
-        if ((threadIdx.x & 63) == 0) a[16 + (threadIdx.x >> 6)] = m;
-        post(s);
-        s = m = 0.0;
-#pragma unroll 1
-        for (int w = 0; w < (n + 63) >> 6; ++w) {
-            s += a[w];
-            m = fmax(m, a[16 + w]);
+        if ((threadIdx.x & 63) == 0) {
+            a[threadIdx.x >> 6] = s;
+            a[16 + (threadIdx.x >> 6)] = m;
         }
+        sync();
+        s = over(a, [](double x, double y) { return x + y; });
+        m = over(a + 16, [](double x, double y) { return fmax(x, y); });
     }
 };
+
+// q / d for q d < 2^32: the high word of q times m = floor(2^32 / d) + 1 (0: d = 1)
+__device__ __forceinline__ int fast_div(int q, unsigned m)
+{
+    return m ? (int)__umulhi((unsigned)q, m) : q;
+}
+static unsigned fast_div_factor(int d)
+{
+    return d == 1 ? 0u : (unsigned)(4294967296.0 / d) + 1u;
+}
+// position q of a row-major array of rows of nx in planes of ny rows
+struct Ijk {
+    int i, j, k;
+};
+__device__ __forceinline__ Ijk ijk_of(int q, int nx, int ny, unsigned mx, unsigned my)
+{
+    const int r = fast_div(q, mx), k = fast_div(r, my);
+    return Ijk{q - r * nx, r - k * ny, k};
+}
 
 // the neighbours of cell q of level L, `none` outside a non-periodic side
 template <int DIM, typename T>
@@ -882,25 +955,6 @@ struct CoarseMap {
 static constexpr int COARSE_MID = COARSE_CELLS / 8 + 1;   // of one level, and the zero cell
 template <typename T> static constexpr int colour0() { return (COARSE_CELLS / 2 + 2) * (int)sizeof(T); }
 template <typename T> static constexpr int colour_mid() { return (COARSE_MID + 1) * (int)sizeof(T); }
-
-// q / d for q d < 2^32: the high word of q times m = floor(2^32 / d) + 1 (0: d = 1)
-__device__ __forceinline__ int fast_div(int q, unsigned m)
-{
-    return m ? (int)__umulhi((unsigned)q, m) : q;
-}
-static unsigned fast_div_factor(int d)
-{
-    return d == 1 ? 0u : (unsigned)(4294967296.0 / d) + 1u;
-}
-// position q of a row-major array of rows of nx in planes of ny rows
-struct Ijk {
-    int i, j, k;
-};
-__device__ __forceinline__ Ijk ijk_of(int q, int nx, int ny, unsigned mx, unsigned my)
-{
-    const int r = fast_div(q, mx), k = fast_div(r, my);
-    return Ijk{q - r * nx, r - k * ny, k};
-}
 
 template <typename T>
 struct CoarseLevs {
@@ -1094,7 +1148,7 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
     // level l + 1, nu2 sweeps, the values for the level above
     auto leg = [&](int l, bool up, auto CSt, auto &P, const auto &pos, auto &&on) {
         constexpr int N = sizeof(P) / sizeof(P[0]), CS = decltype(CSt)::value;
-        const Lev<T> &L = LV.l[l];
+        const Lev<T> L = held_ih2(LV.l[l]);
         T v[N][2];
 #pragma unroll
         for (int a = 0; a < N; ++a) {
@@ -1114,7 +1168,8 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
             }
         }
         if (up) __syncthreads();
-        const bool sor = l == 0 && L.omega != T(1);
+        const T omega = l == 0 ? L.omega : T(1);
+        const bool sor = omega != T(1);
         const int count = up ? o.nu2 : o.nu1;
         for (int it = 0; it < count; ++it)
 #pragma unroll
@@ -1124,7 +1179,7 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
                     if (on(a)) {
                         T p[2 * DIM];
                         nbrs(pos[a], c, CS, v[a][1 - c], p);
-                        v[a][c] = pair_update<DIM, T>(L, P[a], c, p, v[a][c], sor, L.omega);
+                        v[a][c] = pair_update<DIM, T>(L, P[a], c, p, v[a][c], sor, omega);
                         ref(pos[a].at + c * CS) = v[a][c];
                     }
                 __syncthreads();
@@ -1220,13 +1275,23 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
             cell(q, w, a, colour);
             BottomBlock<DIM> X;
             X.live = live;
-            X.n = n;
-            X.flip = X.fs = 0;
+            X.n = held(n);
+            X.flip = X.fs = X.bar = 0;
             X.xs = reinterpret_cast<double *>(smem_ + M.xs);
             X.sh = reinterpret_cast<double *>(smem_ + M.sh);
-            cell_nbrs<DIM, T>(L, q, n, X.nb);
-            const T v = bottom_solve<DIM, T>(L, X, w, a, colour, live ? E[q] : T(0), live ? R[q] : T(0), o, n);
-            if (live) E[t] = v;
+            X.last = reinterpret_cast<int *>(X.sh + 64);
+            if (t == 0) X.xs[0] = X.xs[n + 1] = 0.0;
+            if (t == 0) *X.last = 0;
+            if (t < 64) X.sh[t] = 0.0;
+            if ((t & ~63) < n) {
+                cell_nbrs<DIM, T>(L, q, -1, X.nb);
+                X.sync();   // the zeros above
+                const T v = bottom_solve<DIM, T>(L, X, w, a, colour, live ? E[q] : T(0), live ? R[q] : T(0), o, n);
+                if (live) E[t] = v;
+                X.finish();
+            } else {
+                X.idle();
+            }
         }
         __syncthreads();
     };
@@ -1350,7 +1415,7 @@ static bool coarse_map(int dim, const Lev<T> *levs, int lc, int nlev, CoarseMap 
     const Lev<T> &B = levs[nlev - 1];
     const long nb = (long)B.nx * B.ny * B.nz;
     M.xs = take(nb > 64 ? 2 * (nb + 1) * 8 : 0);
-    M.sh = take(nb > 64 ? 64 * 8 : 0);
+    M.sh = take(nb > 64 ? 65 * 8 : 0);
     M.mid = (int)mid;
     M.park = take(dim == 3 ? mid * (long)sizeof(Pair<3, T>) : 0);
     M.bytes = (int)off;
