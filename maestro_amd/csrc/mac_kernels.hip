@@ -789,83 +789,6 @@ struct RowSweepGrid {
     int per_xcd;   // ceil(total / 8)
 };
 
-// Load/store at a wave-uniform base plus a per-lane 32-bit byte offset,
-// through a raw buffer resource built from the base (the resource sits in
-// SGPRs and the offset is one VGPR; a plain pointer form lets the compiler
-// hoist a 64-bit per-lane address per array out of the march, which costs
-// two VGPRs per array).  The range is not limited (num_records = 2^32-1);
-// every offset used stays inside its array.
-static constexpr int BUF_CFG = 0x00020000;   // gfx9-family raw buffer dword 3
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *base)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)0xffffffff, BUF_CFG);
-}
-template <typename V>
-__device__ __forceinline__ V ld_off(const void *base, unsigned boff)
-{
-    const __amdgpu_buffer_rsrc_t r = buf_rsrc(base);
-    static_assert(sizeof(V) == 4 || sizeof(V) == 8 || sizeof(V) == 16, "buffer load width");
-    if constexpr (sizeof(V) == 4)
-        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, boff, 0, 0));
-    else if constexpr (sizeof(V) == 8)
-        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, boff, 0, 0));
-    else
-        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, boff, 0, 0));
-}
-template <typename V>
-__device__ __forceinline__ void st_off(void *base, unsigned boff, const V &v)
-{
-    const __amdgpu_buffer_rsrc_t r = buf_rsrc(base);
-    static_assert(sizeof(V) == 4 || sizeof(V) == 8 || sizeof(V) == 16, "buffer store width");
-    if constexpr (sizeof(V) == 4)
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, boff, 0, 0);
-    else if constexpr (sizeof(V) == 8)
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, v),
-                                              r, boff, 0, 0);
-    else
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, v),
-                                               r, boff, 0, 0);
-}
-
-__device__ __forceinline__ unsigned short ld_u16(const void *base, unsigned boff)
-{
-    return __builtin_amdgcn_raw_buffer_load_b16(buf_rsrc(base), boff, 0, 0);
-}
-
-template <typename V>
-__device__ __forceinline__ V ld_rs(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff)
-{
-    static_assert(sizeof(V) == 2 || sizeof(V) == 4 || sizeof(V) == 8 || sizeof(V) == 16, "buffer load width");
-    if constexpr (sizeof(V) == 2)
-        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b16(r, voff, soff, 0));
-    else if constexpr (sizeof(V) == 4)
-        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
-    else if constexpr (sizeof(V) == 8)
-        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
-    else
-        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
-}
-// Cache policy of a buffer access: 0 default; CPOL_NT the non-temporal
-// (streaming) hint.  The sweeps write their output with it: the new iterate
-// is written once and read by the next launch, and the streaming stores
-// measured 2-3% faster per sweep at 256^3 (FP32 111 -> 108.6 us, FP64 173 ->
-// 167.8 us).  Their loads keep the default: the y-ring rows a neighbouring
-// tile re-reads come from L2 only if the first read allocated them there.
-static constexpr int CPOL_NT = 2;
-
-template <typename V, int CPOL = 0>
-__device__ __forceinline__ void st_rs(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff, const V &v)
-{
-    static_assert(sizeof(V) == 8 || sizeof(V) == 16, "buffer store width");
-    if constexpr (sizeof(V) == 8)
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, v),
-                                              r, voff, soff, CPOL);
-    else
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, v),
-                                               r, voff, soff, CPOL);
-}
-
 // Full-row sweep, nx = 128 W (W a template parameter, so every LDS offset is
 // an immediate).  A wave covers 128 columns of one row, two per lane (one red
 // and one black cell on every plane).  Each array's buffer resource is built

@@ -67,10 +67,12 @@ struct CoarseOpts {
     EllBC bc;
 };
 
+// two red-black sweeps of a 3D level in one pass, pin -> pout (mode SWEEP_*,
+// mac_sweep2.hip); false (nothing launched) where it does not apply
+template <typename T> bool launch_sweep2(const Lev<T> &L, const T *pin, T *pout, int mode, hipStream_t s);
 // ---- the small levels (mac_legs.hip)
 // levels whose way down or up runs as one launch: measured limits
 static constexpr long LEG_MAX_3D = 1L << 18, LEG_MAX_2D = 1L << 22;
-static constexpr long LEG_SMALL_3D = 1L << 16;
 // the single-workgroup coarse cycle: cells of its first level, cells of the
 // bottom, levels, threads, LDS bytes
 static constexpr int COARSE_CELLS = 4096, COARSE_BOTTOM = 1024, COARSE_LEVELS = 8, COARSE_THREADS = 1024;

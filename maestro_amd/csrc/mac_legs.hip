@@ -44,19 +44,6 @@ __device__ __forceinline__ void store2(T *p, T a, T b)
     *reinterpret_cast<Two<T> *>(p) = Two<T>{a, b};
 }
 
-// n / d from r = 1 / d (both correctly rounded): a product and two correction
-// steps, after which the quotient is the correctly rounded one (P. Markstein,
-// IBM J. Res. Dev. 34 (1990) 111-119) away from under- and overflow, the value
-// that the division of gs_value gives.  A cell is updated four times with one
-// diagonal; five operations replace the division's eleven in FP64.
-template <typename T>
-__device__ __forceinline__ T quot(T n, T d, T r)
-{
-    T q = n * r;
-    q = dfma(dfma(-d, q, n), r, q);
-    return dfma(dfma(-d, q, n), r, q);
-}
-
 // A copy of x that stays in a register.  A kernel argument used in a loop with
 // barriers is otherwise loaded again in each round, at 100 to 200 cycles in a
 // chain of some 300.

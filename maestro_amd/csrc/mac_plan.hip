@@ -403,7 +403,10 @@ static void fused_sweeps(mac_plan *P, Hier<T> &H, int l, int nsweep, int first_m
                                            : (f64 ? MAC_PROF_GSRB64 : MAC_PROF_GSRB32);
         int q = (l == 0) ? prof_begin(P, cls) : -1;
         bool ok;
-        if constexpr (sizeof(T) == 4)
+        if (it + 1 < nsweep && !K && !Rh && launch_sweep2<T>(L, pin, pout, mode, P->stream)) {
+            ++it;
+            ok = true;
+        } else if constexpr (sizeof(T) == 4)
             ok = Rh ? launch_gsrb_rho(L, *Rh, pin, pout, mode, P->stream)
                     : launch_gsrb_fused<T>(L, pin, pout, mode, P->stream, K);
         else
@@ -1786,16 +1789,10 @@ extern "C" int mac_debug_op(mac_plan *P, int level, int op, int count)
         if (level == 0 && (rc = compact_level0(P, &K, false))) return rc;
         if (K) launch_to_bf16(F.rhs, K->rhs, n, s);
         int cur = 0;
-        for (int c = 0; c < count; ++c) {
-            if (use_fused(P)) {
-                if (!launch_gsrb_fused<float>(F, cur ? F.phi2 : F.phi, cur ? F.phi : F.phi2, SWEEP_PLAIN, s, K))
-                    return MAC_ERR_INVALID;
-                cur ^= 1;
-            } else {
-                launch_gsrb<float>(P->dim, F, 0, s);
-                launch_gsrb<float>(P->dim, F, 1, s);
-            }
-        }
+        P->launch_failed = false;
+        if (use_fused(P)) fused_sweeps<float>(P, P->H32, level, count, SWEEP_PLAIN, cur, K);
+        else smooth<float>(P, F, level, count);
+        if (P->launch_failed) return MAC_ERR_INVALID;
         launch_convert<float, double>(cur ? F.phi2 : F.phi, L.phi, n, s);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(s));
@@ -1820,26 +1817,17 @@ extern "C" int mac_debug_op(mac_plan *P, int level, int op, int count)
         HIPCHK(hipStreamSynchronize(s));
         return MAC_OK;
     }
-    if (op == MAC_OP_GSRB && use_fused(P)) {   // sweeps alternate phi <-> phi2
-        for (int c = 0; c < count; ++c)
-            launch_gsrb_fused<double>(L, (c & 1) ? L.phi2 : L.phi, (c & 1) ? L.phi : L.phi2, SWEEP_PLAIN, s);
-        if (count & 1)
+    if (op == MAC_OP_GSRB && use_fused(P)) {   // in pairs where one launch takes two sweeps
+        int cur = 0;
+        fused_sweeps<double>(P, H, level, count, SWEEP_PLAIN, cur);
+        if (cur)
             HIPCHK(hipMemcpyAsync(L.phi, L.phi2, sizeof(double) * (size_t)L.nx * L.ny * L.nz,
                                   hipMemcpyDeviceToDevice, s));
         count = 0;
     }
     for (int c = 0; c < count; ++c) {
         switch (op) {
-        case MAC_OP_GSRB:
-            if (use_fused(P)) {
-                launch_gsrb_fused<double>(L, L.phi, L.phi2, SWEEP_PLAIN, s);
-                HIPCHK(hipMemcpyAsync(L.phi, L.phi2, sizeof(double) * (size_t)L.nx * L.ny * L.nz,
-                                      hipMemcpyDeviceToDevice, s));
-            } else {
-                launch_gsrb<double>(P->dim, L, 0, s);
-                launch_gsrb<double>(P->dim, L, 1, s);
-            }
-            break;
+        case MAC_OP_GSRB: smooth<double>(P, L, level, 1); break;   // 2D
         case MAC_OP_RESIDUAL: launch_residual<double>(P->dim, L, L.res, nullptr, s); break;
         case MAC_OP_RESTRICT:
             if (!has_next) return MAC_ERR_INVALID;
