@@ -56,91 +56,218 @@ void launch_cell_to_edge(const double *c, int nr, double *e, hipStream_t s)
 // put_1d_array_on_cart_3d_sphr for a bin-centred, scalar profile: type 1
 // piecewise constant, 2 piecewise linear, 3 quadratic (quad_interp,
 // fill_3d_data.f90:535-546, limited to the range of its three points)
-__device__ double sphr_cell_value(const double *__restrict__ s0, const SphrGeom &G, int i, int j, int k)
+// What the interpolation takes from the cell's place (at), shared by the
+// profiles interpolated there, and a profile's value (of).  Divisors are few (dr
+// and differences of radii near it), so quotients are formed from their
+// reciprocals (quot), five or six operations for a division's eleven or more.
+struct SphrAt {
+    int i0, i1, i2;
+    bool one;           // s0[i0] itself
+    double w0, w1;      // interp 2: weights of i0, i1; 3: radius - x0, radius - x1
+    double d0, d1, d2;  // x1 - x0, x2 - x1, x2 - x0
+    double r0, r1, r2;  // their reciprocals
+};
+
+// whether quot(n, d, r) is n / d: its correction steps round correctly while
+// nothing under- or overflows, d being a radial spacing within 1e-40 .. 1e40
+// (spacing_recip gives 0 for one outside)
+__device__ __forceinline__ bool quot_range(double n)
 {
-    const double x = G.prob_lo[0] + ((double)i + 0.5) * G.dx[0] - G.center[0];
-    const double y = G.prob_lo[1] + ((double)j + 0.5) * G.dx[1] - G.center[1];
-    const double z = G.prob_lo[2] + ((double)k + 0.5) * G.dx[2] - G.center[2];
+    const double m = fabs(n);
+    return (m > 1e-200 && m < 1e200) || n == 0.0;
+}
+__device__ __forceinline__ double spacing_recip(double d)
+{
+    return d > 1e-40 && d < 1e40 ? 1.0 / d : 0.0;
+}
+
+__device__ __forceinline__ SphrAt sphr_at(const SphrGeom &G, double x, double y, double z, double rdr)
+{
+    SphrAt A;
     const double radius = sqrt(x * x + y * y + z * z);
     const double dr = G.dr;
     const int nr = G.nr;
-    int index = (int)(radius / dr);
-    if (G.interp == 1) return s0[index];
+    int index = (int)(rdr != 0.0 && quot_range(radius) ? quot(radius, dr, rdr) : radius / dr);
+    A.one = true;
+    A.i0 = A.i1 = A.i2 = index;
+    if (G.interp == 1) return A;
     if (G.interp == 2) {
         const double rc = ((double)index + 0.5) * dr;
         if (radius >= rc) {
-            if (index >= nr - 1) return s0[nr - 1];
+            if (index >= nr - 1) {
+                A.i0 = nr - 1;
+                return A;
+            }
             const double rc1 = ((double)(index + 1) + 0.5) * dr;
-            return s0[index + 1] * (radius - rc) / dr + s0[index] * (rc1 - radius) / dr;
+            A.i0 = index + 1;
+            A.w0 = radius - rc;
+            A.i1 = index;
+            A.w1 = rc1 - radius;
+        } else {
+            if (index == 0) return A;
+            if (index > nr - 1) {
+                A.i0 = nr - 1;
+                return A;
+            }
+            const double rcm = ((double)(index - 1) + 0.5) * dr;
+            A.i0 = index;
+            A.w0 = radius - rcm;
+            A.i1 = index - 1;
+            A.w1 = rc - radius;
         }
-        if (index == 0) return s0[index];
-        if (index > nr - 1) return s0[nr - 1];
-        const double rcm = ((double)(index - 1) + 0.5) * dr;
-        return s0[index] * (radius - rcm) / dr + s0[index - 1] * (rc - radius) / dr;
+        A.one = false;
+        A.d0 = dr;
+        A.r0 = rdr;
+        return A;
     }
     if (index == 0) index = 1;
     else if (index >= nr - 1) index = nr - 2;
     const double x0 = ((double)(index - 1) + 0.5) * dr, x1 = ((double)index + 0.5) * dr,
                  x2 = ((double)(index + 1) + 0.5) * dr;
-    const double y0 = s0[index - 1], y1 = s0[index], y2 = s0[index + 1];
-    double v = y0 + (y1 - y0) / (x1 - x0) * (radius - x0) +
-               ((y2 - y1) / (x2 - x1) - (y1 - y0) / (x1 - x0)) / (x2 - x0) * (radius - x0) * (radius - x1);
-    const double mx = fmax(fmax(y0, y1), y2), mn = fmin(fmin(y0, y1), y2);
-    if (v > mx) v = mx;
-    if (v < mn) v = mn;
+    A.i0 = index - 1;
+    A.i1 = index;
+    A.i2 = index + 1;
+    A.one = false;
+    A.w0 = radius - x0;
+    A.w1 = radius - x1;
+    A.d0 = x1 - x0;
+    A.d1 = x2 - x1;
+    A.d2 = x2 - x0;
+    A.r0 = spacing_recip(A.d0);
+    A.r1 = spacing_recip(A.d1);
+    A.r2 = spacing_recip(A.d2);
+    return A;
+}
+
+// DIV: by division, what the other form takes where a quotient's operands are
+// out of quot's range (one test per profile: no branch between its quotients)
+template <bool DIV = false>
+__device__ __forceinline__ double sphr_of(const SphrGeom &G, const SphrAt &A, const double *__restrict__ s0)
+{
+    const double y0 = s0[A.i0];
+    if (A.one) return y0;
+    bool ok = true;
+    auto ratio = [&](double n, double d, double r) {
+        if constexpr (DIV) return n / d;
+        ok = ok && r != 0.0 && quot_range(n);
+        return quot(n, d, r);
+    };
+    const double y1 = s0[A.i1];
+    double v;
+    if (G.interp == 2) {
+        v = ratio(y0 * A.w0, A.d0, A.r0) + ratio(y1 * A.w1, A.d0, A.r0);
+    } else {
+        const double y2 = s0[A.i2];
+        const double q = ratio(y1 - y0, A.d0, A.r0);
+        v = y0 + q * A.w0 + ratio(ratio(y2 - y1, A.d1, A.r1) - q, A.d2, A.r2) * A.w0 * A.w1;
+        const double mx = fmax(fmax(y0, y1), y2), mn = fmin(fmin(y0, y1), y2);
+        if (v > mx) v = mx;
+        if (v < mn) v = mn;
+    }
+    if constexpr (!DIV) {
+        if (!ok) v = sphr_of<true>(G, A, s0);
+    }
     return v;
+}
+__device__ __forceinline__ double sphr_x(const SphrGeom &G, int d, int i)
+{
+    return G.prob_lo[d] + ((double)i + 0.5) * G.dx[d] - G.center[d];
 }
 
 // ----------------------------------------------------------- make_macrhs
-// one thread per valid cell of box blockIdx.y
-template <int DIM, bool SPH>
-__global__ void __launch_bounds__(ITPB) k_make_macrhs(MacrhsArgs A)
+// One thread per column (i, j) of box blockIdx.y's valid cells, blockIdx.z's
+// planes of it.  TAB: the radial profiles are copied to LDS first.  A row of
+// cells reaches over as many cache lines of a profile as it has bins across,
+// and a cell takes 15 such gathers (five quadratic profiles).  Bound by the
+// interpolations' FP64 instructions and their latency: 256^3 cells, six arrays
+// of 0.13 GB, take 255 us; with the profiles in memory, a branch per quotient
+// and the streams' loads after the interpolation 326, with a division per
+// quotient and 64-bit index divisions per cell 336.  Blocks of 512 threads
+// (three to a CU with 44 KB of profiles) 255, of 1024 (one) 269.
+static constexpr int MACRHS_PLANES = 16;
+template <int DIM, bool SPH, bool TAB>
+__global__ void __launch_bounds__(TAB ? 512 : ITPB) k_make_macrhs(MacrhsArgs A)
 {
+    constexpr int NT = TAB ? 512 : ITPB;
     const int b = blockIdx.y;
     const BoxDev B = A.boxes[b];
     const int ex = B.hi[0] - B.lo[0] + 1, ey = B.hi[1] - B.lo[1] + 1;
     const int ez = (DIM == 3) ? B.hi[2] - B.lo[2] + 1 : 1;
-    const long q = (long)blockIdx.x * ITPB + threadIdx.x;
-    if (q >= (long)ex * ey * ez) return;
-    const int i = B.lo[0] + (int)(q % ex), j = B.lo[1] + (int)((q / ex) % ey);
-    const int k = (DIM == 3) ? B.lo[2] + (int)(q / ((long)ex * ey)) : 0;
-    const int I = i - A.dlo[0], J = j - A.dlo[1], K = (DIM == 3) ? k - A.dlo[2] : 0;
-    double b0, sb, g1 = 0.0, pp = 0.0;
-    bool below;
+    const int k0 = blockIdx.z * MACRHS_PLANES, k1 = min(k0 + MACRHS_PLANES, ez);
+    const int p = blockIdx.x * NT + threadIdx.x;
+    if (k0 >= ez) return;
+    extern __shared__ double tab[];
+    const int nr = A.geo.nr;
+    if constexpr (TAB) {
+        const int np = A.dpdt_on ? 5 : 2;
+        for (int q = threadIdx.x; q < nr; q += NT) {
+            tab[q] = A.beta0[q];
+            tab[nr + q] = A.Sbar[q];
+            if (np == 5) {
+                tab[2 * nr + q] = A.gamma1bar[q];
+                tab[3 * nr + q] = A.p0[q];
+                tab[4 * nr + q] = A.rho0[q];
+            }
+        }
+        __syncthreads();
+    }
+    if (p >= ex * ey) return;
+    const int lj = p / ex, li = p - lj * ex;
+    const int i = B.lo[0] + li, j = B.lo[1] + lj;
+    const int J = j - A.dlo[1];
+    double x = 0.0, y = 0.0, rdr = 0.0;
     if constexpr (SPH) {
-        b0 = sphr_cell_value(A.beta0, A.geo, I, J, K);
-        sb = sphr_cell_value(A.Sbar, A.geo, I, J, K);
-        double r0 = 0.0;
-        if (A.dpdt_on) {
-            g1 = sphr_cell_value(A.gamma1bar, A.geo, I, J, K);
-            pp = sphr_cell_value(A.p0, A.geo, I, J, K);
-            r0 = sphr_cell_value(A.rho0, A.geo, I, J, K);
-        }
-        below = r0 > A.cutoff_density;
-    } else {
-        const int r = (DIM == 3) ? K : J;
-        b0 = A.beta0[r];
-        sb = A.Sbar[r];
-        if (A.dpdt_on) {
-            g1 = A.gamma1bar[r];
-            pp = A.p0[r];
-        }
-        below = r < A.cutoff_coord;
+        x = sphr_x(A.geo, 0, i - A.dlo[0]);
+        y = sphr_x(A.geo, 1, J);
+        rdr = spacing_recip(A.geo.dr);
     }
-    const double S = A.S[b][box_index(B, A.ng_S, -1, DIM, i, j, k)];
-    const double dg = A.dg[b][box_index(B, A.ng_dg, -1, DIM, i, j, k)];
-    double v = b0 * (S - sb + dg);
-    if (A.dpdt_on) {
-        double *dchi = A.dchi[b] + box_index(B, A.ng_dchi, -1, DIM, i, j, k);
-        double x = A.predictor ? 0.0 : *dchi;
-        if (below) {
-            const double dp = A.dp[b][box_index(B, A.ng_dp, -1, DIM, i, j, k)];
-            x = x + A.dpdt * dp / (A.dt * g1 * pp);
-            v = v + b0 * x;
+    const double *__restrict__ pS = A.S[b], *__restrict__ pdg = A.dg[b];
+    const double *__restrict__ pdp = A.dpdt_on ? A.dp[b] : nullptr;
+    double *__restrict__ pchi = A.dpdt_on ? A.dchi[b] : nullptr, *__restrict__ prhs = A.rhs[b];
+    for (int l = k0; l < k1; ++l) {
+        const int k = (DIM == 3) ? B.lo[2] + l : 0, K = (DIM == 3) ? k - A.dlo[2] : 0;
+        // the streams' loads before the interpolation
+        const double S = pS[box_index(B, A.ng_S, -1, DIM, i, j, k)];
+        const double dg = pdg[box_index(B, A.ng_dg, -1, DIM, i, j, k)];
+        double *dchi = nullptr, c = 0.0;
+        if (A.dpdt_on) {
+            dchi = pchi + box_index(B, A.ng_dchi, -1, DIM, i, j, k);
+            if (!A.predictor) c = *dchi;
         }
-        *dchi = x;
+        double b0, sb, g1 = 0.0, pp = 0.0;
+        bool below;
+        if constexpr (SPH) {
+            const SphrAt at = sphr_at(A.geo, x, y, sphr_x(A.geo, 2, K), rdr);
+            b0 = sphr_of(A.geo, at, TAB ? tab : A.beta0);
+            sb = sphr_of(A.geo, at, TAB ? tab + 1 * nr : A.Sbar);
+            double r0 = 0.0;
+            if (A.dpdt_on) {
+                g1 = sphr_of(A.geo, at, TAB ? tab + 2 * nr : A.gamma1bar);
+                pp = sphr_of(A.geo, at, TAB ? tab + 3 * nr : A.p0);
+                r0 = sphr_of(A.geo, at, TAB ? tab + 4 * nr : A.rho0);
+            }
+            below = r0 > A.cutoff_density;
+        } else {
+            const int r = (DIM == 3) ? K : J;
+            b0 = A.beta0[r];
+            sb = A.Sbar[r];
+            if (A.dpdt_on) {
+                g1 = A.gamma1bar[r];
+                pp = A.p0[r];
+            }
+            below = r < A.cutoff_coord;
+        }
+        double v = b0 * (S - sb + dg);
+        if (A.dpdt_on) {
+            if (below) {
+                const double dp = pdp[box_index(B, A.ng_dp, -1, DIM, i, j, k)];
+                c = c + A.dpdt * dp / (A.dt * g1 * pp);
+                v = v + b0 * c;
+            }
+            *dchi = c;
+        }
+        prhs[box_index(B, A.ng_rhs, -1, DIM, i, j, k)] = v;
     }
-    A.rhs[b][box_index(B, A.ng_rhs, -1, DIM, i, j, k)] = v;
 }
 
 // the reference zeroes a predictor's delta_chi over the whole array, ghost
@@ -160,64 +287,108 @@ __global__ void __launch_bounds__(ITPB) k_zero_ghosts(MacrhsArgs A, int dim)
     }
 }
 
-void launch_make_macrhs(const MacrhsArgs &A, int maxcells, bool sph, hipStream_t s)
+void launch_make_macrhs(const MacrhsArgs &A, const int maxext[3], bool sph, hipStream_t s)
 {
-    dim3 g((unsigned)((maxcells + ITPB - 1) / ITPB), A.nboxes, 1);
-    if (A.dim == 3) {
-        if (sph) hipLaunchKernelGGL((k_make_macrhs<3, true>), g, dim3(ITPB), 0, s, A);
-        else hipLaunchKernelGGL((k_make_macrhs<3, false>), g, dim3(ITPB), 0, s, A);
+    auto go = [&](auto k, int nt, size_t lds) {
+        const dim3 g((unsigned)(((long)maxext[0] * maxext[1] + nt - 1) / nt), A.nboxes,
+                     (unsigned)((maxext[2] + MACRHS_PLANES - 1) / MACRHS_PLANES));
+        hipLaunchKernelGGL(k, g, dim3(nt), lds, s, A);
+    };
+    if (A.dim == 3 && sph) {
+        // two blocks or more to a CU
+        const size_t lds = sizeof(double) * (size_t)A.geo.nr * (A.dpdt_on ? 5 : 2);
+        if (lds <= 64 * 1024) go(k_make_macrhs<3, true, true>, 512, lds);
+        else go(k_make_macrhs<3, true, false>, ITPB, 0);
+    } else if (A.dim == 3) {
+        go(k_make_macrhs<3, false, false>, ITPB, 0);
     } else {
-        hipLaunchKernelGGL((k_make_macrhs<2, false>), g, dim3(ITPB), 0, s, A);
+        go(k_make_macrhs<2, false, false>, ITPB, 0);
     }
     if (A.dpdt_on && A.predictor && A.ng_dchi > 0)
         hipLaunchKernelGGL(k_zero_ghosts, dim3(64, A.nboxes, 1), dim3(ITPB), 0, s, A, A.dim);
 }
 
 // ------------------------------------------------------------ make_s0mac
-// (1) the profile on every cell of the domain (whole-domain scratch, C order
-// with x fastest), one interpolation per cell
-__global__ void __launch_bounds__(ITPB) k_s0_cells(S0macArgs A)
+// Box blockIdx.y's face arrays of the three directions (one ghost layer: every
+// face of the grown box), each face the mean of its two cells, the cells
+// clamped into the domain (first-order extrapolation outside it).  A block
+// marches a tile of R rows of W columns through 16 planes, one thread per
+// column: it interpolates the profile on its cell, gives the value to its
+// neighbours in x and y through LDS and keeps it for the face above; the first
+// row, column and plane only lead in.  W covers a whole row of the box up to
+// 80 faces: long runs to write, and few of the threads only leading in.
+//
+// Bound by the interpolation and the faces' writes about equally: 256^3 cells
+// (boxes of 64^3, 0.45 GB of faces) take 155 us; a pass for the cells (110 us)
+// and one for the faces took 330.  TAB: the profile is copied to LDS (157 us
+// and 163 without).
+static constexpr int S0_THREADS = 1024, S0_PLANES = 16, S0_ROW = 80;
+template <bool TAB>
+__global__ void __launch_bounds__(S0_THREADS) k_make_s0mac(S0macArgs A)
 {
-    const long nc = (long)A.n[0] * A.n[1] * A.n[2];
-    for (long q = (long)blockIdx.x * ITPB + threadIdx.x; q < nc; q += (long)gridDim.x * ITPB) {
-        const int i = (int)(q % A.n[0]), j = (int)((q / A.n[0]) % A.n[1]), k = (int)(q / ((long)A.n[0] * A.n[1]));
-        A.cells[q] = sphr_cell_value(A.s0, A.geo, i, j, k);
-    }
-}
-
-// (2) one thread per element of box blockIdx.y's face array of direction
-// blockIdx.z (one ghost layer: every face of the grown box): the mean of the
-// face's two cells, clamped into the domain (first-order extrapolation of
-// the cell values outside it)
-__global__ void __launch_bounds__(ITPB) k_make_s0mac(S0macArgs A)
-{
-    const int b = blockIdx.y, d = blockIdx.z;
+    const int b = blockIdx.y;
     const BoxDev B = A.boxes[b];
-    const int ex = B.hi[0] - B.lo[0] + 3 + (d == 0), ey = B.hi[1] - B.lo[1] + 3 + (d == 1);
-    const int ez = B.hi[2] - B.lo[2] + 3 + (d == 2);
-    const long q = (long)blockIdx.x * ITPB + threadIdx.x;
-    if (q >= (long)ex * ey * ez) return;
-    const int g[3] = {B.lo[0] - 1 + (int)(q % ex) - A.dlo[0], B.lo[1] - 1 + (int)((q / ex) % ey) - A.dlo[1],
-                      B.lo[2] - 1 + (int)(q / ((long)ex * ey)) - A.dlo[2]};
-    double v[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        int c[3] = {g[0], g[1], g[2]};
-        c[d] -= s;   // s = 0: the face's high cell, 1: its low cell
-#pragma unroll
-        for (int e = 0; e < 3; ++e) c[e] = c[e] < 0 ? 0 : (c[e] > A.n[e] - 1 ? A.n[e] - 1 : c[e]);
-        v[s] = A.cells[c[0] + (long)A.n[0] * (c[1] + (long)A.n[1] * c[2])];
+    const int n[3] = {B.hi[0] - B.lo[0] + 1, B.hi[1] - B.lo[1] + 1, B.hi[2] - B.lo[2] + 1};
+    // faces: n + 3 along their direction, n + 2 along the others
+    const int nseg = (n[0] + 3 + S0_ROW - 1) / S0_ROW, w = (n[0] + 3 + nseg - 1) / nseg, W = w + 1;
+    const int R = S0_THREADS / W, rows = R - 1;
+    const int nrow = (n[1] + 3 + rows - 1) / rows;
+    if ((int)blockIdx.x >= nseg * nrow) return;
+    const int k0 = blockIdx.z * S0_PLANES, k1 = min(k0 + S0_PLANES, n[2] + 3);
+    if (k0 >= n[2] + 3) return;
+    extern __shared__ double tab[];   // the profile
+    if constexpr (TAB) {
+        for (int q = threadIdx.x; q < A.geo.nr; q += S0_THREADS) tab[q] = A.s0[q];
+        __syncthreads();
     }
-    A.out[b * 3 + d][q] = 0.5 * (v[0] + v[1]);
+    const int tr = blockIdx.x / nseg, ts = blockIdx.x - tr * nseg;
+    const int r = threadIdx.x / W, m = threadIdx.x - r * W;
+    // face (li, lj, k) of the grown box's arrays; cell g of the domain
+    const int li = ts * w + m - 1, lj = tr * rows + r - 1;
+    const bool live = r < R;
+    auto clamp = [&](int d, int l) {
+        const int g = B.lo[d] - 1 + l - A.dlo[d];
+        return g < 0 ? 0 : (g > A.n[d] - 1 ? A.n[d] - 1 : g);
+    };
+    const double x = sphr_x(A.geo, 0, clamp(0, li)), y = sphr_x(A.geo, 1, clamp(1, lj));
+    const double rdr = spacing_recip(A.geo.dr);
+    const bool own = live && m > 0 && r > 0 && li < n[0] + 3 && lj < n[1] + 3;
+    const bool wx = own && lj < n[1] + 2, wy = own && li < n[0] + 2, wz = wx && wy;
+    double *__restrict__ fx = A.out[b * 3], *__restrict__ fy = A.out[b * 3 + 1], *__restrict__ fz = A.out[b * 3 + 2];
+    const long ox = li + (long)(n[0] + 3) * lj, px = (long)(n[0] + 3) * (n[1] + 2);
+    const long oy = li + (long)(n[0] + 2) * lj, py = (long)(n[0] + 2) * (n[1] + 3);
+    const long pz = (long)(n[0] + 2) * (n[1] + 2);
+    __shared__ double v[2][S0_THREADS];
+    const int t = threadIdx.x;
+    double below = 0.0;
+    for (int k = k0 - 1; k < k1; ++k) {
+        const double c = sphr_of(A.geo, sphr_at(A.geo, x, y, sphr_x(A.geo, 2, clamp(2, k)), rdr), TAB ? tab : A.s0);
+        v[k & 1][t] = c;
+        __syncthreads();
+        if (k >= k0) {
+            if (k < n[2] + 2) {
+                if (wx) fx[ox + px * k] = 0.5 * (c + v[k & 1][t - 1]);
+                if (wy) fy[oy + py * k] = 0.5 * (c + v[k & 1][t - W]);
+            }
+            if (wz) fz[oy + pz * k] = 0.5 * (c + below);
+        }
+        below = c;
+    }
 }
 
-void launch_make_s0mac(const S0macArgs &A, int maxfaces, hipStream_t s)
+void launch_make_s0mac(const S0macArgs &A, const int maxext[3], hipStream_t s)
 {
-    const long nc = (long)A.n[0] * A.n[1] * A.n[2];
-    hipLaunchKernelGGL(k_s0_cells, dim3((unsigned)std::min<long>((nc + ITPB - 1) / ITPB, 65536)), dim3(ITPB), 0, s,
-                       A);
-    dim3 g((unsigned)((maxfaces + ITPB - 1) / ITPB), A.nboxes, 3);
-    hipLaunchKernelGGL(k_make_s0mac, g, dim3(ITPB), 0, s, A);
+    // the most tiles of any box: a narrow box has fewer, longer ones in x and
+    // more rows to a tile
+    long tiles = 0;
+    for (int e = 1; e <= maxext[0]; ++e) {
+        const int nseg = (e + 3 + S0_ROW - 1) / S0_ROW, W = (e + 3 + nseg - 1) / nseg + 1, rows = S0_THREADS / W - 1;
+        tiles = std::max(tiles, (long)nseg * ((maxext[1] + 3 + rows - 1) / rows));
+    }
+    const dim3 g((unsigned)tiles, A.nboxes, (unsigned)((maxext[2] + 3 + S0_PLANES - 1) / S0_PLANES));
+    const size_t lds = sizeof(double) * (size_t)A.geo.nr;
+    if (lds <= 48 * 1024) hipLaunchKernelGGL(k_make_s0mac<true>, g, dim3(S0_THREADS), lds, s, A);
+    else hipLaunchKernelGGL(k_make_s0mac<false>, g, dim3(S0_THREADS), 0, s, A);
 }
 
 }  // namespace mac

@@ -150,7 +150,6 @@ struct S0macArgs {
     const BoxDev *boxes;
     int dlo[3], n[3];
     const double *s0;   // radial profile, device
-    double *cells;      // whole-domain scratch: the profile on the cells
     double *const *out; // [box*3 + d]
     SphrGeom geo;
 };
@@ -256,8 +255,8 @@ void launch_ml_grown(int dim, const MlGrown &A, int nboxes, int maxgrown, hipStr
 
 
 void launch_cell_to_edge(const double *c, int nr, double *e, hipStream_t s);
-void launch_make_macrhs(const MacrhsArgs &A, int maxcells, bool sph, hipStream_t s);
-void launch_make_s0mac(const S0macArgs &A, int maxfaces, hipStream_t s);
+void launch_make_macrhs(const MacrhsArgs &A, const int maxext[3], bool sph, hipStream_t s);
+void launch_make_s0mac(const S0macArgs &A, const int maxext[3], hipStream_t s);
 
 // maxcols: the largest x-y cross-section (ex * ey) of a box, maxez the
 // largest z extent; one thread per column and chunk of planes of each box

@@ -141,6 +141,7 @@ struct mac_plan {
     std::vector<BoxDev> boxes;
     BoxDev *boxes_dev = nullptr;
     int maxcells = 0, maxfaces = 0, maxghost = 0;
+    int maxext[3] = {1, 1, 1};   // largest box extent per direction
     int maxcols = 0, maxez = 1;   // largest x-y cross-section and z extent of a box (column kernels)
     long maxplane = 0;
     int *boxmap_dev = nullptr;
@@ -177,7 +178,7 @@ struct mac_plan {
     hipStream_t stream = nullptr;
     hipEvent_t ev[8];
     HostStage hs;
-    double *scratch_cells = nullptr;   // one FP64 cell array (adjoint, make_s0mac)
+    double *scratch_cells = nullptr;   // one FP64 cell array (adjoint)
     void *call_tab = nullptr;          // device pointer tables of the producer calls
     size_t call_tab_cap = 0;
     int device = 0;
@@ -941,6 +942,7 @@ static int plan_create(const mac_layout *lay, const mac_opts *opts, mac_plan **o
         int e[3];
         for (int d = 0; d < 3; ++d) e[d] = (d < P->dim) ? B.hi[d] - B.lo[d] + 1 : 1;
         P->maxcells = std::max(P->maxcells, e[0] * e[1] * e[2]);
+        for (int d = 0; d < 3; ++d) P->maxext[d] = std::max(P->maxext[d], (int)e[d]);
         P->maxcols = std::max(P->maxcols, e[0] * e[1]);
         P->maxez = std::max(P->maxez, e[2]);
         for (int d = 0; d < P->dim; ++d) {
@@ -2075,7 +2077,7 @@ extern "C" int mac_make_macrhs(mac_plan *P, double *const *macrhs, const mac_mac
     A.cutoff_density = in->base_cutoff_density;
     if (sph) A.geo = sphr_geom(P, sph);
     else memset(&A.geo, 0, sizeof A.geo);
-    launch_make_macrhs(A, P->maxcells, sph != nullptr, P->stream);
+    launch_make_macrhs(A, P->maxext, sph != nullptr, P->stream);
     HIPCHK(hipGetLastError());
     if ((rc = S.back_all(macrhs, v_rhs, n_rhs))) return rc;
     if (dpdt_on && (rc = S.back_all(in->delta_chi, v_dchi, n_dchi))) return rc;
@@ -2092,18 +2094,13 @@ extern "C" int mac_make_s0mac(mac_plan *P, const double *s0, const mac_sphr *sph
     int rc;
     CallStage S(P);
     std::vector<size_t> n_f((size_t)nb * 3);
-    int maxfaces = 0;
     for (int b = 0; b < nb; ++b)
-        for (int d = 0; d < 3; ++d) {
-            n_f[b * 3 + d] = box_elems(P, b, 1, d);
-            maxfaces = std::max(maxfaces, (int)n_f[b * 3 + d]);
-        }
+        for (int d = 0; d < 3; ++d) n_f[b * 3 + d] = box_elems(P, b, 1, d);
     std::vector<double *> v_f;
     double **t_f;
     double *d_s0;
     if ((rc = S.reserve(3 * (size_t)nb))) return rc;
     if ((rc = S.table(s0mac, n_f, false, v_f, &t_f)) || (rc = S.view(s0, sph->nr, true, &d_s0))) return rc;
-    if (!P->scratch_cells) HIPCHK(hipMalloc(&P->scratch_cells, sizeof(double) * (size_t)ncell(P->n)));
     S0macArgs A;
     A.nboxes = nb;
     A.boxes = P->boxes_dev;
@@ -2112,10 +2109,9 @@ extern "C" int mac_make_s0mac(mac_plan *P, const double *s0, const mac_sphr *sph
         A.n[d] = P->n[d];
     }
     A.s0 = d_s0;
-    A.cells = P->scratch_cells;
     A.out = t_f;
     A.geo = sphr_geom(P, sph);
-    launch_make_s0mac(A, maxfaces, P->stream);
+    launch_make_s0mac(A, P->maxext, P->stream);
     HIPCHK(hipGetLastError());
     if ((rc = S.back_all(s0mac, v_f, n_f))) return rc;
     HIPCHK(hipStreamSynchronize(P->stream));
