@@ -1514,25 +1514,34 @@ __device__ __forceinline__ void block_max_atomic(double a, unsigned long long *n
 // neighbour rows (a multiple of 8 blocks away for ny a multiple of 32) land
 // on the same XCD.  (Giving each XCD one contiguous slab of rows measured
 // 16% slower on the 256^3 residual.)
+//
+// Levels of fewer than 2048 rows (2D) give each wave one segment of 64 cells of
+// a row instead: the refinement residual of 640 x 384 takes 9.0 us, and took 18.6
+// as 384 waves of ten steps.
 static constexpr int ROW_WAVES = TPB / 64;
+
+__host__ __device__ __forceinline__ int row_segs(int nx, int ny, int nz)
+{
+    return (long)ny * nz < 2048 ? (nx + 63) / 64 : 1;
+}
 
 template <typename F>
 __device__ __forceinline__ void for_rows(int nx, int ny, int nz, F &&f)
 {
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nrow = ny * nz;
-    for (int row = blockIdx.x * ROW_WAVES + wv; row < nrow; row += gridDim.x * ROW_WAVES) {
-        const int k = row / ny, j = row - k * ny;
+    const int nseg = row_segs(nx, ny, nz), n = ny * nz * nseg;
+    for (int u = blockIdx.x * ROW_WAVES + wv; u < n; u += gridDim.x * ROW_WAVES) {
+        const int row = u / nseg, k = row / ny, j = row - k * ny;
         const long base = (long)row * nx;
-        for (int i = lane; i < nx; i += 64) f(i, j, k, base + i);
+        for (int i = lane + 64 * (u - row * nseg); i < nx; i += 64 * nseg) f(i, j, k, base + i);
     }
 }
 
-// grid for for_rows: one wave per row
-static inline unsigned row_blocks(int ny, int nz)
+// grid for for_rows: one wave per row or segment
+static inline unsigned row_blocks(int nx, int ny, int nz)
 {
-    return (unsigned)(((long)ny * nz + ROW_WAVES - 1) / ROW_WAVES);
+    return (unsigned)(((long)ny * nz * row_segs(nx, ny, nz) + ROW_WAVES - 1) / ROW_WAVES);
 }
 
 // residual array and/or its max norm; grid-stride so the norm costs at most
@@ -1601,7 +1610,12 @@ __global__ void __launch_bounds__(TPB) k_ir_update_residual(Lev<double> L, const
 // the plane below, the plane and the plane above in registers, so every
 // array is read from HBM once; the y- and x-neighbour values come from the
 // neighbouring rows and lanes' loads (L1/L2).  Loads are two-element vectors
-// at a uniform plane base plus a lane offset.  Needs 3D and nx = 128 W.
+// at a uniform plane base plus a lane offset.  3D; nx = 128 W, or with FLAT any
+// even nx: the pairs of a plane are dealt to lanes row after row, 64 to a wave,
+// so that a short or ragged row leaves no lanes idle (the row is then the lane's
+// own, which costs address registers: 128 W keeps the uniform form).  Against
+// the row-per-wave kernels: 96 x 80 x 112 MODE 0 31.7 -> 15.8 us, 192^3 with
+// alpha MODE 1 120 -> 92 us, MODE 2 157 -> 107 us (0.45 GB, 4.2 TB/s: memory).
 //   MODE 0: max |rhs - A phi|
 //   MODE 1: r = rhs - A phi written as FP32 (the refinement's right side)
 //   MODE 2: phi' = phi + e (e FP32) formed on the fly for the cell and its
@@ -1617,7 +1631,7 @@ struct RowMarchGrid {
 
 // B16: the FP32 right side goes out as bfloat16 (r16) instead of r32.
 // AL: the level has alpha (+ alpha phi in each residual, as one fma).
-template <int MODE, bool B16, bool AL = false>
+template <int MODE, bool B16, bool AL = false, bool FLAT = false>
 __global__ void __launch_bounds__(256) k_resid_rows(Lev<double> L, const float *__restrict__ e,
                                                    double *__restrict__ phi_out, float *__restrict__ r32,
                                                    unsigned short *__restrict__ r16, unsigned long long *nrm,
@@ -1633,10 +1647,21 @@ __global__ void __launch_bounds__(256) k_resid_rows(Lev<double> L, const float *
     double a = 0.0;
     if (gw < G.total) {
         const int nx = L.nx, ny = L.ny, nz = L.nz, plane = nx * ny;
-        const int seg = gw % G.W, t = gw / G.W;
-        const int j = t % ny, chunk = t / ny;
-        const int z0 = chunk * G.tz, z1 = min(z0 + G.tz, nz);
-        const int x0 = 2 * (lane + 64 * seg);
+        int j, chunk, x0;
+        bool live = true;
+        if constexpr (FLAT) {
+            const int half = nx >> 1, q = gw % G.W * 64 + lane;
+            live = q < half * ny;
+            chunk = gw / G.W;
+            j = live ? q / half : 0;
+            x0 = live ? 2 * (q - j * half) : 0;
+        } else {
+            const int seg = gw % G.W, t = gw / G.W;
+            j = t % ny;
+            chunk = t / ny;
+            x0 = 2 * (lane + 64 * seg);
+        }
+        const int z0 = chunk * G.tz, z1 = live ? min(z0 + G.tz, nz) : z0;
         // neighbour rows / columns: index in range, plus whether it exists
         const bool okym = j > 0 || L.pery, okyp = j < ny - 1 || L.pery;
         const int jm = j > 0 ? j - 1 : ny - 1, jp = j < ny - 1 ? j + 1 : 0;
@@ -1809,10 +1834,12 @@ __global__ void __launch_bounds__(256) k_resid_rows(Lev<double> L, const float *
 // owns one coarse column, i.e. the fine column pair 2I, 2I+1 of the fine row
 // pair 2J, 2J+1, and marches fine planes with the planes below and above in
 // registers.  Per-cell arithmetic and the summation order of the eight fine
-// residuals are those of k_resid_restrict.  3D, fine nx = 128 W.
+// residuals are those of k_resid_restrict.  3D; fine nx = 128 W, or with FLAT
+// any even one (as in k_resid_rows): 192^3 FP32 with alpha 69 us in
+// k_resid_restrict and 31 here, 96 x 80 x 112 FP64 11.8 and 7.5.
 // B16: the fine weights and right side come from compact storage K.
 // AL: the fine level has alpha (+ alpha phi in each residual, as one fma).
-template <typename T, bool B16, bool AL = false>
+template <typename T, bool B16, bool AL = false, bool FLAT = false>
 __global__ void __launch_bounds__(256) k_rr_rows(Lev<T> F, const T *__restrict__ phi, Lev<T> C,
                                                 RowMarchGrid G, Compact16 K)
 {
@@ -1826,10 +1853,21 @@ __global__ void __launch_bounds__(256) k_rr_rows(Lev<T> F, const T *__restrict__
     const int gw = bidx * 4 + wv;
     if (gw >= G.total) return;
     const int nx = F.nx, ny = F.ny, nz = F.nz, plane = nx * ny;
-    const int seg = gw % G.W, t = gw / G.W;
-    const int J = t % C.ny, chunk = t / C.ny;
+    int I, J, chunk;
+    if constexpr (FLAT) {
+        const int q = gw % G.W * 64 + lane;
+        if (q >= C.nx * C.ny) return;
+        chunk = gw / G.W;
+        J = q / C.nx;
+        I = q - J * C.nx;
+    } else {
+        const int seg = gw % G.W, t = gw / G.W;
+        J = t % C.ny;
+        chunk = t / C.ny;
+        I = lane + 64 * seg;
+    }
     const int K0 = chunk * G.tz, K1 = min(K0 + G.tz, C.nz);
-    const int I = lane + 64 * seg, x0 = 2 * I;
+    const int x0 = 2 * I;
     const int j0 = 2 * J, j1 = j0 + 1;
     // rows j0-1 and j1+1 (y-neighbours outside the pair), x-neighbour columns
     const bool okym = j0 > 0 || F.pery, okyp = j1 < ny - 1 || F.pery;
@@ -3393,6 +3431,24 @@ bool launch_gsrb_fused(const Lev<T> &L, const T *pin, T *pout, int mode, hipStre
     return true;
 }
 
+// The flat forms of the row marches: pairs of columns, byte offsets within a
+// plane of 32 bits.
+static bool flat_ok(int nx, int ny)
+{
+    return nx % 2 == 0 && (long)nx * ny < (1L << 28);
+}
+// waves of 64 columns, planes per chunk between lo and hi for some 4096 waves
+static RowMarchGrid flat_grid(long cols, int nz, int lo, int hi)
+{
+    RowMarchGrid G;
+    G.W = (int)((cols + 63) / 64);
+    G.tz = (int)std::max((long)lo, std::min((long)hi, (long)G.W * nz / 4096));
+    G.tz = std::min(G.tz, nz);
+    G.total = G.W * ((nz + G.tz - 1) / G.tz);
+    G.per_xcd = ((G.total + 3) / 4 + 7) / 8;
+    return G;
+}
+
 template <typename T>
 bool launch_resid_restrict(int dim, const Lev<T> &F, const T *phi, const Lev<T> &C, hipStream_t s,
                            const Compact16 *K, const RhoLev *Rh)
@@ -3432,6 +3488,15 @@ bool launch_resid_restrict(int dim, const Lev<T> &F, const T *phi, const Lev<T> 
         return true;
     }
     if (K) return false;
+    if (dim == 3 && flat_ok(F.nx, F.ny) && F.nx == 2 * C.nx && F.ny == 2 * C.ny && F.nz == 2 * C.nz) {
+        const RowMarchGrid G = flat_grid((long)C.nx * C.ny, C.nz, 1, 16);
+        const Compact16 K0 = {};
+        if (F.alpha)
+            hipLaunchKernelGGL((k_rr_rows<T, false, true, true>), dim3(8 * G.per_xcd), dim3(256), 0, s, F, phi, C, G, K0);
+        else
+            hipLaunchKernelGGL((k_rr_rows<T, false, false, true>), dim3(8 * G.per_xcd), dim3(256), 0, s, F, phi, C, G, K0);
+        return true;
+    }
     dim3 g((C.nx + 63) / 64, C.ny, C.nz);
     if (dim == 3)
         hipLaunchKernelGGL((k_resid_restrict<3, T>), g, dim3(256), 0, s, F, phi, C);
@@ -3470,14 +3535,25 @@ void launch_to_bf16(const float *in, unsigned short *out, long n, hipStream_t s)
 
 static constexpr unsigned NORM_GRID = 2048;   // 256 CUs x 8 blocks
 
-// Row-march form of the FP64 residual passes where it applies (3D, nx a
-// multiple of 128); false otherwise (the row-per-wave kernels then run).
+// Row-march form of the FP64 residual passes where it applies (3D, nx even);
+// false otherwise (the row-per-wave kernels then run).
 // The z-chunk length is 32 planes, fewer on small levels.
 template <int MODE>
 static bool launch_resid_rows(const Lev<double> &L, const float *e, double *phi_out, float *r32,
                               unsigned long long *nrm, hipStream_t s, unsigned short *r16 = nullptr)
 {
-    if (L.nx % 128 != 0 || L.nz < 2) return false;
+    if (L.nz < 2) return false;
+    if (L.nx % 128 != 0) {
+        if (r16 || !flat_ok(L.nx, L.ny)) return false;
+        const RowMarchGrid G = flat_grid((long)(L.nx / 2) * L.ny, L.nz, 2, 32);
+        if (L.alpha)
+            hipLaunchKernelGGL((k_resid_rows<MODE, false, true, true>), dim3(8 * G.per_xcd), dim3(256), 0, s, L, e,
+                               phi_out, r32, r16, nrm, G);
+        else
+            hipLaunchKernelGGL((k_resid_rows<MODE, false, false, true>), dim3(8 * G.per_xcd), dim3(256), 0, s, L, e,
+                               phi_out, r32, r16, nrm, G);
+        return true;
+    }
     RowMarchGrid G;
     G.W = L.nx / 128;
     // planes per chunk: 32, fewer on small levels (some 4096 waves in all)
@@ -3509,7 +3585,7 @@ void launch_residual(int dim, const Lev<T> &L, T *out, unsigned long long *nrm, 
             launch_resid_rows<0>(L, nullptr, nullptr, nullptr, nrm, s))
             return;
     }
-    const unsigned rb = row_blocks(L.ny, L.nz);
+    const unsigned rb = row_blocks(L.nx, L.ny, L.nz);
     unsigned g = nrm ? std::min(rb, NORM_GRID) : rb;
     DISPATCH_DIM(dim, hipLaunchKernelGGL((k_residual<D_, T>), dim3(g), dim3(TPB), 0, s, L, out, nrm));
 }
@@ -3518,7 +3594,7 @@ void launch_ir_residual(int dim, const Lev<double> &L, float *r32, unsigned long
                         hipStream_t s, unsigned short *r16)
 {
     if (dim == 3 && launch_resid_rows<1>(L, nullptr, nullptr, r32, nrm, s, r16)) return;
-    unsigned g = std::min(row_blocks(L.ny, L.nz), NORM_GRID);
+    unsigned g = std::min(row_blocks(L.nx, L.ny, L.nz), NORM_GRID);
     DISPATCH_DIM(dim, hipLaunchKernelGGL(k_ir_residual<D_>, dim3(g), dim3(TPB), 0, s, L, r32, nrm));
 }
 
@@ -3526,7 +3602,7 @@ void launch_ir_update_residual(int dim, const Lev<double> &L, const float *e, do
                                unsigned long long *nrm, hipStream_t s, unsigned short *r16)
 {
     if (dim == 3 && launch_resid_rows<2>(L, e, phi_out, r32, nrm, s, r16)) return;
-    unsigned g = std::min(row_blocks(L.ny, L.nz), NORM_GRID);
+    unsigned g = std::min(row_blocks(L.nx, L.ny, L.nz), NORM_GRID);
     DISPATCH_DIM(dim, hipLaunchKernelGGL(k_ir_update_residual<D_>, dim3(g), dim3(TPB), 0, s, L, e, phi_out,
                                          r32, nrm));
 }
@@ -3585,7 +3661,7 @@ void launch_prolong(int dim, const Lev<T> &F, const Lev<T> &C, const EllBC &bc, 
                            C.nx, C.ny, C.nz, bc, W, pz, total);
         return;
     }
-    DISPATCH_DIM(dim, hipLaunchKernelGGL((k_prolong<D_, T>), dim3(row_blocks(F.ny, F.nz)), dim3(TPB), 0, s,
+    DISPATCH_DIM(dim, hipLaunchKernelGGL((k_prolong<D_, T>), dim3(row_blocks(F.nx, F.ny, F.nz)), dim3(TPB), 0, s,
                                          F, (const T *)C.phi, C.nx, C.ny, C.nz, bc));
 }
 

@@ -398,7 +398,7 @@ __device__ __forceinline__ void ml_norm_max(double amax, unsigned long long *nrm
     if (threadIdx.x == 0) {
         double m = wm[0];
         for (int w = 1; w < MTPB / 64; ++w) m = fmax(m, wm[w]);
-        if (m > 0.0) atomicMax(nrm, (unsigned long long)__double_as_longlong(m));
+        atomic_max_nonneg(nrm, m);
     }
 }
 
