@@ -786,7 +786,7 @@ struct BottomWave {
 // all its readers have passed).  Only the waves that hold cells run the solve;
 // the others wait at its barriers (idle), since their instructions would take
 // the busy waves' turns: 6 x 5 x 7 cells FP64, 3100 -> 2150 cycles a CG step.
-template <int DIM>
+template <int DIM, bool FOLD>   // FOLD: more than 512 cells
 struct BottomBlock {
     static constexpr bool POW2 = false;
     bool live;
@@ -853,8 +853,24 @@ struct BottomBlock {
         fs ^= 1;
         return a;
     }
+    // Beyond 512 cells a sum takes cells t and t + 512 together, then the waves
+    // in order.  A singular bottom's constant mode is whatever the rounding of
+    // its sums leaves in it, and phi's constant with it: the order is part of
+    // the result (k_bottom's blocks of 512 threads add alike).
+    __device__ __forceinline__ double folded(double v)
+    {
+        if constexpr (!FOLD) return v;
+        double *a = xs + (flip ? n + 2 : 1);
+        flip ^= 1;
+        const int t = threadIdx.x;
+        if (live && t >= 512) a[t] = v;
+        sync();
+        if (t >= 512) return 0.0;
+        return t + 512 < n ? v + a[t + 512] : v;
+    }
     __device__ __forceinline__ double sum(double v)
     {
+        v = folded(v);
         double *a = slot();
         v = wsum(v);
         if ((threadIdx.x & 63) == 0) a[threadIdx.x >> 6] = v;
@@ -871,6 +887,7 @@ struct BottomBlock {
     }
     __device__ __forceinline__ void sum_max(double &s, double &m)   // one barrier for both
     {
+        s = folded(s);
         double *a = slot();
         s = wsum(s);
         m = wmax(m);
@@ -1260,25 +1277,29 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
             const bool live = t < n;
             const int q = live ? t : 0;
             cell(q, w, a, colour);
-            BottomBlock<DIM> X;
-            X.live = live;
-            X.n = held(n);
-            X.flip = X.fs = X.bar = 0;
-            X.xs = reinterpret_cast<double *>(smem_ + M.xs);
-            X.sh = reinterpret_cast<double *>(smem_ + M.sh);
-            X.last = reinterpret_cast<int *>(X.sh + 64);
-            if (t == 0) X.xs[0] = X.xs[n + 1] = 0.0;
-            if (t == 0) *X.last = 0;
-            if (t < 64) X.sh[t] = 0.0;
-            if ((t & ~63) < n) {
-                cell_nbrs<DIM, T>(L, q, -1, X.nb);
-                X.sync();   // the zeros above
-                const T v = bottom_solve<DIM, T>(L, X, w, a, colour, live ? E[q] : T(0), live ? R[q] : T(0), o, n);
-                if (live) E[t] = v;
-                X.finish();
-            } else {
-                X.idle();
-            }
+            auto block = [&](auto FC) __attribute__((always_inline)) {
+                BottomBlock<DIM, decltype(FC)::value> X;
+                X.live = live;
+                X.n = held(n);
+                X.flip = X.fs = X.bar = 0;
+                X.xs = reinterpret_cast<double *>(smem_ + M.xs);
+                X.sh = reinterpret_cast<double *>(smem_ + M.sh);
+                X.last = reinterpret_cast<int *>(X.sh + 64);
+                if (t == 0) X.xs[0] = X.xs[n + 1] = 0.0;
+                if (t == 0) *X.last = 0;
+                if (t < 64) X.sh[t] = 0.0;
+                if ((t & ~63) < n) {
+                    cell_nbrs<DIM, T>(L, q, -1, X.nb);
+                    X.sync();   // the zeros above
+                    const T v = bottom_solve<DIM, T>(L, X, w, a, colour, live ? E[q] : T(0), live ? R[q] : T(0), o, n);
+                    if (live) E[t] = v;
+                    X.finish();
+                } else {
+                    X.idle();
+                }
+            };
+            if (n > 512) block(std::true_type{});
+            else block(std::false_type{});
         }
         __syncthreads();
     };

@@ -138,3 +138,26 @@ def test_bottoms(gpu, oracle_lib, n, bottom, cycle):
     ref, _, _, _ = O.mg_solve(g, b, phi, rhs, O.default_opts(max_iter=1, eps_rel=1e-300, bottom_maxit=400, **opts))
     got = plan.debug_get(0, "phi").reshape(phi.shape)
     assert np.abs(got - ref).max() <= max(1e-12, 6.5 * dim * max(m) ** 2 * 1e-15) * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("bottom", [1, 2])
+@pytest.mark.parametrize("n", [(11, 7, 9), (9, 9, 8), (27, 31), (19, 27), (32, 31)])
+def test_bottom_sums_beyond_512_cells(gpu, oracle_lib, n, bottom):
+    """A singular bottom of 513 to 1024 cells: the solution is the oracle's but
+    for a constant, and the same bits on every call."""
+    O = oracle_lib
+    dim = len(n)
+    bc = [[WALL, WALL]] * dim
+    g, b, _, rhs = level(O, n, bc, 37)
+    rhs -= rhs.mean()
+    got = []
+    opts = dict(bottom_eps=1e-13, bottom_solver=bottom)
+    for _ in range(2):
+        plan = make_plan(n, bc, bottom_max_iter=400, **opts)
+        push_level(plan, 0, bc, n, b, np.zeros_like(rhs), rhs, dim)
+        plan.debug_op(0, "vcycle")
+        got.append(plan.debug_get(0, "phi").reshape(rhs.shape))
+    ref, _, _, _ = O.mg_solve(g, b, np.zeros_like(rhs), rhs, O.default_opts(max_iter=1, eps_rel=1e-300, bottom_maxit=400, **opts))
+    assert np.array_equal(got[0], got[1])
+    d, e = got[0] - got[0].mean(), ref - ref.mean()
+    assert np.abs(d - e).max() <= 6.5 * dim * max(n) ** 2 * 1e-13 * np.abs(e).max()
