@@ -49,14 +49,15 @@ OMEGA_HEADLINE = 1.25
 
 def sweep_kernel_name(s: int, b16: bool = False, nx: int = 256, rho: bool = False, sor: bool = False,
                       pz: bool = False) -> str:
-    """Name of the finest-level sweep kernel the library launches (b16: the
+    """Name of the finest-level sweep kernel the library launches.  FP64, and
+    FP32 with stored weights but at nx = 128: k_sweep2, two sweeps in one pass.
+    Else one sweep per launch (b16: the
     compact bfloat16-storage form of the FP32 full-row kernel; rho: the FP32
     form that forms its weights from the density, which the plane-parallel
     mixed path runs).  Full rows,
-    W = nx / 128 waves per row; rows x threads per block: FP64 6 x 768, FP32
-    6 x 768 with the weights fetched one plane ahead (16 x 1024 at nx = 128),
-    FP32 with bfloat16 storage 6 x 768; the template's last two arguments: no
-    alpha term, the weights' prefetch distance; the last: over-relaxed (sor).
+    W = nx / 128 waves per row; rows x threads per block: FP32 16 x 1024 at
+    nx = 128, with bfloat16 storage 6 x 768; the template's last arguments: no
+    alpha term, the weights' prefetch distance, over-relaxed (sor).
     The rho form's last argument: z periodic (pz; the workloads here have z
     walls)."""
     t = "double" if s == 8 else "float"
@@ -66,10 +67,11 @@ def sweep_kernel_name(s: int, b16: bool = False, nx: int = 256, rho: bool = Fals
     if rho:   # FP32, the weights formed from rho: 6 rows x 768 (12 x 768 at nx = 128)
         z = "true" if pz else "false"
         return f"k_gsrb_rows_rho<0, 6, 768, {w}, {o}, {z}>" if w == 2 else f"k_gsrb_rows_rho<0, 12, 768, 1, {o}, {z}>"
-    if s == 8 or b16:
+    if b16:
         return f"k_gsrb_rows<{t}, 0, 6, 768, {c}, {w}, false, 2, {o}>"
-    return (f"k_gsrb_rows<{t}, 0, 16, 1024, {c}, 1, false, 2, {o}>" if w == 1
-            else f"k_gsrb_rows<{t}, 0, 6, 768, {c}, {w}, false, 1, {o}>")
+    if s == 8 or w != 1:
+        return f"k_sweep2<{t}, {16 if s == 8 else 32}, 32, false, false, {o}>"
+    return f"k_gsrb_rows<{t}, 0, 16, 1024, {c}, 1, false, 2, {o}>"
 
 
 def measured_traffic(name: str):
@@ -90,7 +92,7 @@ def measured_traffic(name: str):
 
 def gsrb_launch_bytes(ncell: int, s: int, ws: int = None, rho: bool = False) -> float:
     """Algorithmic bytes of one launch of the fused 3D red-black sweep (one
-    full sweep): three face weights and rhs (element size ws), the old
+    full sweep, or k_sweep2's two): three face weights and rhs (element size ws), the old
     iterate read and the new one written (element size s), each once per
     cell -> 2 s + 4 ws per cell; in the rho form (the weights formed from
     the FP32 density) rho and rhs -> 2 s + 2 ws."""
@@ -614,7 +616,8 @@ def main():
         name = sweep_kernel_name(s_, b16, n[0], rho, sor)
         return {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": measured_traffic(name),
-                "kernel": name + " (finest level, one full red-black sweep)",
+                "kernel": name + (" (finest level, two red-black sweeps)" if name.startswith("k_sweep2")
+                                  else " (finest level, one full red-black sweep)"),
                 "avg_launch_us": round(1e3 * avg, 2), "launches": cnt_, "bytes_per_launch": nbytes}
 
     producers = None if args.no_producers else time_producers(plan, n, args.box, torch)

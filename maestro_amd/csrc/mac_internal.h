@@ -35,13 +35,12 @@ struct Lev {
     T *bx, *by, *bz;
     T *bxh, *byh, *bzh;
     // cell coefficient of the Helmholtz operator (alpha - D beta G); null for
-    // the projection (alpha = 0).  Only the generic kernels (per-colour
-    // sweep, residual, coarsening, coarse cycle) read it.
+    // the projection (alpha = 0).
     T *alpha;
     // over-relaxation of this level's red-black sweeps: a cell moves to
     // old + omega (gs - old); 1 (set when the level is built) keeps
     // Gauss-Seidel, and only then do the sweeps store the Gauss-Seidel value
-    // itself (the single-workgroup coarse cycle never reads it)
+    // itself
     T omega;
 };
 

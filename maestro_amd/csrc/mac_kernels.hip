@@ -12,8 +12,8 @@
 //   k_residual         compute_defect (mg.tex:351)
 //   k_restrict         conservative-average restriction (mg.tex:353-354)
 //   k_prolong          linear prolongation + correction (mg.tex:363-365)
-//   k_coarse_cycle     the cycle (V, W or F) on the coarse levels plus the
-//                      FP64 CG bottom solve (mg.tex:221-262) in one workgroup
+//   k_bottom           the FP64 bottom solve (mg.tex:221-262) of a bottom level
+//                      of more than 1024 cells in one workgroup
 //   k_correct_valid    mkumac_3d (:908-975) fused with the division by beta0
 //                      (:232-236)
 //   k_fill_ghost       multifab_fill_boundary of umac (:245-251)

@@ -710,9 +710,8 @@ static int inner_per_step(const mac_opts &o, bool compact)
 }
 
 // Solve A phi = rhs on level 0 of H64 (phi holds the warm start).
-// Over-relaxation of the red-black sweeps on the levels above the
-// single-workgroup coarse cycle (which keeps Gauss-Seidel): mac_opts.omega
-// where set, else 1 (FBoxLib's GSRB).  With 1.25 the 256^3 plane-parallel
+// Over-relaxation of the red-black sweeps on the levels of more than
+// relaxed_above() cells (the others keep Gauss-Seidel): mac_opts.omega where set, else 1 (FBoxLib's GSRB).  With 1.25 the 256^3 plane-parallel
 // projection converges in 6 V-cycles instead of 9 and the 512^3 star in 12
 // instead of 16 (to 1e-10, the oracle's FP64 cycle), but at the same relative
 // residual the over-relaxed iterate leaves more of its error in smooth modes:
