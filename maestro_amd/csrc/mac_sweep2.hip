@@ -337,14 +337,13 @@ static int chunk_planes(int nz, int tiles, int slots)
 template <typename T, int HX, int RY>
 static void launch_sweep2_t(const Lev<T> &L, const T *pin, T *pout, int mode, hipStream_t s)
 {
-    static int slots = 0;   // one block per CU (registers)
-    if (slots == 0) {
+    static const int slots = [] {   // one block per CU (registers)
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
             cus = 256;
-        slots = cus;
-    }
+        return cus;
+    }();
     Sweep2Grid G;
     G.ntx = (L.nx + 2 * HX - 9) / (2 * HX - 8);
     G.nty = (L.ny + RY - 9) / (RY - 8);
