@@ -481,10 +481,14 @@ static void cycle_from(mac_plan *P, Hier<T> &H, int l, int type, bool zero, cons
     const mac_opts &o = P->opts;
     Lev<T> &L = H.lev[l];
     const long n = (long)L.nx * L.ny * L.nz;
-    if (l == H.lc) {
+    // the coarse cycle reads the FP32 weights and right side, which a level 0
+    // in compact or rho form does not have (128 x 4 x 8 cells fit it): that level
+    // runs its own kernels and the cycle starts below it
+    const bool own_form = l == 0 && H.nlev > 1 && (K || Rh);
+    if (l >= H.lc && !own_form) {
         const CoarseOpts co = coarse_opts(P, type);
         int q = prof_begin(P, MAC_PROF_COARSE);
-        if (!launch_coarse<T>(dim, H.lev.data(), H.lc, H.nlev, co, zero, s)) {
+        if (!launch_coarse<T>(dim, H.lev.data(), l, H.nlev, co, zero, s)) {
             if (zero) launch_fill<T>(L.phi, n, T(0), s);
             launch_bottom<T>(dim, L, co, P->cg, s);
         }
