@@ -563,6 +563,10 @@ static bool compact_applies(mac_plan *P)
            compact_level_ok(P->dim, P->H32.lev[0]);
 }
 
+// whether a solve keeps it so: a level that is also the bottom is solved from
+// the FP32 weights and right side
+static bool compact_solve(mac_plan *P) { return compact_applies(P) && P->H32.nlev > 1; }
+
 // whether the FP32 finest level runs in the rho form: MAC_PREC_MIXED, a 3D
 // projection with a planar beta0 (the face coefficients are 2 beta0^p /
 // (rho_L + rho_R)), x and y periodic, nx = 128 or 256, at least two levels
@@ -763,7 +767,7 @@ static int solve(mac_plan *P, mac_stats *st)
             for (int l = 2; l < P->H32.nlev; ++l)
                 launch_coarsen<float>(P->dim, P->H32.lev[l - 1], P->H32.lev[l], P->stream);
             Rh = &P->H32.rho0;
-        } else if (compact_applies(P) && P->H32.nlev > 1) {
+        } else if (compact_solve(P)) {
             // compact level 0 and FP32 level 1 in one pass, then the rest
             if ((rc = compact_level0(P, &K, true))) return rc;
             for (int l = 2; l < P->H32.nlev; ++l)
@@ -771,7 +775,6 @@ static int solve(mac_plan *P, mac_stats *st)
         } else {
             launch_weights_to_f32(P->dim, P->H64.lev[0], P->H32.lev[0], P->stream);
             coarsen_all<float>(P, P->H32);
-            if ((rc = compact_level0(P, &K, false))) return rc;
         }
         P->launch_failed = false;
         int bad = 0;
@@ -1361,7 +1364,7 @@ static bool storage_ready(mac_plan *P)
     if (!P->H64.built) return false;
     if (P->opts.precision == MAC_PREC_FP64) return true;
     if (!P->H32.built) return false;
-    return !(compact_applies(P) && P->c16_allocs.empty());
+    return !(compact_solve(P) && P->c16_allocs.empty());
 }
 
 // mac_project; noalloc: the call's buffers come from the scratch array and

@@ -8,8 +8,11 @@ from maestro_amd import mac
 from maestro_amd import workloads as W
 
 from .helpers import rel_err, run_gpu, run_oracle
+from .test_gpu_kernels import make_plan, rand_level
 
 pytestmark = pytest.mark.gpu
+
+P, WALL, OUT = W.PERIODIC, W.SLIP_WALL, W.OUTLET
 
 
 @pytest.mark.parametrize("cycle", [mac.CYCLE_V, mac.CYCLE_F, mac.CYCLE_W])
@@ -33,3 +36,21 @@ def test_finest_level_of_4096_cells(gpu, oracle_lib, prec, cycle, top):
     # NaN fails both; the bounds are those of the parity tests
     assert e_phi <= max(1e-8, 2.0 * e_ref)
     assert e_u <= 1e-8
+
+
+@pytest.mark.parametrize("n,levels", [((128, 3, 8), 0), ((256, 3, 9), 0), ((128, 4, 8), 1), ((128, 12, 16), 1)])
+@pytest.mark.parametrize("bc", [[[P, P], [WALL, WALL], [WALL, OUT]], [[OUT, WALL], [WALL, OUT], [WALL, WALL]]])
+def test_bf16_of_one_level(gpu, oracle_lib, n, levels, bc):
+    """MAC_PREC_MIXED_BF16 where the finest level is the bottom."""
+    torch, O = gpu, oracle_lib
+    g = O.make_grid(n, [1.0 / n[0]] * 3, bc)
+    b, phi, rhs = rand_level(g, n, 3, np.random.default_rng(61), O)
+    plan = make_plan(n, bc, precision=mac.PREC_MIXED_BF16, max_levels=levels, device_ptrs=1)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    ph = t(np.zeros_like(phi))
+    st = plan.project_level(*[t(np.zeros(O.face_shape(g, d))) for d in range(3)], ph, *[t(x) for x in b], t(rhs), check=False)
+    res, _ = O.residual(g, b, ph.cpu().numpy(), rhs)
+    print(n, st["iters"], np.abs(res).max())
+    # the tolerance asked for, and the rounding of a residual: some 20 operations on terms of 6 w ih2 |phi|
+    tol = 1e-10 * np.abs(rhs).max() + 20 * 2.0 ** -53 * 12 * 2.0 * n[0] ** 2 * np.abs(ph.cpu().numpy()).max()
+    assert st["converged"] and np.abs(res).max() <= tol
