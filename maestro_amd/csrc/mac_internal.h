@@ -98,6 +98,35 @@ __device__ __forceinline__ T quot(T n, T d, T r)
     q = dfma(dfma(-d, q, n), r, q);
     return dfma(dfma(-d, q, n), r, q);
 }
+// Where d or 1 / d is no normal number quot has nothing to work with.  Two ways
+// out, both off the chain of the updates (a test per quotient costs a bottom
+// solve 3%): a wave that has met such a d divides (quot_ok), or the cell's whole
+// equation is scaled by a power of two where d is small (is_tiny; the reciprocal of
+// a large d, a division's, is denormal, which the correction steps make good).
+//
+// Whether quot serves two divisors, in four operations on their exponents
+__device__ __forceinline__ bool quot_ok(float a, float b)
+{
+    const unsigned lo = 0x00800000u << 1, hi = 0x7e800000u << 1;   // 2^-126, 2^126
+    const unsigned x = (__float_as_uint(a) << 1) - lo, y = (__float_as_uint(b) << 1) - lo;
+    return max(x, y) <= hi - lo;
+}
+__device__ __forceinline__ bool quot_ok(double a, double b)
+{
+    const unsigned lo = 0x00100000u << 1, hi = 0x7fc00000u << 1;   // 2^-1022, 2^1021
+    const unsigned x = ((unsigned)__double2hiint(a) << 1) - lo, y = ((unsigned)__double2hiint(b) << 1) - lo;
+    return max(x, y) <= hi - lo;
+}
+template <typename T>
+__device__ __forceinline__ bool is_tiny(T d)
+{
+    return fabs(d) < (sizeof(T) == 8 ? T(0x1p-960) : T(0x1p-96f));
+}
+// a factor that brings every tiny d into the range, and the way back
+template <typename T>
+__device__ __forceinline__ T tiny_up() { return sizeof(T) == 8 ? T(0x1p+160) : T(0x1p+80f); }
+template <typename T>
+__device__ __forceinline__ T tiny_down() { return T(1) / tiny_up<T>(); }
 
 // Neighbour values and face weights of cell (i,j,k), index c.
 // Order: x-, x+, y-, y+, z-, z+.

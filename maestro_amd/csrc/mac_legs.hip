@@ -98,10 +98,12 @@ __device__ __forceinline__ T apply_w(const Lev<T> &L, const T *w, const T *p, T 
 
 // A pair of cells: [0] the red one, [1] the black one.  Where j + k is odd the
 // red cell is the right one.
+// tiny: the cell's weights, diagonal and right side are scaled by tiny_up().
 template <int DIM, typename T>
 struct Pair {
     T w[2][2 * DIM];
     T den[2], inv[2], rhs[2];
+    bool tiny[2];
 };
 
 // what a pair is made of, as loaded
@@ -132,6 +134,36 @@ __device__ __forceinline__ PairRaw<DIM, T> load_raw(const Lev<T> &L, int i, int 
     return R;
 }
 
+template <int DIM, typename T>
+__device__ __forceinline__ void scale_tiny(Pair<DIM, T> &P)
+{
+    P.tiny[0] = is_tiny(P.den[0]);
+    P.tiny[1] = is_tiny(P.den[1]);
+    if (__builtin_expect(__any(P.tiny[0] || P.tiny[1]), 0)) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const T f = P.tiny[c] ? tiny_up<T>() : T(1);
+#pragma unroll
+            for (int q = 0; q < 2 * DIM; ++q) P.w[c][q] *= f;
+            P.den[c] *= f;
+            P.rhs[c] *= f;
+        }
+    }
+}
+
+// the right side of the pair's cell c, and its ap = A phi, without that scale
+template <int DIM, typename T>
+__device__ __forceinline__ T true_scale(const Pair<DIM, T> &P, int c, T &ap)
+{
+    T r = P.rhs[c];
+    if (__builtin_expect(__any(P.tiny[c]), 0)) {
+        const T f = P.tiny[c] ? tiny_down<T>() : T(1);
+        ap *= f;
+        r *= f;
+    }
+    return r;
+}
+
 // s: j + k is odd
 template <int DIM, typename T>
 __device__ __forceinline__ Pair<DIM, T> make_pair(const Lev<T> &L, const PairRaw<DIM, T> &R, bool s)
@@ -153,6 +185,7 @@ __device__ __forceinline__ Pair<DIM, T> make_pair(const Lev<T> &L, const PairRaw
     P.rhs[1] = s ? R.r.a : R.r.b;
     P.den[0] = gs_den<DIM, T>(L, P.w[0], s ? R.al.b : R.al.a);
     P.den[1] = gs_den<DIM, T>(L, P.w[1], s ? R.al.a : R.al.b);
+    scale_tiny(P);
 #pragma unroll
     for (int c = 0; c < 2; ++c) P.inv[c] = T(1) / P.den[c];
     return P;
@@ -175,6 +208,7 @@ __device__ __forceinline__ Pair<DIM, T> dead_pair()
         for (int q = 0; q < 2 * DIM; ++q) P.w[c][q] = T(0);
         P.den[c] = P.inv[c] = T(1);
         P.rhs[c] = T(0);
+        P.tiny[c] = false;
     }
     return P;
 }
@@ -439,8 +473,9 @@ __global__ void __launch_bounds__(NTH) k_leg(Lev<T> L, const T *__restrict__ pin
                 pair_nbrs<DIM, T>(S[1 - c], s[a], c, v[a][1 - c], o - 1, o + 1, o - G::SY, o + G::SY, o - G::SZ,
                                   o + G::SZ, p);
                 T ap = apply_w<DIM, T>(L, P[a].w[c], p, v[a][c]);
+                const T r = true_scale(P[a], c, ap);
                 if (L.alpha) ap = dfma(L.alpha[c0 + (s[a] != (c == 1) ? 1 : 0)], v[a][c], ap);
-                res[c] = P[a].rhs[c] - ap;
+                res[c] = r - ap;
             }
             rs[(m - 2) + CX * ((jj - H) + TY * (DIM == 3 ? kk - H : 0))] = res[0] + res[1];
         }
@@ -599,10 +634,19 @@ __device__ __forceinline__ T bottom_solve(const Lev<T> &L_, X &x_, const T *w, T
     const bool has_alpha = held((int)(L_.alpha != nullptr));
     const int n_sweeps = held(o.nub), singular = held(o.singular);
     const double eps = held(o.bottom_eps);
-    const T den = gs_den<DIM, T>(L, w, acell), inv = T(1) / den;
-    T wn[2 * DIM];   // for the sweeps' sums of neighbours
+    // for the sweeps: the weights of the neighbours, the diagonal and the right
+    // side, scaled as a pair's where the diagonal is tiny
+    T wn[2 * DIM], den = gs_den<DIM, T>(L, w, acell), rn = rhs;
 #pragma unroll
     for (int s = 0; s < 2 * DIM; ++s) wn[s] = x_.has(s) ? w[s] : T(0);
+    if (__builtin_expect(__any(live && is_tiny(den)), 0)) {
+        const T f = is_tiny(den) ? tiny_up<T>() : T(1);
+#pragma unroll
+        for (int s = 0; s < 2 * DIM; ++s) wn[s] *= f;
+        den *= f;
+        rn *= f;
+    }
+    const T inv = T(1) / den;
     // the mean of a sum over the cells
     auto mean = [&](double v) -> double { return X::POW2 ? v * (1.0 / n) : v / (double)n; };
     Lev<double> D;
@@ -623,7 +667,7 @@ __device__ __forceinline__ T bottom_solve(const Lev<T> &L_, X &x_, const T *w, T
         for (int h = 0; h < 2 * n_sweeps; ++h) {
             T p[2 * DIM];
             x_.nbrs_any(phi, p);
-            const T v = quot(gs_num<DIM, T>(L, wn, p, rhs), den, inv);
+            const T v = quot(gs_num<DIM, T>(L, wn, p, rn), den, inv);
             if (live && colour == (h & 1)) phi = v;
         }
         if (part == 1 || o.bottom == MAC_BOTTOM_SMOOTH) continue;
@@ -689,7 +733,8 @@ __device__ __forceinline__ T bottom_solve(const Lev<T> &L_, X &x_, const T *w, T
                 double rr1 = r * r, am = fabs(r);
                 x_.sum_max(rr1, am);
                 if (am <= eps * r0) break;
-                const double beta = quot(rr1, rr, irr);
+                double beta = quot(rr1, rr, irr);
+                if (__builtin_expect(!__builtin_isnormal(irr), 0)) beta = rr1 / rr;
                 rr = rr1;
                 p = r + beta * p;
             }
@@ -1018,6 +1063,7 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
     Pair<DIM, T> Pm;      // the pair of a level between that this thread owns
     PairPos om;
     int lm = 0, qm = 0;   // that level (0: none), the pair's place in it
+    bool tiny0 = false, tiny1 = false;   // Pair::tiny of Pm
     // the deeper levels' pairs, the bottom's weights and level 0's iterate
     // (pairs at o0): every load issued before the first is waited for
     auto stage = [&](const PairPos(&o0)[NP]) {
@@ -1070,6 +1116,8 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
         }
         if (lm) {
             Pm = make_pair<DIM, T>(LV.l[lm], Rm, om.s);
+            tiny0 = Pm.tiny[0];
+            tiny1 = Pm.tiny[1];
             if constexpr (PARK) {
                 T *f = arr(M.park) + t;
 #pragma unroll
@@ -1134,7 +1182,8 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
             if constexpr (PARK) pos = pair_pos<DIM, T>(C, qm, M.S[l], M.mx[l], M.my[l]);
             else pos = om;
             const T a = restricted(F, 2 * pos.m, pos.j, pos.k), b = restricted(F, 2 * pos.m + 1, pos.j, pos.k);
-            const T r0 = pos.s ? b : a, r1 = pos.s ? a : b;
+            const T r0 = (pos.s ? b : a) * (tiny0 ? tiny_up<T>() : T(1));
+            const T r1 = (pos.s ? a : b) * (tiny1 ? tiny_up<T>() : T(1));
             if constexpr (PARK) {
                 arr(M.park)[(4 * DIM + 4) * M.mid + t] = r0;
                 arr(M.park)[(4 * DIM + 5) * M.mid + t] = r1;
@@ -1203,8 +1252,9 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
                 T p[2 * DIM];
                 nbrs(pos[a], c, CS, v[a][1 - c], p);
                 T ap = apply_w<DIM, T>(L, P[a].w[c], p, v[a][c]);
+                const T r = true_scale(P[a], c, ap);
                 if (L.alpha) ap = dfma(L.alpha[2 * pos[a].q + (pos[a].s != (c == 1) ? 1 : 0)], v[a][c], ap);
-                res[c] = P[a].rhs[c] - ap;
+                res[c] = r - ap;
             }
             arr(M.rs)[pos[a].q] = res[0] + res[1];
         }
@@ -1225,6 +1275,8 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
                     P[0].inv[c] = f[(4 * DIM + 2 + c) * M.mid];
                     P[0].rhs[c] = f[(4 * DIM + 4 + c) * M.mid];
                 }
+                P[0].tiny[0] = tiny0;
+                P[0].tiny[1] = tiny1;
             }
             leg(l, up, std::integral_constant<int, CM>{}, P, pos, [&](int) { return lm == l; });
         } else {
@@ -1425,7 +1477,7 @@ static bool coarse_map(int dim, const Lev<T> *levs, int lc, int nlev, CoarseMap 
     M.xs = take(nb > 64 ? 2 * (nb + 1) * 8 : 0);
     M.sh = take(nb > 64 ? 65 * 8 : 0);
     M.mid = (int)mid;
-    M.park = take(dim == 3 ? mid * (long)sizeof(Pair<3, T>) : 0);
+    M.park = take(dim == 3 ? 18 * mid * sz : 0);   // 12 weights, diagonals, reciprocals, right sides
     M.bytes = (int)off;
     return off <= COARSE_LDS;
 }

@@ -54,7 +54,7 @@ __device__ __forceinline__ T pick(bool c, T a, T b)
 // of which gives the correctly rounded value (P. Markstein, IBM J. Res. Dev.
 // 34 (1990) 111-119; a d with all mantissa bits set may be one off, which quot
 // makes good).  A division does the same with scaling for the ends of the
-// exponent range.
+// exponent range; there (quot_ok) the march divides.
 __device__ __forceinline__ float recip(float d)
 {
     const float r = __builtin_amdgcn_rcpf(d);
@@ -210,6 +210,7 @@ __global__ void __launch_bounds__(HX *RY) k_sweep2(Lev<T> L, const T *__restrict
     }
     T2 pc = load_p(q0), pn = load_p(q1);   // old values of planes k, k + 1
     T2 zc = load_z(q0), zn = load_z(q1);   // low z faces of planes k, k + 1
+    bool by_div = false;   // quot does not serve a diagonal so far
     bool tp1 = false, tp2 = false, tp3 = false;   // whether planes k - 1, k - 2, k - 3 are the domain's top
     load_w(q0);
     __syncthreads();
@@ -254,6 +255,7 @@ __global__ void __launch_bounds__(HX *RY) k_sweep2(Lev<T> L, const T *__restrict
             }
             w.i[0] = recip(w.d[0]);
             w.i[1] = recip(w.d[1]);
+            by_div = by_div || __any(!quot_ok(w.d[0], w.d[1]));
             zc = zn;
             load_w(q1);
             zn = load_z(q2);
@@ -266,14 +268,15 @@ __global__ void __launch_bounds__(HX *RY) k_sweep2(Lev<T> L, const T *__restrict
             __syncthreads();
             // the update of column C of plane p: O its plane's other colour in
             // LDS, zm, zp the column's values below and above, zh its high z face
-            auto update = [&](auto CC, const W &q, const T *O, T own, T oth, T zm, T zp, T zh) -> T {
+            auto update = [&](auto CC, auto DC, const W &q, const T *O, T own, T oth, T zm, T zp, T zh) -> T {
                 constexpr int C = decltype(CC)::value;
+                constexpr bool DIV = decltype(DC)::value;
                 const T xo = O[C ? pos + 1 : pos - 1];
                 const T tx = dfma(C ? T(q.x1) : T(q.x0), C ? T(oth) : T(xo), (C ? T(q.x2) : T(q.x1)) * (C ? T(xo) : T(oth)));
                 const T ty = dfma(q.yl[C], O[pos - PX], q.yh[C] * O[pos + PX]);
                 const T tz = dfma(q.zl[C], zm, zh * zp);
                 const T num = dfma(ih2x, tx, dfma(ih2y, ty, dfma(ih2z, tz, q.r[C])));
-                return relax<SOR>(quot(num, q.d[C], q.i[C]), own, omega);
+                return relax<SOR>(DIV ? num / q.d[C] : quot(num, q.d[C], q.i[C]), own, omega);
             };
             using CA = std::integral_constant<int, R0>;
             using CB = std::integral_constant<int, R0 ^ 1>;
@@ -283,19 +286,27 @@ __global__ void __launch_bounds__(HX *RY) k_sweep2(Lev<T> L, const T *__restrict
                 const T a = pick(t, R0 ? T(top1) : T(top0), above);
                 return pick(below && k - b < 0, T(0), a);
             };
-            // first red half-sweep, plane k, column R0
-            v[S][R0] = update(CA{}, w, A[0][B], v[S][R0], v[S][R0 ^ 1], v[S1][R0], R0 ? T(pc.b) : T(pc.a), R0 ? T(zh1) : T(zh0));
-            A[1][B][pos] = v[S][R0];
-            // first black half-sweep, plane k - 1: its black column is R1 ^ 1 = R0
-            v[S1][R0] = update(CA{}, wq[S1], A[1][B ^ 1], v[S1][R0], v[S1][R1], v[S2][R0], v[S][R0], zhi(1, tp1, w.zl[R0]));
-            A[2][B ^ 1][pos] = v[S1][R0];
-            // second red, plane k - 2, column R2 = R0
-            v[S2][R2] = update(CA{}, wq[S2], A[2][B], v[S2][R2], v[S2][R2 ^ 1], v[S3][R2], v[S1][R2],
-                               zhi(2, tp2, wq[S1].zl[R0]));
-            A[3][B][pos] = v[S2][R2];
-            // second black, plane k - 3, column R3 ^ 1 = R0
-            v[S3][R0] = update(CA{}, wq[S3], A[3][B ^ 1], v[S3][R0], v[S3][R3], R0 ? T(last1) : T(last0), v[S2][R0],
-                               zhi(3, tp3, wq[S2].zl[R0]));
+            auto halves = [&](auto DC) __attribute__((always_inline)) {
+                // first red half-sweep, plane k, column R0
+                v[S][R0] = update(CA{}, DC, w, A[0][B], v[S][R0], v[S][R0 ^ 1], v[S1][R0], R0 ? T(pc.b) : T(pc.a),
+                                  R0 ? T(zh1) : T(zh0));
+                A[1][B][pos] = v[S][R0];
+                // first black half-sweep, plane k - 1: its black column is R1 ^ 1 = R0
+                v[S1][R0] = update(CA{}, DC, wq[S1], A[1][B ^ 1], v[S1][R0], v[S1][R1], v[S2][R0], v[S][R0],
+                                   zhi(1, tp1, w.zl[R0]));
+                A[2][B ^ 1][pos] = v[S1][R0];
+                // second red, plane k - 2, column R2 = R0
+                v[S2][R2] = update(CA{}, DC, wq[S2], A[2][B], v[S2][R2], v[S2][R2 ^ 1], v[S3][R2], v[S1][R2],
+                                   zhi(2, tp2, wq[S1].zl[R0]));
+                A[3][B][pos] = v[S2][R2];
+                // second black, plane k - 3, column R3 ^ 1 = R0
+                v[S3][R0] = update(CA{}, DC, wq[S3], A[3][B ^ 1], v[S3][R0], v[S3][R3], R0 ? T(last1) : T(last0), v[S2][R0],
+                                   zhi(3, tp3, wq[S2].zl[R0]));
+            };
+            // the second form costs 1.5 us a launch (its instructions), a test in
+            // each update 1.5% of a 256^3 FP64 pair
+            if (__builtin_expect(by_div, 0)) halves(std::true_type{});
+            else halves(std::false_type{});
             tp3 = tp2;
             tp2 = tp1;
             tp1 = tp0;
