@@ -2341,23 +2341,32 @@ __device__ __forceinline__ double blk_max(double v, double *sh)
     return s;
 }
 
+// One red-black sweep.  Two cells of a colour are neighbours across an odd
+// period: a half-sweep then takes all its values (tmp, one per cell) before it
+// writes one, as the single-workgroup cycle's bottom does.
 template <int DIM, typename T>
-__device__ void blk_gsrb(const Lev<T> &L)
+__device__ void blk_gsrb(const Lev<T> &L, T *tmp)
 {
     const int hx = (L.nx + 1) >> 1;
     const int nq = hx * L.ny * L.nz;
+    const bool seam = (L.perx && (L.nx & 1)) || (L.pery && (L.ny & 1)) || (DIM == 3 && L.perz && (L.nz & 1));
+    T *out = seam ? tmp : L.phi;
     for (int color = 0; color < 2; ++color) {
-        for (int q = threadIdx.x; q < nq; q += blockDim.x) {
-            const int r = q / hx, m = q - r * hx;
-            const int k = r / L.ny, j = r - k * L.ny;
-            int i = 2 * m + ((j + k + color) & 1);
-            if (i >= L.nx) continue;
-            const int c = i + L.nx * (j + L.ny * k);
+        auto cells = [&](auto &&f) {
+            for (int q = threadIdx.x; q < nq; q += blockDim.x) {
+                const int r = q / hx, m = q - r * hx;
+                const int k = r / L.ny, j = r - k * L.ny;
+                const int i = 2 * m + ((j + k + color) & 1);
+                if (i < L.nx) f(i, j, k, i + L.nx * (j + L.ny * k));
+            }
+            __syncthreads();
+        };
+        cells([&](int i, int j, int k, int c) {
             T w[6], p[6];
             stencil<DIM, T>(L, L.phi, i, j, k, c, w, p);
-            L.phi[c] = gs_value<DIM, T>(L, w, p, L.rhs[c], alpha_at(L, c));
-        }
-        __syncthreads();
+            out[c] = gs_value<DIM, T>(L, w, p, L.rhs[c], alpha_at(L, c));
+        });
+        if (seam) cells([&](int, int, int, int c) { L.phi[c] = tmp[c]; });
     }
 }
 
@@ -2576,12 +2585,12 @@ template <int DIM, typename T>
 __global__ void __launch_bounds__(CTPB) k_bottom(Lev<T> L, CoarseOpts o, double *cg)
 {
     __shared__ double sh[CTPB / 64];
-    for (int s = 0; s < o.nub; ++s) blk_gsrb<DIM, T>(L);
+    for (int s = 0; s < o.nub; ++s) blk_gsrb<DIM, T>(L, reinterpret_cast<T *>(cg));
     if (o.bottom == MAC_BOTTOM_CG)
         blk_bottom_cg<DIM, T>(L, cg, o.bottom_eps, o.bottom_maxit, o.singular, sh);
     else if (o.bottom == MAC_BOTTOM_BICGSTAB)
         blk_bottom_bicgstab<DIM, T>(L, cg, o.bottom_eps, o.bottom_maxit, o.singular, sh);
-    for (int s = 0; s < o.nub; ++s) blk_gsrb<DIM, T>(L);
+    for (int s = 0; s < o.nub; ++s) blk_gsrb<DIM, T>(L, reinterpret_cast<T *>(cg));
 }
 
 // ------------------------------------------------------ face correction
