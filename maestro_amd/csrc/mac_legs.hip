@@ -139,7 +139,7 @@ __device__ __forceinline__ void scale_tiny(Pair<DIM, T> &P)
 {
     P.tiny[0] = is_tiny(P.den[0]);
     P.tiny[1] = is_tiny(P.den[1]);
-    if (__builtin_expect(__any(P.tiny[0] || P.tiny[1]), 0)) {
+    if (__builtin_expect(__ballot(P.tiny[0] || P.tiny[1]) != 0, 0)) {
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             const T f = P.tiny[c] ? tiny_up<T>() : T(1);
@@ -156,7 +156,7 @@ template <int DIM, typename T>
 __device__ __forceinline__ T true_scale(const Pair<DIM, T> &P, int c, T &ap)
 {
     T r = P.rhs[c];
-    if (__builtin_expect(__any(P.tiny[c]), 0)) {
+    if (__builtin_expect(__ballot(P.tiny[c]) != 0, 0)) {
         const T f = P.tiny[c] ? tiny_down<T>() : T(1);
         ap *= f;
         r *= f;
@@ -639,7 +639,7 @@ __device__ __forceinline__ T bottom_solve(const Lev<T> &L_, X &x_, const T *w, T
     T wn[2 * DIM], den = gs_den<DIM, T>(L, w, acell), rn = rhs;
 #pragma unroll
     for (int s = 0; s < 2 * DIM; ++s) wn[s] = x_.has(s) ? w[s] : T(0);
-    if (__builtin_expect(__any(live && is_tiny(den)), 0)) {
+    if (__builtin_expect(__ballot(live && is_tiny(den)) != 0, 0)) {
         const T f = is_tiny(den) ? tiny_up<T>() : T(1);
 #pragma unroll
         for (int s = 0; s < 2 * DIM; ++s) wn[s] *= f;
@@ -734,7 +734,7 @@ __device__ __forceinline__ T bottom_solve(const Lev<T> &L_, X &x_, const T *w, T
                 x_.sum_max(rr1, am);
                 if (am <= eps * r0) break;
                 double beta = quot(rr1, rr, irr);
-                if (__builtin_expect(!__builtin_isnormal(irr), 0)) beta = rr1 / rr;
+                if (__builtin_expect(__ballot(!__builtin_isnormal(irr)) != 0, 0)) beta = rr1 / rr;
                 rr = rr1;
                 p = r + beta * p;
             }

@@ -210,7 +210,7 @@ __global__ void __launch_bounds__(HX *RY) k_sweep2(Lev<T> L, const T *__restrict
     }
     T2 pc = load_p(q0), pn = load_p(q1);   // old values of planes k, k + 1
     T2 zc = load_z(q0), zn = load_z(q1);   // low z faces of planes k, k + 1
-    bool by_div = false;   // quot does not serve a diagonal so far
+    unsigned long long by_div = 0;   // the lanes where quot does not serve a diagonal so far
     bool tp1 = false, tp2 = false, tp3 = false;   // whether planes k - 1, k - 2, k - 3 are the domain's top
     load_w(q0);
     __syncthreads();
@@ -255,7 +255,7 @@ __global__ void __launch_bounds__(HX *RY) k_sweep2(Lev<T> L, const T *__restrict
             }
             w.i[0] = recip(w.d[0]);
             w.i[1] = recip(w.d[1]);
-            by_div = by_div || __any(!quot_ok(w.d[0], w.d[1]));
+            by_div |= __ballot(!quot_ok(w.d[0], w.d[1]));
             zc = zn;
             load_w(q1);
             zn = load_z(q2);
@@ -303,9 +303,10 @@ __global__ void __launch_bounds__(HX *RY) k_sweep2(Lev<T> L, const T *__restrict
                 v[S3][R0] = update(CA{}, DC, wq[S3], A[3][B ^ 1], v[S3][R0], v[S3][R3], R0 ? T(last1) : T(last0), v[S2][R0],
                                    zhi(3, tp3, wq[S2].zl[R0]));
             };
-            // the second form costs 1.5 us a launch (its instructions), a test in
-            // each update 1.5% of a 256^3 FP64 pair
-            if (__builtin_expect(by_div, 0)) halves(std::true_type{});
+            // a scalar branch on the ballot keeps the second form out of the march
+            // (0.5 us a launch; a branch on a lane mask 1.5, a test in each update
+            // 1.5% of a 256^3 FP64 pair)
+            if (__builtin_expect(by_div != 0, 0)) halves(std::true_type{});
             else halves(std::false_type{});
             tp3 = tp2;
             tp2 = tp1;
