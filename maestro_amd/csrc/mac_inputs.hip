@@ -175,26 +175,27 @@ __device__ __forceinline__ double sphr_x(const SphrGeom &G, int d, int i)
 }
 
 // ----------------------------------------------------------- make_macrhs
-// One thread per column (i, j) of box blockIdx.y's valid cells, blockIdx.z's
-// planes of it.  TAB: the radial profiles are copied to LDS first.  A row of
-// cells reaches over as many cache lines of a profile as it has bins across,
-// and a cell takes 15 such gathers (five quadratic profiles).  Bound by the
-// interpolations' FP64 instructions and their latency: 256^3 cells, six arrays
-// of 0.13 GB, take 255 us; with the profiles in memory, a branch per quotient
-// and the streams' loads after the interpolation 326, with a division per
-// quotient and 64-bit index divisions per cell 336.  Blocks of 512 threads
-// (three to a CU with 44 KB of profiles) 255, of 1024 (one) 269.
-static constexpr int MACRHS_PLANES = 16;
+// One thread per column (i, j) of box blockIdx.y's valid cells; blockIdx.x is a
+// tile of NT columns and a chunk of `planes` planes, the tiles of a chunk first
+// (with the chunks outermost of all a 256^3 planar call takes 310 us for 294).
+// TAB: the radial profiles are copied to LDS first.  A row of cells reaches over
+// as many cache lines of a profile as it has bins across, and a cell takes 15
+// such gathers (five quadratic profiles).  Bound by the interpolations' FP64
+// instructions and their latency: 256^3 cells, six arrays of 0.13 GB, take 255
+// us; with the profiles in memory, a branch per quotient and the streams' loads
+// after the interpolation 326, with a division per quotient and 64-bit index
+// divisions per cell 336.  Blocks of 512 threads (three to a CU with 44 KB of
+// profiles) 255, of 1024 (one) 269.
 template <int DIM, bool SPH, bool TAB>
-__global__ void __launch_bounds__(TAB ? 512 : ITPB) k_make_macrhs(MacrhsArgs A)
+__global__ void __launch_bounds__(TAB ? 512 : ITPB) k_make_macrhs(MacrhsArgs A, int planes, int tiles)
 {
     constexpr int NT = TAB ? 512 : ITPB;
     const int b = blockIdx.y;
     const BoxDev B = A.boxes[b];
     const int ex = B.hi[0] - B.lo[0] + 1, ey = B.hi[1] - B.lo[1] + 1;
     const int ez = (DIM == 3) ? B.hi[2] - B.lo[2] + 1 : 1;
-    const int k0 = blockIdx.z * MACRHS_PLANES, k1 = min(k0 + MACRHS_PLANES, ez);
-    const int p = blockIdx.x * NT + threadIdx.x;
+    const int chunk = blockIdx.x / tiles, k0 = chunk * planes, k1 = min(k0 + planes, ez);
+    const int p = ((int)blockIdx.x - chunk * tiles) * NT + threadIdx.x;
     if (k0 >= ez) return;
     extern __shared__ double tab[];
     const int nr = A.geo.nr;
@@ -287,22 +288,33 @@ __global__ void __launch_bounds__(ITPB) k_zero_ghosts(MacrhsArgs A, int dim)
     }
 }
 
+// Planes of a chunk (spherical): as many as leave some 2048 blocks of 512
+// threads, 16 at most.  A thread's planes follow each other in a chain of square
+// roots and interpolations, so a small domain wants them side by side, and the
+// profiles from memory (a block of few cells does not repay the copy).  Calls in
+// microseconds, by planes 1, 2, 4, 8, 16: 64^3 50, 50, 55, 63, 82 (profiles in memory,
+// blocks of 256: 50, 51, 54, 63, 80), 96^3 77, 76, 77, 79, 98 (75, 74, 77, 82, 96), 128^3
+// 96, 92, 90, 92, 99 (94, 91, 92, 96, 109), 256^3 467, 420, 398, 386, 387 (476 .. 486).
+// A planar cell is a few loads and little else: one plane a chunk at every size.
 void launch_make_macrhs(const MacrhsArgs &A, const int maxext[3], bool sph, hipStream_t s)
 {
-    auto go = [&](auto k, int nt, size_t lds) {
-        const dim3 g((unsigned)(((long)maxext[0] * maxext[1] + nt - 1) / nt), A.nboxes,
-                     (unsigned)((maxext[2] + MACRHS_PLANES - 1) / MACRHS_PLANES));
-        hipLaunchKernelGGL(k, g, dim3(nt), lds, s, A);
+    const long cols = (long)maxext[0] * maxext[1];
+    auto go = [&](auto k, int nt, size_t lds, int planes) {
+        const int tiles = (int)((cols + nt - 1) / nt);
+        const dim3 g((unsigned)((long)tiles * ((maxext[2] + planes - 1) / planes)), A.nboxes);
+        hipLaunchKernelGGL(k, g, dim3(nt), lds, s, A, planes, tiles);
     };
     if (A.dim == 3 && sph) {
+        const long blocks = (cols + 511) / 512 * maxext[2] * A.nboxes;
+        const int planes = blocks <= 1024 ? 1 : (int)std::max(2L, std::min(16L, (blocks + 2047) / 2048));
         // two blocks or more to a CU
         const size_t lds = sizeof(double) * (size_t)A.geo.nr * (A.dpdt_on ? 5 : 2);
-        if (lds <= 64 * 1024) go(k_make_macrhs<3, true, true>, 512, lds);
-        else go(k_make_macrhs<3, true, false>, ITPB, 0);
+        if (blocks > 2048 && lds <= 64 * 1024) go(k_make_macrhs<3, true, true>, 512, lds, planes);
+        else go(k_make_macrhs<3, true, false>, ITPB, 0, planes);
     } else if (A.dim == 3) {
-        go(k_make_macrhs<3, false, false>, ITPB, 0);
+        go(k_make_macrhs<3, false, false>, ITPB, 0, 1);
     } else {
-        go(k_make_macrhs<2, false, false>, ITPB, 0);
+        go(k_make_macrhs<2, false, false>, ITPB, 0, 1);
     }
     if (A.dpdt_on && A.predictor && A.ng_dchi > 0)
         hipLaunchKernelGGL(k_zero_ghosts, dim3(64, A.nboxes, 1), dim3(ITPB), 0, s, A, A.dim);
@@ -311,37 +323,38 @@ void launch_make_macrhs(const MacrhsArgs &A, const int maxext[3], bool sph, hipS
 // ------------------------------------------------------------ make_s0mac
 // Box blockIdx.y's face arrays of the three directions (one ghost layer: every
 // face of the grown box), each face the mean of its two cells, the cells
-// clamped into the domain (first-order extrapolation outside it).  A block
-// marches a tile of R rows of W columns through 16 planes, one thread per
-// column: it interpolates the profile on its cell, gives the value to its
-// neighbours in x and y through LDS and keeps it for the face above; the first
-// row, column and plane only lead in.  W covers a whole row of the box up to
-// 80 faces: long runs to write, and few of the threads only leading in.
+// clamped into the domain (first-order extrapolation outside it).  A block of
+// NT threads marches a tile of R rows of W columns through `planes` planes, one
+// thread per column: it interpolates the profile on its cell, gives the value to
+// its neighbours in x and y through LDS and keeps it for the face above; the
+// first row, column and plane only lead in.  W covers a whole row of the box up
+// to 80 faces: long runs to write, and few of the threads only leading in.
 //
 // Bound by the interpolation and the faces' writes about equally: 256^3 cells
 // (boxes of 64^3, 0.45 GB of faces) take 155 us; a pass for the cells (110 us)
 // and one for the faces took 330.  TAB: the profile is copied to LDS (157 us
 // and 163 without).
-static constexpr int S0_THREADS = 1024, S0_PLANES = 16, S0_ROW = 80;
-template <bool TAB>
-__global__ void __launch_bounds__(S0_THREADS) k_make_s0mac(S0macArgs A)
+static constexpr int S0_ROW = 80;
+template <bool TAB, int NT>
+__global__ void __launch_bounds__(NT) k_make_s0mac(S0macArgs A, int planes)
 {
     const int b = blockIdx.y;
     const BoxDev B = A.boxes[b];
     const int n[3] = {B.hi[0] - B.lo[0] + 1, B.hi[1] - B.lo[1] + 1, B.hi[2] - B.lo[2] + 1};
     // faces: n + 3 along their direction, n + 2 along the others
     const int nseg = (n[0] + 3 + S0_ROW - 1) / S0_ROW, w = (n[0] + 3 + nseg - 1) / nseg, W = w + 1;
-    const int R = S0_THREADS / W, rows = R - 1;
+    const int R = NT / W, rows = R - 1;
     const int nrow = (n[1] + 3 + rows - 1) / rows;
-    if ((int)blockIdx.x >= nseg * nrow) return;
-    const int k0 = blockIdx.z * S0_PLANES, k1 = min(k0 + S0_PLANES, n[2] + 3);
+    const int tile = blockIdx.x;
+    if (tile >= nseg * nrow) return;
+    const int k0 = blockIdx.z * planes, k1 = min(k0 + planes, n[2] + 3);
     if (k0 >= n[2] + 3) return;
     extern __shared__ double tab[];   // the profile
     if constexpr (TAB) {
-        for (int q = threadIdx.x; q < A.geo.nr; q += S0_THREADS) tab[q] = A.s0[q];
+        for (int q = threadIdx.x; q < A.geo.nr; q += NT) tab[q] = A.s0[q];
         __syncthreads();
     }
-    const int tr = blockIdx.x / nseg, ts = blockIdx.x - tr * nseg;
+    const int tr = tile / nseg, ts = tile - tr * nseg;
     const int r = threadIdx.x / W, m = threadIdx.x - r * W;
     // face (li, lj, k) of the grown box's arrays; cell g of the domain
     const int li = ts * w + m - 1, lj = tr * rows + r - 1;
@@ -358,7 +371,7 @@ __global__ void __launch_bounds__(S0_THREADS) k_make_s0mac(S0macArgs A)
     const long ox = li + (long)(n[0] + 3) * lj, px = (long)(n[0] + 3) * (n[1] + 2);
     const long oy = li + (long)(n[0] + 2) * lj, py = (long)(n[0] + 2) * (n[1] + 3);
     const long pz = (long)(n[0] + 2) * (n[1] + 2);
-    __shared__ double v[2][S0_THREADS];
+    __shared__ double v[2][NT];
     const int t = threadIdx.x;
     double below = 0.0;
     for (int k = k0 - 1; k < k1; ++k) {
@@ -376,19 +389,39 @@ __global__ void __launch_bounds__(S0_THREADS) k_make_s0mac(S0macArgs A)
     }
 }
 
-void launch_make_s0mac(const S0macArgs &A, const int maxext[3], hipStream_t s)
+// the most tiles of any box: a narrow box has fewer, longer ones in x and more
+// rows to a tile
+static long s0_tiles(const int maxext[3], int nt)
 {
-    // the most tiles of any box: a narrow box has fewer, longer ones in x and
-    // more rows to a tile
     long tiles = 0;
     for (int e = 1; e <= maxext[0]; ++e) {
-        const int nseg = (e + 3 + S0_ROW - 1) / S0_ROW, W = (e + 3 + nseg - 1) / nseg + 1, rows = S0_THREADS / W - 1;
+        const int nseg = (e + 3 + S0_ROW - 1) / S0_ROW, W = (e + 3 + nseg - 1) / nseg + 1, rows = nt / W - 1;
         tiles = std::max(tiles, (long)nseg * ((maxext[1] + 3 + rows - 1) / rows));
     }
-    const dim3 g((unsigned)tiles, A.nboxes, (unsigned)((maxext[2] + 3 + S0_PLANES - 1) / S0_PLANES));
+    return tiles;
+}
+
+// Planes of a chunk: as many as leave some 800 blocks of 512 threads, 16 at most
+// (one more plane leads in).  Blocks of 1024 threads for chunks of 16 planes where
+// their tiles fit the boxes as well.  Calls in microseconds, by planes 1, 2, 4, 8,
+// 16: 64^3 35, 33, 33, 37, 45 (blocks of 1024: 35, 33, 36, 43, 56), 128^3 85, 70,
+// 64, 59, 65, 256^3 in boxes of 64 455, 341, 291, 259, 246 (1024: 434 .. 234), of
+// 32 978, 861, 804, 778, 774 (1141 .. 818).
+void launch_make_s0mac(const S0macArgs &A, const int maxext[3], hipStream_t s)
+{
+    const long t512 = s0_tiles(maxext, 512), t1024 = s0_tiles(maxext, 1024);
+    const int nz = maxext[2] + 3;
+    const int planes = (int)std::min(16L, (t512 * nz * A.nboxes + 799) / 800);
     const size_t lds = sizeof(double) * (size_t)A.geo.nr;
-    if (lds <= 48 * 1024) hipLaunchKernelGGL(k_make_s0mac<true>, g, dim3(S0_THREADS), lds, s, A);
-    else hipLaunchKernelGGL(k_make_s0mac<false>, g, dim3(S0_THREADS), 0, s, A);
+    auto go = [&](auto k, long tiles, int nt, size_t bytes) {
+        const dim3 g((unsigned)tiles, A.nboxes, (unsigned)((nz + planes - 1) / planes));
+        hipLaunchKernelGGL(k, g, dim3(nt), bytes, s, A, planes);
+    };
+    const bool tab = lds <= 48 * 1024;
+    if (planes == 16 && 2 * t1024 <= t512)
+        tab ? go(k_make_s0mac<true, 1024>, t1024, 1024, lds) : go(k_make_s0mac<false, 1024>, t1024, 1024, 0);
+    else
+        tab ? go(k_make_s0mac<true, 512>, t512, 512, lds) : go(k_make_s0mac<false, 512>, t512, 512, 0);
 }
 
 }  // namespace mac
