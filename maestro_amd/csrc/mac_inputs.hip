@@ -175,8 +175,8 @@ __device__ __forceinline__ double sphr_x(const SphrGeom &G, int d, int i)
 }
 
 // ----------------------------------------------------------- make_macrhs
-// One thread per column (i, j) of box blockIdx.y's valid cells; blockIdx.x is a
-// tile of NT columns and a chunk of `planes` planes, the tiles of a chunk first
+// One thread per column (i, j) of box blockIdx.y's valid cells and chunk of
+// `planes` planes; blockIdx.x is a tile of NT columns and a chunk, the tiles first
 // (with the chunks outermost of all a 256^3 planar call takes 310 us for 294).
 // TAB: the radial profiles are copied to LDS first.  A row of cells reaches over
 // as many cache lines of a profile as it has bins across, and a cell takes 15
@@ -194,8 +194,16 @@ __global__ void __launch_bounds__(TAB ? 512 : ITPB) k_make_macrhs(MacrhsArgs A, 
     const BoxDev B = A.boxes[b];
     const int ex = B.hi[0] - B.lo[0] + 1, ey = B.hi[1] - B.lo[1] + 1;
     const int ez = (DIM == 3) ? B.hi[2] - B.lo[2] + 1 : 1;
-    const int chunk = blockIdx.x / tiles, k0 = chunk * planes, k1 = min(k0 + planes, ez);
-    const int p = ((int)blockIdx.x - chunk * tiles) * NT + threadIdx.x;
+    int chunk, p;
+    if constexpr (SPH && !TAB) {   // small domains: no lanes left over at a chunk's end
+        const int q = blockIdx.x * NT + threadIdx.x;
+        chunk = q / (ex * ey);
+        p = q - chunk * (ex * ey);
+    } else {
+        chunk = blockIdx.x / tiles;
+        p = ((int)blockIdx.x - chunk * tiles) * NT + threadIdx.x;
+    }
+    const int k0 = chunk * planes, k1 = min(k0 + planes, ez);
     if (k0 >= ez) return;
     extern __shared__ double tab[];
     const int nr = A.geo.nr;
@@ -289,23 +297,23 @@ __global__ void __launch_bounds__(ITPB) k_zero_ghosts(MacrhsArgs A, int dim)
 }
 
 // Planes of a chunk (spherical): as many as leave some 2048 blocks of 512
-// threads, 16 at most.  A thread's planes follow each other in a chain of square
+// threads, 16 at most (cells: of all boxes).  A thread's planes follow each other in a chain of square
 // roots and interpolations, so a small domain wants them side by side, and the
 // profiles from memory (a block of few cells does not repay the copy).  Calls in
 // microseconds, by planes 1, 2, 4, 8, 16: 64^3 50, 50, 55, 63, 82 (profiles in memory,
 // blocks of 256: 50, 51, 54, 63, 80), 96^3 77, 76, 77, 79, 98 (75, 74, 77, 82, 96), 128^3
 // 96, 92, 90, 92, 99 (94, 91, 92, 96, 109), 256^3 467, 420, 398, 386, 387 (476 .. 486).
 // A planar cell is a few loads and little else: one plane a chunk at every size.
-void launch_make_macrhs(const MacrhsArgs &A, const int maxext[3], bool sph, hipStream_t s)
+void launch_make_macrhs(const MacrhsArgs &A, const int maxext[3], long cells, bool sph, hipStream_t s)
 {
     const long cols = (long)maxext[0] * maxext[1];
     auto go = [&](auto k, int nt, size_t lds, int planes) {
-        const int tiles = (int)((cols + nt - 1) / nt);
-        const dim3 g((unsigned)((long)tiles * ((maxext[2] + planes - 1) / planes)), A.nboxes);
-        hipLaunchKernelGGL(k, g, dim3(nt), lds, s, A, planes, tiles);
+        const long tiles = (cols + nt - 1) / nt;   // enough for either order
+        const dim3 g((unsigned)(tiles * ((maxext[2] + planes - 1) / planes)), A.nboxes);
+        hipLaunchKernelGGL(k, g, dim3(nt), lds, s, A, planes, (int)tiles);
     };
     if (A.dim == 3 && sph) {
-        const long blocks = (cols + 511) / 512 * maxext[2] * A.nboxes;
+        const long blocks = cells / 512;   // at one plane a chunk
         const int planes = blocks <= 1024 ? 1 : (int)std::max(2L, std::min(16L, (blocks + 2047) / 2048));
         // two blocks or more to a CU
         const size_t lds = sizeof(double) * (size_t)A.geo.nr * (A.dpdt_on ? 5 : 2);

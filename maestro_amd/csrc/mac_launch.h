@@ -255,7 +255,7 @@ void launch_ml_grown(int dim, const MlGrown &A, int nboxes, int maxgrown, hipStr
 
 
 void launch_cell_to_edge(const double *c, int nr, double *e, hipStream_t s);
-void launch_make_macrhs(const MacrhsArgs &A, const int maxext[3], bool sph, hipStream_t s);
+void launch_make_macrhs(const MacrhsArgs &A, const int maxext[3], long cells, bool sph, hipStream_t s);
 void launch_make_s0mac(const S0macArgs &A, const int maxext[3], hipStream_t s);
 
 // maxcols: the largest x-y cross-section (ex * ey) of a box, maxez the

@@ -2083,7 +2083,9 @@ extern "C" int mac_make_macrhs(mac_plan *P, double *const *macrhs, const mac_mac
     A.cutoff_density = in->base_cutoff_density;
     if (sph) A.geo = sphr_geom(P, sph);
     else memset(&A.geo, 0, sizeof A.geo);
-    launch_make_macrhs(A, P->maxext, sph != nullptr, P->stream);
+    long cells = 0;
+    for (int b = 0; b < nb; ++b) cells += (long)box_elems(P, b, 0, -1);
+    launch_make_macrhs(A, P->maxext, cells, sph != nullptr, P->stream);
     HIPCHK(hipGetLastError());
     if ((rc = S.back_all(macrhs, v_rhs, n_rhs))) return rc;
     if (dpdt_on && (rc = S.back_all(in->delta_chi, v_dchi, n_dchi))) return rc;

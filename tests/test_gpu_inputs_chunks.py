@@ -1,7 +1,7 @@
 """make_macrhs and make_s0mac where their chunks of planes and blocks of
 threads depend on the domain: one plane a chunk, two from profiles in memory,
-several from profiles in LDS, the last chunk short; chunks of 16 planes in blocks
-of 1024 threads.  Bit for bit against the oracle."""
+several from profiles in LDS or too long for it, the last chunk short; chunks of
+16 planes in blocks of 512 and 1024 threads.  Bit for bit against the oracle."""
 import pytest
 
 from . import test_gpu_inputs_profiles as T
@@ -10,12 +10,11 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,box,bins,interp,dpdt", [
-    ((15, 10, 20), 5, 5, 3, 0.5),     # one plane
-    ((30, 30, 30), 5, 5, 3, 0.5),     # two planes, profiles in memory: 2, 2, 1
-    ((56, 56, 56), 8, 5, 2, -1.0),    # two planes, profiles in LDS
-    ((70, 70, 70), 7, 5, 3, 0.5),     # four: 4, 3
-    ((70, 70, 70), 7, 100, 3, 0.5),   # the same, profiles too long for LDS
-    ((72, 72, 72), 6, 5, 1, 0.5),     # six, the whole box
+    ((15, 10, 20), 5, 5, 3, 0.5),        # one plane
+    ((90, 90, 90), 9, 5, 3, 0.5),        # two planes, profiles in memory: 2, 2, 2, 2, 1
+    ((108, 108, 108), 9, 5, 2, -1.0),    # two planes, profiles in LDS
+    ((150, 150, 150), 10, 5, 3, 0.5),    # four: 4, 4, 2
+    ((150, 150, 150), 10, 20, 3, 0.5),   # the same, profiles too long for LDS
 ])
 def test_macrhs_chunks(gpu, oracle_lib, n, box, bins, interp, dpdt):
     T.test_macrhs_profiles_bitwise(gpu, oracle_lib, n, box, bins, interp, dpdt, "normal")
