@@ -7,7 +7,7 @@
 //                      solver, fused into one pass over the caller's boxes
 //   k_mean_*           solvability: compensated FP64 mean of rh (singular BCs)
 //   k_coarsen          coarse-level face coefficients (FBoxLib stencil fill,
-//                      Docs/mg/mg.tex:333-336; averaging rule of this build)
+//                      Docs/mg/mg.tex:333-336; averaging rule of this library)
 //   k_gsrb             red-black Gauss-Seidel (MG_SMOOTHER_GS_RB, mg.tex:201)
 //   k_residual         compute_defect (mg.tex:351)
 //   k_restrict         conservative-average restriction (mg.tex:353-354)
@@ -3404,7 +3404,9 @@ bool compact_level_ok(int dim, const Lev<float> &L)
 }
 
 // One fused red-black sweep of a 3D level (pin -> pout); false where no fused
-// form applies (the caller then sweeps per colour).
+// form applies (the caller then sweeps per colour).  What the pairs of
+// launch_sweep2 and the legs leave: an odd sweep, FP32 at nx = 128, the compact
+// form, odd nx or periods, arrays of 4 GiB and more.
 //   - nx = 128 or 256: the full-row sweep.  FP32 at nx = 256 and the compact
 //     (bfloat16) form run 6 rows in blocks of 768 threads with 80 VGPRs (the
 //     FP32 form with the weights fetched one plane ahead), two blocks per CU:
@@ -3414,7 +3416,8 @@ bool compact_level_ok(int dim, const Lev<float> &L)
 //     nx = 128 runs 16 rows of 1024 threads, and 8 rows of 1024 with alpha.
 //     FP64 runs 6 rows of 768 threads, and 4 rows of 512 with alpha (the
 //     alpha ring does not fit the 168 VGPRs a 768-thread block leaves a lane).
-//   - other sizes: one column per thread (k_gsrb_deep, two planes of prefetch).
+//   - other sizes: one column per thread (k_gsrb_deep, two planes of prefetch),
+//     which only single sweeps and those refusals reach.
 template <typename T>
 bool launch_gsrb_fused(const Lev<T> &L, const T *pin, T *pout, int mode, hipStream_t s, const Compact16 *K)
 {
@@ -3501,11 +3504,15 @@ bool launch_resid_restrict(int dim, const Lev<T> &F, const T *phi, const Lev<T> 
         const RowMarchGrid G = flat_grid((long)C.nx * C.ny, C.nz, 1, 16);
         const Compact16 K0 = {};
         if (F.alpha)
-            hipLaunchKernelGGL((k_rr_rows<T, false, true, true>), dim3(8 * G.per_xcd), dim3(256), 0, s, F, phi, C, G, K0);
+            hipLaunchKernelGGL((k_rr_rows<T, false, true, true>), dim3(8 * G.per_xcd), dim3(256), 0, s, F, phi, C, G,
+                               K0);
         else
-            hipLaunchKernelGGL((k_rr_rows<T, false, false, true>), dim3(8 * G.per_xcd), dim3(256), 0, s, F, phi, C, G, K0);
+            hipLaunchKernelGGL((k_rr_rows<T, false, false, true>), dim3(8 * G.per_xcd), dim3(256), 0, s, F, phi, C, G,
+                               K0);
         return true;
     }
+    // planes of 2^28 cells and more; in 2D the debug operator alone, a solve's
+    // restriction being the legs'
     dim3 g((C.nx + 63) / 64, C.ny, C.nz);
     if (dim == 3)
         hipLaunchKernelGGL((k_resid_restrict<3, T>), g, dim3(256), 0, s, F, phi, C);
@@ -3680,8 +3687,7 @@ void launch_fill(T *x, long n, T v, hipStream_t s)
     hipLaunchKernelGGL(k_fill<T>, dim3(nblk(n)), dim3(TPB), 0, s, x, n, v);
 }
 
-// LDS bytes the coarse cycle needs to keep levels lc..nlev-1 and the bottom
-// CG vectors on chip
+// One workgroup, on the level in global memory.
 template <typename T>
 void launch_bottom(int dim, const Lev<T> &L, const CoarseOpts &o, double *cg, hipStream_t s)
 {

@@ -151,17 +151,21 @@ __device__ __forceinline__ void scale_tiny(Pair<DIM, T> &P)
     }
 }
 
-// the right side of the pair's cell c, and its ap = A phi, without that scale
+// the right sides r of the pair and its ap = A phi without that scale (one
+// branch for both: it parts the loads before it from those behind)
 template <int DIM, typename T>
-__device__ __forceinline__ T true_scale(const Pair<DIM, T> &P, int c, T &ap)
+__device__ __forceinline__ void true_scale(const Pair<DIM, T> &P, T *r, T *ap)
 {
-    T r = P.rhs[c];
-    if (__builtin_expect(__ballot(P.tiny[c]) != 0, 0)) {
-        const T f = P.tiny[c] ? tiny_down<T>() : T(1);
-        ap *= f;
-        r *= f;
+    r[0] = P.rhs[0];
+    r[1] = P.rhs[1];
+    if (__builtin_expect(__ballot(P.tiny[0] || P.tiny[1]) != 0, 0)) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const T f = P.tiny[c] ? tiny_down<T>() : T(1);
+            ap[c] *= f;
+            r[c] *= f;
+        }
     }
-    return r;
 }
 
 // s: j + k is odd
@@ -465,19 +469,21 @@ __global__ void __launch_bounds__(NTH) k_leg(Lev<T> L, const T *__restrict__ pin
         const int c0 = gi + nx * (gj + ny * gk);
         store2(pout + c0, s[a] ? v[a][1] : v[a][0], s[a] ? v[a][0] : v[a][1]);
         if constexpr (!UP) {
-            T res[2];
+            T r[2], ap[2];
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 T p[2 * DIM];
                 const int o = pos[a];
                 pair_nbrs<DIM, T>(S[1 - c], s[a], c, v[a][1 - c], o - 1, o + 1, o - G::SY, o + G::SY, o - G::SZ,
                                   o + G::SZ, p);
-                T ap = apply_w<DIM, T>(L, P[a].w[c], p, v[a][c]);
-                const T r = true_scale(P[a], c, ap);
-                if (L.alpha) ap = dfma(L.alpha[c0 + (s[a] != (c == 1) ? 1 : 0)], v[a][c], ap);
-                res[c] = r - ap;
+                ap[c] = apply_w<DIM, T>(L, P[a].w[c], p, v[a][c]);
             }
-            rs[(m - 2) + CX * ((jj - H) + TY * (DIM == 3 ? kk - H : 0))] = res[0] + res[1];
+            true_scale(P[a], r, ap);
+            if (L.alpha) {
+#pragma unroll
+                for (int c = 0; c < 2; ++c) ap[c] = dfma(L.alpha[c0 + (s[a] != (c == 1) ? 1 : 0)], v[a][c], ap[c]);
+            }
+            rs[(m - 2) + CX * ((jj - H) + TY * (DIM == 3 ? kk - H : 0))] = (r[0] - ap[0]) + (r[1] - ap[1]);
         }
     }
     if constexpr (!UP) {
@@ -899,9 +905,11 @@ struct BottomBlock {
         return a;
     }
     // Beyond 512 cells a sum takes cells t and t + 512 together, then the waves
-    // in order.  A singular bottom's constant mode is whatever the rounding of
-    // its sums leaves in it, and phi's constant with it: the order is part of
-    // the result (k_bottom's blocks of 512 threads add alike).
+    // in order, as a block of 512 threads does (k_bottom).  A singular bottom's
+    // constant mode is whatever the rounding of its sums leaves in it, and phi's
+    // constant with it: with another order it moved by up to 1e-5 of phi's range
+    // (192 x 80 x 256).  The tests hold the solution up to that constant, and its
+    // bits from call to call; nothing compares the order itself.
     __device__ __forceinline__ double folded(double v)
     {
         if constexpr (!FOLD) return v;
@@ -1212,8 +1220,9 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
             if (up) {
                 const Lev<T> &C = LV.l[l + 1];
                 const T *e = arr(M.E[l + 1]);
-                const Two<T> d = prolong_pair<DIM, T>(C.nx, C.ny, C.nz, o.bc, 2 * pos[a].m, pos[a].j, pos[a].k,
-                                                      [&](int I, int J, int K) { return e[I + C.nx * (J + C.ny * K)]; });
+                auto at = [&](int I, int J, int K) { return e[I + C.nx * (J + C.ny * K)]; };
+                const Two<T> d =
+                    prolong_pair<DIM, T>(C.nx, C.ny, C.nz, o.bc, 2 * pos[a].m, pos[a].j, pos[a].k, at);
                 v[a][0] = v[a][0] + (pos[a].s ? d.b : d.a);
                 v[a][1] = v[a][1] + (pos[a].s ? d.a : d.b);
                 ref(pos[a].at) = v[a][0];   // read and written by this thread only until the barrier
@@ -1246,17 +1255,20 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
                 else store2(arr(M.E[l]) + 2 * pos[a].q, lo, hi);
                 continue;
             }
-            T res[2];
+            T r[2], ap[2];
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 T p[2 * DIM];
                 nbrs(pos[a], c, CS, v[a][1 - c], p);
-                T ap = apply_w<DIM, T>(L, P[a].w[c], p, v[a][c]);
-                const T r = true_scale(P[a], c, ap);
-                if (L.alpha) ap = dfma(L.alpha[2 * pos[a].q + (pos[a].s != (c == 1) ? 1 : 0)], v[a][c], ap);
-                res[c] = r - ap;
+                ap[c] = apply_w<DIM, T>(L, P[a].w[c], p, v[a][c]);
             }
-            arr(M.rs)[pos[a].q] = res[0] + res[1];
+            true_scale(P[a], r, ap);
+            if (L.alpha) {
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+                    ap[c] = dfma(L.alpha[2 * pos[a].q + (pos[a].s != (c == 1) ? 1 : 0)], v[a][c], ap[c]);
+            }
+            arr(M.rs)[pos[a].q] = (r[0] - ap[0]) + (r[1] - ap[1]);
         }
         if (!up || l > 0) __syncthreads();
         if (!up) to_level(l + 1);

@@ -405,7 +405,8 @@ __device__ __forceinline__ void ml_norm_max(double amax, unsigned long long *nrm
 // ------------------------------------------------------ composite residual
 // r = rh - A phi on the uncovered coarse cells (into rc; covered cells left
 // alone) and the fine cells (into rf), max |r| into *nrm.  fine_only: the
-// fine cells only.  The form for a region with holes (MlGeom::cov).  Cells whose six neighbours are plain cells of their own
+// fine cells only.  The form for a region with holes (MlGeom::cov).
+// Cells whose six neighbours are plain cells of their own
 // level (no wall, wrap, covered cell or region boundary) take the 7-point
 // form directly; the others go through the flux functions.  32-bit index
 // arithmetic (a level holds fewer than 2^31 cells).

@@ -355,7 +355,7 @@ static void free_hier(Hier<T> &H)
 }
 
 // point the levels' alpha at the hierarchy's alpha storage (on) or at
-// nothing (off); the device copy of the level table follows
+// nothing (off)
 template <typename T>
 static int set_alpha(mac_plan *P, Hier<T> &H, bool on)
 {
@@ -467,8 +467,8 @@ static int second_visit(int type)
 
 static int cycle_shape(const mac_opts &o) { return o.cycle_type == 0 ? MAC_CYCLE_V : o.cycle_type; }
 
-// One cycle of shape `type` from level l (levels lc.. run inside the
-// single-workgroup coarse cycle).  zero: level l's iterate is known to be
+// One cycle of shape `type` from level l (levels from lc on run inside the
+// single-workgroup coarse cycle, but for a level 0 in another form).  zero: level l's iterate is known to be
 // zero (a first visit below level 0, or a refinement step at level 0); a
 // second visit starts from the first one's iterate.  K: level 0's weights
 // and right side in compact storage; Rh: level 0 in the rho form (fused path).
@@ -719,12 +719,13 @@ static int inner_per_step(const mac_opts &o, bool compact)
 
 // Solve A phi = rhs on level 0 of H64 (phi holds the warm start).
 // Over-relaxation of the red-black sweeps on the levels of more than
-// relaxed_above() cells (the others keep Gauss-Seidel): mac_opts.omega where set, else 1 (FBoxLib's GSRB).  With 1.25 the 256^3 plane-parallel
-// projection converges in 6 V-cycles instead of 9 and the 512^3 star in 12
-// instead of 16 (to 1e-10, the oracle's FP64 cycle), but at the same relative
-// residual the over-relaxed iterate leaves more of its error in smooth modes:
-// 6.5e-9 from the 1e-13 solution in phi at 256^3 against 5.1e-10, so it is
-// an option, not the default.
+// relaxed_above() cells (the others keep Gauss-Seidel): mac_opts.omega where
+// set, else 1 (FBoxLib's GSRB).  With 1.25 the 256^3 plane-parallel projection
+// converges in 6 V-cycles instead of 9 and the 512^3 star in 12 instead of 16
+// (to 1e-10, the oracle's FP64 cycle), but at the same relative residual the
+// over-relaxed iterate leaves more of its error in smooth modes: 6.5e-9 from the
+// 1e-13 solution in phi at 256^3 against 5.1e-10, so it is an option, not the
+// default.
 static double sweep_omega(const mac_plan *P)
 {
     return P->opts.omega > 0 ? P->opts.omega : 1.0;

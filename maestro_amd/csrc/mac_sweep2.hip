@@ -75,7 +75,8 @@ struct __align__(2 * sizeof(T)) Cols {
 // HX pairs x RY rows per block (the tile and its halo), one thread each.
 // ZERO: the old iterate is zero and not read.  AL: the level has alpha.
 template <typename T, int HX, int RY, bool ZERO, bool AL, bool SOR>
-__global__ void __launch_bounds__(HX *RY) k_sweep2(Lev<T> L, const T *__restrict__ pin, T *__restrict__ pout, Sweep2Grid G)
+__global__ void __launch_bounds__(HX *RY) k_sweep2(Lev<T> L, const T *__restrict__ pin, T *__restrict__ pout,
+                                                   Sweep2Grid G)
 {
     using T2 = Cols<T>;
     constexpr int NW = HX * RY / 64, RW = 64 / HX;          // waves, rows of a wave
@@ -272,7 +273,8 @@ __global__ void __launch_bounds__(HX *RY) k_sweep2(Lev<T> L, const T *__restrict
                 constexpr int C = decltype(CC)::value;
                 constexpr bool DIV = decltype(DC)::value;
                 const T xo = O[C ? pos + 1 : pos - 1];
-                const T tx = dfma(C ? T(q.x1) : T(q.x0), C ? T(oth) : T(xo), (C ? T(q.x2) : T(q.x1)) * (C ? T(xo) : T(oth)));
+                const T tx = dfma(C ? T(q.x1) : T(q.x0), C ? T(oth) : T(xo),
+                                  (C ? T(q.x2) : T(q.x1)) * (C ? T(xo) : T(oth)));
                 const T ty = dfma(q.yl[C], O[pos - PX], q.yh[C] * O[pos + PX]);
                 const T tz = dfma(q.zl[C], zm, zh * zp);
                 const T num = dfma(ih2x, tx, dfma(ih2y, ty, dfma(ih2z, tz, q.r[C])));
@@ -300,8 +302,8 @@ __global__ void __launch_bounds__(HX *RY) k_sweep2(Lev<T> L, const T *__restrict
                                    zhi(2, tp2, wq[S1].zl[R0]));
                 A[3][B][pos] = v[S2][R2];
                 // second black, plane k - 3, column R3 ^ 1 = R0
-                v[S3][R0] = update(CA{}, DC, wq[S3], A[3][B ^ 1], v[S3][R0], v[S3][R3], R0 ? T(last1) : T(last0), v[S2][R0],
-                                   zhi(3, tp3, wq[S2].zl[R0]));
+                v[S3][R0] = update(CA{}, DC, wq[S3], A[3][B ^ 1], v[S3][R0], v[S3][R3], R0 ? T(last1) : T(last0),
+                                   v[S2][R0], zhi(3, tp3, wq[S2].zl[R0]));
             };
             // a scalar branch on the ballot keeps the second form out of the march
             // (0.5 us a launch; a branch on a lane mask 1.5, a test in each update
@@ -376,10 +378,12 @@ static void launch_sweep2_t(const Lev<T> &L, const T *pin, T *pout, int mode, hi
 
 // Where a pair goes this way: wherever its layout holds it (pairs of columns;
 // byte offsets within an array of 32 bits; a colour that holds across a
-// periodic face), but for FP32 at nx = 128, whose rows k_gsrb_rows sweeps out
-// of the caches: a 128^3 pair takes 34.0 us there and 33.4 here, from a zero
-// iterate 30.8 and 32.6, and whole solves with such a level are 1 to 3% faster
-// with the single sweeps.
+// periodic face), but for FP32 at nx = 128, which k_gsrb_rows sweeps out of the
+// caches where the level is no larger than 128^3: there a pair takes 34.0 us in
+// single sweeps and 33.4 here, from a zero iterate 30.8 and 32.6, and whole solves
+// with such a level are 1 to 3% faster with the single sweeps.  The rule looks at
+// nx alone; longer domains of such rows, levels with alpha and fewer than 8 planes
+// (k_gsrb_deep) have not been measured either way.
 // Two single sweeps (k_gsrb_rows at 128 and 256, k_gsrb_deep) and one pass,
 // microseconds:
 //   FP32  192^3 129, 66   256^3 215, 178   512^3 2190, 1194

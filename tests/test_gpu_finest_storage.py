@@ -31,7 +31,8 @@ def test_finest_level_of_4096_cells(gpu, oracle_lib, prec, cycle, top):
     e_phi = rel_err(out["phi"], truth["phi"], remove_mean=sing)
     e_ref = rel_err(same["phi"], truth["phi"], remove_mean=sing)
     e_u = max(rel_err(out["faces"][d], truth["faces"][d]) for d in range(3))
-    print(f"prec {prec} cycle {cycle}: {out['stats']['iters']} steps, phi {e_phi:.2e} (oracle {e_ref:.2e}), U {e_u:.2e}")
+    print(f"prec {prec} cycle {cycle}: {out['stats']['iters']} steps, phi {e_phi:.2e} (oracle {e_ref:.2e}), "
+          f"U {e_u:.2e}")
     assert out["stats"]["converged"]
     # NaN fails both; the bounds are those of the parity tests
     assert e_phi <= max(1e-8, 2.0 * e_ref)
@@ -48,7 +49,8 @@ def test_bf16_of_one_level(gpu, oracle_lib, n, levels, bc):
     plan = make_plan(n, bc, precision=mac.PREC_MIXED_BF16, max_levels=levels, device_ptrs=1)
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
     ph = t(np.zeros_like(phi))
-    st = plan.project_level(*[t(np.zeros(O.face_shape(g, d))) for d in range(3)], ph, *[t(x) for x in b], t(rhs), check=False)
+    z = [t(np.zeros(O.face_shape(g, d))) for d in range(3)]
+    st = plan.project_level(*z, ph, *[t(x) for x in b], t(rhs), check=False)
     res, _ = O.residual(g, b, ph.cpu().numpy(), rhs)
     print(n, st["iters"], np.abs(res).max())
     # the tolerance asked for, and the rounding of a residual: some 20 operations on terms of 6 w ih2 |phi|

@@ -52,7 +52,8 @@ def test_fp32_cycle_at_the_ends_of_the_range(gpu, oracle_lib, n, top, cycle):
     m = list(n)
     while all(x % 2 == 0 and x >= 4 for x in m):
         m = [x // 2 for x in m]
-    bc = [[P, P] if m[d] % 2 == 0 and d < dim - 1 else [WALL, OUT] for d in range(dim)]   # an odd period has no colouring
+    # an odd period has no colouring
+    bc = [[P, P] if m[d] % 2 == 0 and d < dim - 1 else [WALL, OUT] for d in range(dim)]
     g = O.make_grid(n, [1.0] * dim, bc)
     b, _, rhs = rand_level(g, n, dim, np.random.default_rng(73), O)
     b = [np.floor(4.0 * x) / 4.0 for x in b]   # at most 1.75: diagonals and sums of four faces below 16
