@@ -1506,6 +1506,19 @@ __device__ __forceinline__ void block_max_atomic(double a, unsigned long long *n
     }
 }
 
+// A thread's part of max |r|.  A maximum passes over NaN, so a residual of NaNs
+// would read 0 and count as converged: r * 0, NaN for NaN and infinity, is carried
+// along, one operation a cell.
+struct ResidMax {
+    double m = 0.0, bad = 0.0;
+    __device__ __forceinline__ void add(double r)
+    {
+        m = fmax(m, fabs(r));
+        bad = fma(r, 0.0, bad);
+    }
+    __device__ __forceinline__ double value() const { return bad == bad ? m : __builtin_huge_val(); }
+};
+
 // Grid-stride walk over the x-rows (j,k) of an nx x ny x nz level: each
 // wave takes whole rows and its lanes stride x.  The row index is
 // wave-uniform, so its division into (j,k) runs once per wave and row on the
@@ -1549,15 +1562,15 @@ static inline unsigned row_blocks(int nx, int ny, int nz)
 template <int DIM, typename T>
 __global__ void __launch_bounds__(TPB) k_residual(Lev<T> L, T *out, unsigned long long *nrm)
 {
-    double a = 0.0;
+    ResidMax a;
     for_rows(L.nx, L.ny, L.nz, [&](int i, int j, int k, long q) {
         T w[6], p[6];
         stencil<DIM, T>(L, L.phi, i, j, k, q, w, p);
         T r = L.rhs[q] - with_alpha(L, q, apply_value<DIM, T>(L, w, p, L.phi[q]), L.phi[q]);
         if (out) out[q] = r;
-        a = fmax(a, fabs((double)r));
+        a.add((double)r);
     });
-    if (nrm) block_max_atomic(a, nrm);
+    if (nrm) block_max_atomic(a.value(), nrm);
 }
 
 // FP64 residual of the refinement loop, written as FP32 right side of the
@@ -1566,15 +1579,15 @@ template <int DIM>
 __global__ void __launch_bounds__(TPB) k_ir_residual(Lev<double> L, float *r32,
                                                     unsigned long long *nrm)
 {
-    double a = 0.0;
+    ResidMax a;
     for_rows(L.nx, L.ny, L.nz, [&](int i, int j, int k, long q) {
         double w[6], p[6];
         stencil<DIM, double>(L, L.phi, i, j, k, q, w, p);
         double r = L.rhs[q] - with_alpha(L, q, apply_value<DIM, double>(L, w, p, L.phi[q]), L.phi[q]);
         r32[q] = (float)r;
-        a = fmax(a, fabs(r));
+        a.add(r);
     });
-    block_max_atomic(a, nrm);
+    block_max_atomic(a.value(), nrm);
 }
 
 // Refinement update fused with the next FP64 residual: phi_new = phi + e
@@ -1587,7 +1600,7 @@ __global__ void __launch_bounds__(TPB) k_ir_update_residual(Lev<double> L, const
                                                            double *__restrict__ phi_out, float *r32,
                                                            unsigned long long *nrm)
 {
-    double a = 0.0;
+    ResidMax a;
     for_rows(L.nx, L.ny, L.nz, [&](int i, int j, int k, long q) {
         double w[6], p[6];
         float pe[6];
@@ -1599,9 +1612,9 @@ __global__ void __launch_bounds__(TPB) k_ir_update_residual(Lev<double> L, const
         double r = L.rhs[q] - with_alpha(L, q, apply_value<DIM, double>(L, w, p, pc), pc);
         phi_out[q] = pc;
         r32[q] = (float)r;
-        a = fmax(a, fabs(r));
+        a.add(r);
     });
-    block_max_atomic(a, nrm);
+    block_max_atomic(a.value(), nrm);
 }
 
 // ---------------------------------------- FP64 residual passes, row march
@@ -1644,7 +1657,7 @@ __global__ void __launch_bounds__(256) k_resid_rows(Lev<double> L, const float *
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int bidx = (blockIdx.x & 7) * G.per_xcd + (blockIdx.x >> 3);   // XCD-contiguous
     const int gw = bidx * 4 + wv;
-    double a = 0.0;
+    ResidMax a;
     if (gw < G.total) {
         const int nx = L.nx, ny = L.ny, nz = L.nz, plane = nx * ny;
         int j, chunk, x0;
@@ -1802,7 +1815,7 @@ __global__ void __launch_bounds__(256) k_resid_rows(Lev<double> L, const float *
                 if constexpr (AL) ap = fma(c ? pc.a1 : pc.a0, pcc, ap);
                 res[c] = (c ? pc.r1 : pc.r0) - ap;
                 pcen[c] = pcc;
-                a = fmax(a, fabs(res[c]));
+                a.add(res[c]);
             }
             const size_t pk = (size_t)plane * k;
             if constexpr (MODE >= 1 && B16) {
@@ -1825,7 +1838,7 @@ __global__ void __launch_bounds__(256) k_resid_rows(Lev<double> L, const float *
             pc = pn;
         }
     }
-    block_max_atomic(a, nrm);
+    block_max_atomic(a.value(), nrm);
 }
 
 // ------------------------------------- residual + restriction, row march

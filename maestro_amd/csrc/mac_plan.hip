@@ -697,6 +697,7 @@ static int ir_norm(mac_plan *P, double *out, const Compact16 *K, int *bad)
 
 static bool converged(const mac_opts &o, double r, double r0)
 {
+    if (!std::isfinite(r)) return false;
     if (r0 == 0.0) return true;
     if (r <= o.eps_rel * r0) return true;
     if (o.eps_abs > 0.0 && r <= o.eps_abs) return true;
@@ -780,12 +781,12 @@ static int solve(mac_plan *P, mac_stats *st)
         P->launch_failed = false;
         int bad = 0;
         if ((rc = ir_norm(P, &r0, K, &bad))) return rc;
-        if (bad) return MAC_ERR_NONFINITE;
+        if (bad || !std::isfinite(r0)) return MAC_ERR_NONFINITE;
         r = r0;
         const Lev<float> &E = P->H32.lev[0];
         const int per_step = inner_per_step(o, K != nullptr);
         Lev<double> &L0 = P->H64.lev[0];
-        while (rc == MAC_OK && !converged(o, r, r0) && it < o.max_iter) {
+        while (rc == MAC_OK && !converged(o, r, r0) && std::isfinite(r) && it < o.max_iter) {
             for (int c = 0; c < per_step; ++c) {
                 vcycle<float>(P, P->H32, c == 0, K, Rh);
                 ++inner;
@@ -809,9 +810,9 @@ static int solve(mac_plan *P, mac_stats *st)
         coarsen_all<double>(P, P->H64);
         int bad = 0;
         if ((rc = fp64_norm(P, &r0, &bad))) return rc;
-        if (bad) return MAC_ERR_NONFINITE;
+        if (bad || !std::isfinite(r0)) return MAC_ERR_NONFINITE;
         r = r0;
-        while (!converged(o, r, r0) && it < o.max_iter) {
+        while (!converged(o, r, r0) && std::isfinite(r) && it < o.max_iter) {
             vcycle<double>(P, P->H64);
             if ((rc = fp64_norm(P, &r))) return rc;
             ++it;
