@@ -47,7 +47,7 @@ extern "C" {
 #define MAC_ERR_INVALID 1        /* invalid argument or option combination */
 #define MAC_ERR_LAYOUT 2         /* boxes do not tile the domain, bad ghosts */
 #define MAC_ERR_NONFINITE 3      /* NaN/Inf in rho, umac or the right side */
-#define MAC_ERR_NOT_CONVERGED 4  /* max_iter reached; stats are filled */
+#define MAC_ERR_NOT_CONVERGED 4  /* max_iter reached, or the iterate overflowed; stats are filled */
 #define MAC_ERR_HIP 5            /* a HIP runtime call failed */
 #define MAC_ERR_NOMEM 6
 #define MAC_ERR_TOO_LARGE 7      /* mac_project_noalloc: the call needs more than its fixed scratch */
@@ -206,7 +206,8 @@ int mac_project_noalloc(mac_plan *plan, double *const *umac, double *const *phi,
  * including beta0).  They require opts.device_ptrs = 1. */
 
 /* Forward: rh = macrhs - D(U); solve (-D beta G) phi = rh; U -= beta G phi.
- * Same operator, boundary handling and stopping rule as mac_project. */
+ * Same operator, boundary handling and stopping rule as mac_project.  A right
+ * side that is not finite gives phi = NaN and MAC_OK, here and in the adjoint. */
 int mac_project_level(mac_plan *plan, double *ux, double *uy, double *uz,
                       double *phi, const double *beta_x, const double *beta_y,
                       const double *beta_z, const double *macrhs, mac_stats *stats);

@@ -14,6 +14,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <limits>
 #include <mutex>
 #include <numeric>
 #include <thread>
@@ -742,9 +743,21 @@ static void set_omega(int dim, Hier<T> &H, double w)
     }
 }
 
-static int solve(mac_plan *P, mac_stats *st)
+// nan_through: a right side that is not finite gives phi = NaN and MAC_OK (the
+// differentiable entries, whose callers pass such values on), else an error.
+static int solve(mac_plan *P, mac_stats *st, bool nan_through = false)
 {
     int rc;
+    auto not_finite = [&](double r0) -> int {
+        if (!nan_through) return MAC_ERR_NONFINITE;
+        const Lev<double> &L = P->H64.lev[0];
+        launch_fill<double>(L.phi, ncell(P->n), std::numeric_limits<double>::quiet_NaN(), P->stream);
+        if (st) {
+            st->res0 = st->res = r0;
+            st->nlevels = P->H64.nlev;
+        }
+        return MAC_OK;
+    };
     const mac_opts &o = P->opts;
     if (o.precision < MAC_PREC_FP64 || o.precision > MAC_PREC_MIXED_BF16) return MAC_ERR_INVALID;
     if (o.cycle_type < 0 || o.cycle_type > MAC_CYCLE_V) return MAC_ERR_INVALID;
@@ -781,7 +794,8 @@ static int solve(mac_plan *P, mac_stats *st)
         P->launch_failed = false;
         int bad = 0;
         if ((rc = ir_norm(P, &r0, K, &bad))) return rc;
-        if (bad || !std::isfinite(r0)) return MAC_ERR_NONFINITE;
+        if (bad) return MAC_ERR_NONFINITE;
+        if (!std::isfinite(r0)) return not_finite(r0);
         r = r0;
         const Lev<float> &E = P->H32.lev[0];
         const int per_step = inner_per_step(o, K != nullptr);
@@ -810,7 +824,8 @@ static int solve(mac_plan *P, mac_stats *st)
         coarsen_all<double>(P, P->H64);
         int bad = 0;
         if ((rc = fp64_norm(P, &r0, &bad))) return rc;
-        if (bad || !std::isfinite(r0)) return MAC_ERR_NONFINITE;
+        if (bad) return MAC_ERR_NONFINITE;
+        if (!std::isfinite(r0)) return not_finite(r0);
         r = r0;
         while (!converged(o, r, r0) && std::isfinite(r) && it < o.max_iter) {
             vcycle<double>(P, P->H64);
@@ -1586,7 +1601,7 @@ extern "C" int mac_project_level(mac_plan *P, double *ux, double *uy, double *uz
     mac_stats local;
     memset(&local, 0, sizeof local);
     P->planar = false;   // the rho form is for mac_project, whose setup writes rho
-    int src = solve(P, &local);
+    int src = solve(P, &local, true);
     if (src != MAC_OK && src != MAC_ERR_NOT_CONVERGED) return src;
     HIPCHK(hipEventRecord(P->ev[2], s));
     const Lev<double> &L0 = P->H64.lev[0];
@@ -1659,7 +1674,7 @@ extern "C" int mac_adjoint_level(mac_plan *P, const double *phi, const double *b
     mac_stats local;
     memset(&local, 0, sizeof local);
     P->planar = false;   // the rho form is for mac_project, whose setup writes rho
-    int src = solve(P, &local);
+    int src = solve(P, &local, true);
     if (src != MAC_OK && src != MAC_ERR_NOT_CONVERGED) return src;
     if (P->singular)
         if ((rc = remove_mean(P, L0.phi, n0))) return rc;

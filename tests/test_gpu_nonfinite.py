@@ -1,10 +1,12 @@
 """A residual with NaN in it is not a small one: solves that overflow, and right
-sides that are not finite, never count as converged."""
+sides that are not finite, never count as converged.  The differentiable entries
+pass the latter on as NaN."""
 import math
 
 import numpy as np
 import pytest
 
+from maestro_amd import autograd
 from maestro_amd import mac
 from maestro_amd import workloads as W
 
@@ -48,6 +50,22 @@ def test_right_side_not_finite(gpu, oracle_lib, n, value, prec):
     plan = make_plan(n, bc, precision=prec, max_iter=5, device_ptrs=1)
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
     z = [t(np.zeros(O.face_shape(g, d))) for d in range(dim)] + [None] * (3 - dim)
-    with pytest.raises(mac.MacError) as e:
-        plan.project_level(*z, t(0.0 * phi), *[t(x) for x in b], *[None] * (3 - dim), t(rhs))
-    assert e.value.code == 3
+    ph = t(0.0 * phi)
+    st = plan.project_level(*z, ph, *[t(x) for x in b], *[None] * (3 - dim), t(rhs))
+    assert bool(torch.isnan(ph).all()) and not st["converged"]
+
+
+def test_gradient_not_finite(gpu):
+    torch = gpu
+    n = (16, 12, 10)
+    plan = autograd.level_plan(n, (1.0 / 16,) * 3, [[P, P], [WALL, WALL], [WALL, WALL]], precision=mac.PREC_FP64)
+    rng = np.random.default_rng(95)
+    shape = lambda d: tuple(n[e] + (e == d) for e in (2, 1, 0))
+    t = lambda a: torch.from_numpy(a).cuda().requires_grad_(True)
+    U = [t(np.zeros(shape(d))) for d in range(3)]
+    B = [t(rng.uniform(0.5, 2.0, shape(d))) for d in range(3)]
+    phi, *u = autograd.mac_project(plan, *U, *B)
+    weight = torch.ones_like(phi)
+    weight[3, 4, 5] = math.nan
+    grads = torch.autograd.grad((weight * phi).sum(), U)
+    assert all(bool(torch.isnan(x).any()) for x in grads)
