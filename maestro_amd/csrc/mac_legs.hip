@@ -134,6 +134,8 @@ __device__ __forceinline__ PairRaw<DIM, T> load_raw(const Lev<T> &L, int i, int 
     return R;
 }
 
+// to be called when a thread's loads are on their way: the branch waits for the
+// diagonals (called pair by pair it cost a round trip to memory, 0.3 us a leg)
 template <int DIM, typename T>
 __device__ __forceinline__ void scale_tiny(Pair<DIM, T> &P)
 {
@@ -147,6 +149,7 @@ __device__ __forceinline__ void scale_tiny(Pair<DIM, T> &P)
             for (int q = 0; q < 2 * DIM; ++q) P.w[c][q] *= f;
             P.den[c] *= f;
             P.rhs[c] *= f;
+            P.inv[c] = T(1) / P.den[c];
         }
     }
 }
@@ -189,7 +192,6 @@ __device__ __forceinline__ Pair<DIM, T> make_pair(const Lev<T> &L, const PairRaw
     P.rhs[1] = s ? R.r.a : R.r.b;
     P.den[0] = gs_den<DIM, T>(L, P.w[0], s ? R.al.b : R.al.a);
     P.den[1] = gs_den<DIM, T>(L, P.w[1], s ? R.al.a : R.al.b);
-    scale_tiny(P);
 #pragma unroll
     for (int c = 0; c < 2; ++c) P.inv[c] = T(1) / P.den[c];
     return P;
@@ -212,7 +214,6 @@ __device__ __forceinline__ Pair<DIM, T> dead_pair()
         for (int q = 0; q < 2 * DIM; ++q) P.w[c][q] = T(0);
         P.den[c] = P.inv[c] = T(1);
         P.rhs[c] = T(0);
-        P.tiny[c] = false;
     }
     return P;
 }
@@ -431,6 +432,7 @@ __global__ void __launch_bounds__(NTH) k_leg(Lev<T> L, const T *__restrict__ pin
     T v[NP][2];
 #pragma unroll
     for (int a = 0; a < NP; ++a) {
+        scale_tiny(P[a]);
         v[a][0] = S[0][pos[a]];
         v[a][1] = S[1][pos[a]];
     }
@@ -1124,6 +1126,7 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
         }
         if (lm) {
             Pm = make_pair<DIM, T>(LV.l[lm], Rm, om.s);
+            scale_tiny(Pm);
             tiny0 = Pm.tiny[0];
             tiny1 = Pm.tiny[1];
             if constexpr (PARK) {
@@ -1386,6 +1389,8 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
             if (sizeof(T) == 8) load0();
 #pragma unroll
             for (int a = 0; a < NP; ++a) P0[a] = make_pair<DIM, T>(L0, R0[a], o0[a].s);
+#pragma unroll
+            for (int a = 0; a < NP; ++a) scale_tiny(P0[a]);
             leg(0, false, std::integral_constant<int, C0>{}, P0, o0, [&](int a) { return o0[a].on; });
         }
     }
@@ -1439,6 +1444,8 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(CoarseLevs<T> LV, Coa
             o0[a] = pair_pos<DIM, T>(L0, tp + a * NT, 0, M.mx[0], M.my[0]);
             P0[a] = load_pair<DIM, T>(L0, 2 * o0[a].m, o0[a].j, o0[a].k);
         }
+#pragma unroll
+        for (int a = 0; a < NP; ++a) scale_tiny(P0[a]);
         leg(0, true, std::integral_constant<int, C0>{}, P0, o0, [&](int a) { return o0[a].on; });
     } else {
         const int n = L0.nx * L0.ny * L0.nz;
