@@ -25,8 +25,8 @@
 //
 // Measured: a pair on 512^3 FP32 takes 1.19 ms for the 3.2 GB it cannot do
 // without (2.7 TB/s; two single sweeps 2.19 ms), on 256^3 FP64 0.28 ms for 0.81
-// GB (2.9 TB/s; 0.35 ms).  Bound by the chain of a step, with half of the waves'
-// cycles spent waiting: the four updates follow each other through LDS and one
+// GB (2.9 TB/s; 0.35 ms).  Bound by the chain of a step, the waves waiting for
+// 47% (512^3 FP32) and 56% (256^3 FP64) of their cycles: the four updates follow each other through LDS and one
 // barrier, and the registers for the weights of four planes leave room for one
 // block per CU.  Loads by 64-bit address instead of buffer descriptors took
 // 1.47 ms at 512^3.
